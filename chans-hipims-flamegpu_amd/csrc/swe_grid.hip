@@ -335,30 +335,29 @@ template <class T>
 __device__ inline void update_state(const CellIn<T>& in, T& h, T& qx, T& qy, T dhf, T dqx, T dqy, T dF, T dt,
                                     T cfl_dx, T& hmax, T& cand, T& vol_h, T& flux_h, T& rain_h,
                                     bool time_control = true) {
-  cand = T(INFINITY);
-  vol_h = T(0);
-  flux_h = T(0);
-  rain_h = T(0);
-  if (!in.on) return;
+  // one branch (the wet cells' friction) and selects around it: nested
+  // branches cost a register copy per output on every side
   const T rdt = in.rain * dt;
   const T dht = (dhf + rdt) - dF;  // flux, + rain, - infiltration (the reference's order)
-  if (!(fabs(dht) > T(0) || h >= T(0))) {
-    vol_h = h;
-    return;
+  const bool upd = both(in.on, either(fabs(dht) > T(0), h >= T(0)));
+  T hn = h;
+  const bool wet = both(!new_depth_dry(hn, dht), upd);
+  T nqx = T(0), nqy = T(0), c = T(60.0);
+  if (wet) {
+    nqx = qx + dqx;
+    nqy = qy + dqy;
+    implicit_friction<T>(hn, in.n, dt, nqx, nqy);
+    if (time_control) c = cfl_candidate<T>(hn, nqx, nqy, cfl_dx);
   }
-  if (new_depth_dry(h, dht)) {
-    qx = T(0);
-    qy = T(0);
-  } else {
-    qx += dqx;
-    qy += dqy;
-    implicit_friction<T>(h, in.n, dt, qx, qy);
-  }
-  hmax = fmax(h, hmax);
-  if (time_control) cand = cfl_candidate<T>(h, qx, qy, cfl_dx);
-  vol_h = h;
-  flux_h = dhf;
-  rain_h = rdt;
+  h = upd ? hn : h;
+  qx = upd ? nqx : qx;
+  qy = upd ? nqy : qy;
+  const T hm = Prec<T>::max2(hn, hmax);
+  hmax = upd ? hm : hmax;
+  cand = upd ? c : T(INFINITY);
+  vol_h = in.on ? h : T(0);
+  flux_h = upd ? dhf : T(0);
+  rain_h = upd ? rdt : T(0);
 }
 
 // FUSED = false: write the flux accumulators dh/dqx/dqy (two-pass step).

@@ -71,6 +71,19 @@ __host__ __device__ inline bool new_depth_dry(float& h, float dh) {
   return hn < kHs;
 }
 
+// && and || that evaluate both sides (no branch).
+__host__ __device__ inline bool both(bool a, bool b) { return a & b; }
+__host__ __device__ inline bool either(bool a, bool b) { return a | b; }
+
+// a * b as a product of its own: never contracted into a multiply-add with
+// the sum it feeds.  Whether the compiler contracts depends on the control
+// flow between the two operations; the products written so give the same bits
+// on every path that forms them.
+template <class T> __host__ __device__ inline T mul_alone(T a, T b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
 template <class T> __host__ __device__ inline T minmod(T x, T y) {
   const T m = fabs(x) < fabs(y) ? x : y;
   return x * y <= T(0) ? T(0) : m;
@@ -117,10 +130,18 @@ template <> struct Prec<float> {
   __device__ static inline float limit(float x, float y) { return __builtin_amdgcn_fmed3f(x, y, 0.0f); }
   // clamp to [lo, hi] (lo <= hi) as one median-of-three
   __device__ static inline float clamp(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
-  // max / min as a median with an infinity: no quieting of the (loaded,
-  // possibly signalling) inputs that fmaxf / fminf need in IEEE mode
-  __device__ static inline float max2(float x, float y) { return __builtin_amdgcn_fmed3f(x, y, INFINITY); }
-  __device__ static inline float min2(float x, float y) { return __builtin_amdgcn_fmed3f(x, y, -INFINITY); }
+  // max / min as the bare instruction: fmaxf / fminf first quiet an input that
+  // was loaded or came through a lane shift (one more instruction each)
+  __device__ static inline float max2(float x, float y) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+  }
+  __device__ static inline float min2(float x, float y) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+  }
   __device__ static inline float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
   __device__ static inline float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
   // h^(-1/3) = exp2(-log2(h) / 3) with the hardware log2 / exp2 (h >= 1e-6)
@@ -236,21 +257,27 @@ template <class T> struct EdgeOut {
 // eL / eR: edge states before reconstruction (h, qn, qt, z) - velocities come
 // from these.  etaC / etaR: the cells' water levels used by the clamp.
 // On return eL.h/eL.z and eR.h/eR.z hold the reconstructed depth and bed.
+// off: no flux passes (both cells dry).
 template <class T, int ORDER>
-__host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T etaC, T etaR, T& fh, T& fn, T& ft) {
+__host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T etaC, T etaR, T& fh, T& fn, T& ft,
+                                          bool off = false) {
   // Written as straight-line code with selects: a wave whose edges fall in
   // different wave-speed regions evaluates one path instead of all three
-  // under divergent branches.  The selected values are the same expressions
-  // the branches would produce.
+  // under divergent branches.  Each alternative is a value of its own before
+  // the select picks it, and conditions are combined by both / either: the
+  // compiler turns a conditional expression whose arms compute something,
+  // and && and ||, into branches of a few instructions each, with the exec
+  // mask saved and restored around them.
   using P = Prec<T>;
   const T g = T(kG);
   // one reciprocal per face serves both velocities (in FP64 two IEEE
   // divisions become one; in FP32 the hardware reciprocal was shared anyway)
   const T rhL = P::div(T(1), eL.h), rhR = P::div(T(1), eR.h);
-  const T uL0 = lt_hs(eL.h) ? T(0) : eL.qn * rhL;
-  const T vL0 = lt_hs(eL.h) ? T(0) : eL.qt * rhL;
-  const T uR0 = lt_hs(eR.h) ? T(0) : eR.qn * rhR;
-  const T vR0 = lt_hs(eR.h) ? T(0) : eR.qt * rhR;
+  const bool dryL = lt_hs(eL.h), dryR = lt_hs(eR.h);
+  const T uLw = mul_alone(eL.qn, rhL), vLw = mul_alone(eL.qt, rhL);
+  const T uRw = mul_alone(eR.qn, rhR), vRw = mul_alone(eR.qt, rhR);
+  const T uL0 = dryL ? T(0) : uLw, vL0 = dryL ? T(0) : vLw;
+  const T uR0 = dryR ? T(0) : uRw, vR0 = dryR ? T(0) : vRw;
 
   // hydrostatic reconstruction
   T wL = eL.h + eL.z;
@@ -276,29 +303,39 @@ __host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T 
   eR.z = wR - eR.h;
 
   const T hL = eL.h, hR = eR.h;
-  const T qnL = uL0 * hL, qtL = vL0 * hL;
-  const T qnR = uR0 * hR, qtR = vR0 * hR;
+  const T qnL = mul_alone(uL0, hL), qtL = vL0 * hL;
+  const T qnR = mul_alone(uR0, hR), qtR = vR0 * hR;
   const T aL = P::sqrt_(g * hL);
   const T aR = P::sqrt_(g * hR);
   const T base = (aL + aR) / T(2) + (uL0 - uR0) / T(4);
   const T u_star = (uL0 + uR0) / T(2) + aL - aR;
   const T a_star = P::star_celerity(base, g);
-  const T sL = le_hs(hL) ? uR0 - T(2) * aR : fmin(uL0 - aL, u_star - a_star);
-  const T sR = le_hs(hR) ? uL0 + T(2) * aL : fmax(uR0 + aR, u_star + a_star);
-  const T sM = P::div(sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), hR * (uR0 - sR) - hL * (uL0 - sL));
+  const T sL_dry = uR0 - T(2) * aR, sL_wet = fmin(uL0 - aL, u_star - a_star);
+  const T sR_dry = uL0 + T(2) * aL, sR_wet = fmax(uR0 + aR, u_star + a_star);
+  const T sL = le_hs(hL) ? sL_dry : sL_wet;
+  const T sR = le_hs(hR) ? sR_dry : sR_wet;
+  // only the sign of the contact speed sM = num / den is used, and num * den
+  // has it without the division (den is 0 only between two dry sides, whose
+  // flux is 0 whatever is chosen here)
+  const T num = sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), den = hR * (uR0 - sR) - hL * (uL0 - sL);
+  const T sM = num * den;
   const T qnfL = uL0 * qnL + T(0.5) * g * hL * hL;
   const T qnfR = uR0 * qnR + T(0.5) * g * hR * hR;
   const T rS = P::div(T(1), sR - sL);
   const T fh_s = (sR * qnL - sL * qnR + sL * sR * (hR - hL)) * rS;
   const T fn_s = (sR * qnfL - sL * qnfR + sL * sR * (qnR - qnL)) * rS;
-  const bool star_l = sL < T(0) && T(0) <= sM;
-  const T ft_s = fh_s * (star_l ? vL0 : vR0);
+  const bool star_l = both(sL < T(0), T(0) <= sM);
+  const T v_s = star_l ? vL0 : vR0;
+  const T ft_s = fh_s * v_s;
+  const T ftL = uL0 * qtL, ftR = uR0 * qtR;
   const bool left = T(0) <= sL;
-  const bool star = star_l || (sM < T(0) && T(0) <= sR);
-  const bool dry = lt_hs(hL) && lt_hs(hR);
-  fh = dry ? T(0) : (left ? qnL : (star ? fh_s : qnR));
-  fn = dry ? T(0) : (left ? qnfL : (star ? fn_s : qnfR));
-  ft = dry ? T(0) : (left ? uL0 * qtL : (star ? ft_s : uR0 * qtR));
+  const bool star = either(star_l, both(sM < T(0), T(0) <= sR));
+  const bool dry = either(both(lt_hs(hL), lt_hs(hR)), off);
+  const T fh_r = star ? fh_s : qnR, fn_r = star ? fn_s : qnfR, ft_r = star ? ft_s : ftR;
+  const T fh_l = left ? qnL : fh_r, fn_l = left ? qnfL : fn_r, ft_l = left ? ftL : ft_r;
+  fh = dry ? T(0) : fh_l;
+  fn = dry ? T(0) : fn_l;
+  ft = dry ? T(0) : ft_l;
 }
 
 // Solve one edge from cell c towards r (direction d).
@@ -374,7 +411,6 @@ __host__ __device__ inline void implicit_friction(T h, T n, T dt, T& qx, T& qy) 
   const T g = T(kG);
   const T C_f = g * n * n * Prec<T>::rcbrt_friction(h);
   const T q_norm = P::sqrt_(qx * qx + qy * qy);
-  if (!(n > T(0))) return;
   const T lim = T(5) * h * P::sqrt_(h * g);
   if (P::local_datum) {
     // cancellation-free: (1 - sqrt(1 + x)) / (-(x/2) / q_k) == 2 q_k / (1 + sqrt(1 + x))
@@ -384,11 +420,14 @@ __host__ __device__ inline void implicit_friction(T h, T n, T dt, T& qx, T& qy) 
     // reflected 2 q' - q, zeroed on a sign change; |q| <= 1e-10 unchanged
     const T tx = k * qx, ty = k * qy;
     const T rx = T(2) * tx - qx, ry = T(2) * ty - qy;
-    const T ox = fabs(tx) > lim ? (rx * tx <= T(0) ? T(0) : rx) : tx;
-    const T oy = fabs(ty) > lim ? (ry * ty <= T(0) ? T(0) : ry) : ty;
-    qx = fabs(qx) > T(1.0e-10) ? ox : qx;
-    qy = fabs(qy) > T(1.0e-10) ? oy : qy;
+    const T zx = rx * tx <= T(0) ? T(0) : rx, zy = ry * ty <= T(0) ? T(0) : ry;
+    const T ox = fabs(tx) > lim ? zx : tx;
+    const T oy = fabs(ty) > lim ? zy : ty;
+    const bool rough = n > T(0);
+    qx = both(rough, fabs(qx) > T(1.0e-10)) ? ox : qx;
+    qy = both(rough, fabs(qy) > T(1.0e-10)) ? oy : qy;
   } else {
+    if (!(n > T(0))) return;
     if (fabs(qx) > T(1.0e-10)) {
       const T tmp = (T(1) - P::sqrt_(T(1) + (T(4) * dt * C_f) / (h * h) * q_norm)) /
                     (T(-2) * dt * C_f / (h * h) * (q_norm / qx));
