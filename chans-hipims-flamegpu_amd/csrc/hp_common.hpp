@@ -51,12 +51,27 @@ constexpr int kXcds = 8;
 // registers across long kernels, which spills them.  The pointer must be
 // uniform across the wave.
 typedef __attribute__((address_space(4))) const hp_grid_desc* KDesc;
+// A control block no launch of the reading kernel writes, likewise.
+typedef __attribute__((address_space(4))) const hp_ctrl* KCtrl;
 template <class DP> __device__ inline DP launder(DP p) {
   asm volatile("" : "+s"(p));
   return p;
 }
 // The descriptor of a kernel whose first argument is its hp_grid_desc.
 __device__ inline KDesc kernarg_desc() { return (KDesc)__builtin_amdgcn_kernarg_segment_ptr(); }
+// Division by a number known at launch: n / d = n * m >> s for 0 <= n < 2^31
+// (m = floor(2^s / d) + 1 with s = 31 + ceil(log2 d)), in scalar registers; the
+// division itself would be some twenty vector instructions per wave.
+struct Divisor {
+  uint32_t m;
+  int s, n;
+  static Divisor of(int d) {
+    int l = 0;
+    while ((int64_t(1) << l) < d) ++l;
+    return Divisor{(uint32_t)((uint64_t(1) << (31 + l)) / (uint64_t)d + 1), 31 + l, d};
+  }
+  __host__ __device__ int div(int x) const { return (int)((uint64_t)(uint32_t)x * m >> s); }
+};
 __device__ inline int xcd_band(int b, int n) {
   const int q = n / kXcds, rem = n - q * kXcds;
   const int x = b % kXcds, local = b / kXcds;

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kAThreads) void k_adj_update(hp_grid_desc a, AdjPla
   const T t_T = T(t_now);
   const int mode = a.rain_mode;
   for (int k = tid; k < a.n_classes; k += kAThreads) s_man[k] = ((const T*)a.manning)[k];
-  const RainRows rr = rain_rows(a, t_now);
+  const RainRows rr = wave_rain_rows(&a, t_now);
   if (mode == HP_RAIN_STATION && tid < kARateCache) {
     s_rb[tid] = station_rate<T>(rr, tid, 1.0);
     s_rs[tid] = station_rate<T>(rr, tid, a.rain_scale);
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(NT, sizeof(T) == 4 ? 6 : 1) void k_adj_step_tile(hp
   const T t_T = T(t_now);
   const int mode = pa->rain_mode;
   for (int k = tid; k < pa->n_classes; k += NT) s_man[k] = ((const T*)pa->manning)[k];
-  const RainRows rr = rain_rows_at(pa, t_now);
+  const RainRows rr = wave_rain_rows(pa, t_now);
   if (mode == HP_RAIN_STATION && tid < kARateCache) {
     s_rb[tid] = station_rate<T>(rr, tid, 1.0);
     s_rs[tid] = station_rate<T>(rr, tid, pa->rain_scale);

@@ -6,13 +6,11 @@
 // so the raster's own nodata ring doubles as the stencil apron.
 //
 // Per step:
-//   flux    tile of 64 x TY cells + 2-cell cross halo staged in LDS; every
-//           edge touching the tile is solved once (swe_physics.hpp), by the
-//           thread that owns its east/south cell, and both cells take their
-//           share (the owner's in registers, the other through LDS); listed
-//           cells (the reference's fluxMask rule) write dh/dqx/dqy.
-//   single-pass step: the flux tile finishes its own cells (the update
-//           below) into a second set of state planes.
+//   flux    column walk (swe_walk.hpp): a wave per unit of 60 columns x R
+//           rows solves every edge of its cells; listed cells (the
+//           reference's fluxMask rule) write dh/dqx/dqy.
+//   single-pass step: the walk finishes its own cells (the update below)
+//           into a second set of state planes.
 //   update  a contiguous chunk of plane elements per block: rain, implicit
 //           friction + update, h_max, the CFL minimum (wave64 shuffle + LDS),
 //           FP64 volume / flux / rain sums; one partial record per block.
@@ -30,6 +28,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <utility>
@@ -43,7 +42,6 @@
 
 namespace hp {
 
-constexpr int kTX = 64;
 constexpr int kThreads = 256;
 constexpr int kChunk = 2048;  // plane elements per update block
 constexpr int kMaxStations = 1024;
@@ -65,26 +63,10 @@ __device__ inline T series_at(const T* tab, int rows, int w, int row, int col) {
   return tab[row * w + col];
 }
 
-struct SeriesRows {
-  int d, w, q;
-};
-
 template <class T> struct BcValues {
   int type;
   T gd, gwl, gqx, gqy;
 };
-
-template <class T>
-__device__ inline BcValues<T> bc_values(const hp_grid_desc& a, int slot, const SeriesRows& rows) {
-  BcValues<T> b;
-  int id;
-  decode_code(a.slot_code[slot], b.type, id);
-  b.gd = series_at<T>((const T*)a.given_depth, a.gd_rows, a.gd_w, rows.d, id + 1);
-  b.gwl = series_at<T>((const T*)a.given_wl, a.gwl_rows, a.gwl_w, rows.w, id + 1);
-  b.gqx = series_at<T>((const T*)a.given_q, a.gq_rows, a.gq_w, rows.q, 1 + 2 * id);
-  b.gqy = series_at<T>((const T*)a.given_q, a.gq_rows, a.gq_w, rows.q, 2 + 2 * id);
-  return b;
-}
 
 // Global (qx, qy) of an edge-frame momentum flux (fn, ft) for direction d.
 template <class T> __device__ inline void to_global(T fn, T ft, int d, T& gx, T& gy) {
@@ -158,127 +140,6 @@ __device__ inline double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
-}
-
-// LDS tile of one flux block.
-template <class T, int TY> struct FluxTile {
-  static constexpr int LW = kTX + 4, LH = TY + 4;
-  T h[LH][LW], qx[LH][LW], qy[LH][LW], z[LH][LW];
-  uint8_t ty[LH][LW];
-  // Edge record (solve_tile_edge), A = west / north cell, B = east / south
-  // cell, fluxes from A's view (subtract at A, add at B):
-  //   double (kRec 5): 0 mass, 1 qx, 2 qy, 3 bed term of A, 4 bed term of B
-  //     (the reference's accumulation order: flux terms, then the bed term);
-  //   float (kRec 4): 0 mass, 1 momentum across the edge axis, 2 momentum
-  //     along the axis + A's bed term, 3 the same - B's bed term.
-  static constexpr int kRec = sizeof(T) == 4 ? 4 : 5;
-  // A record splits into the part its A cell reads and the part its B cell
-  // reads (kSide words each: mass, the two momentum terms and that side's
-  // bed term, folded as above).  The thread that owns a cell solves the
-  // cell's west x-edge and north y-edge, where the cell is B: it keeps the B
-  // part in registers and leaves the A part here, under the A cell - the
-  // west neighbour's east-edge part (a[0]) and the north neighbour's
-  // south-edge part (a[1]).
-  static constexpr int kSide = kRec - 1;
-  T a[2][kSide][TY][kTX];
-};
-
-// The part of record e that cell A (side 0) or cell B (side 1) reads.
-template <class T, int kRec>
-__device__ inline T side_word(const T* e, int side, int k) {
-  if (kRec == 5) return k < 3 ? e[k] : e[3 + side];
-  return k < 2 ? e[k] : e[2 + side];
-}
-
-template <class T, int TY>
-__device__ inline FrameCell<T> frame_cell(const FluxTile<T, TY>& s, int r, int c, int d, T zref) {
-  FrameCell<T> f;
-  const T qx = s.qx[r][c], qy = s.qy[r][c];
-  f.h = s.h[r][c];
-  f.qn = rot_n(qx, qy, d);
-  f.qt = rot_t(qx, qy, d);
-  f.z = s.z[r][c] - zref;
-  return f;
-}
-
-// Frame view for a compile-time direction D (0 E for x-edges, 3 S for
-// y-edges): the rotation is a fixed renaming, no selects.
-template <int D, class T, int TY>
-__device__ inline FrameCell<T> frame_cell_d(const FluxTile<T, TY>& s, int r, int c, T zref) {
-  FrameCell<T> f;
-  const T qx = s.qx[r][c], qy = s.qy[r][c];
-  f.h = s.h[r][c];
-  f.qn = D == 0 ? qx : -qy;
-  f.qt = D == 0 ? qy : qx;
-  f.z = s.z[r][c] - zref;
-  return f;
-}
-
-// Write one edge record (layouts in FluxTile).  gx, gy: global momentum flux
-// from A's view; bedA / bedB: the two sides' bed terms along the edge axis.
-template <class T, int D, int kRec>
-__device__ inline void store_record(T* out, T fh, T gx, T gy, T bedA, T bedB) {
-  out[0] = fh;
-  if (kRec == 5) {
-    out[1] = gx;
-    out[2] = gy;
-    out[3] = bedA;
-    out[4] = bedB;
-  } else {
-    const T axis = D == 0 ? gx : gy;
-    out[1] = D == 0 ? gy : gx;
-    out[2] = axis + bedA;
-    out[3] = axis - bedB;
-  }
-}
-
-// Solve the edge between LDS cells A and B, where B lies in direction D from
-// A (D = 0: x-edge, B east of A; D = 3: y-edge, B south of A).  A is
-// (ra, ca); L is A's neighbour opposite to B, RR is B's neighbour beyond B.
-// Writes the edge record out[0 .. kRec-1].
-template <class T, int ORDER, int TY, int D>
-__device__ inline void solve_tile_edge(const FluxTile<T, TY>& s, const hp_grid_desc& a, const SeriesRows& rows,
-                                       int ra, int ca, T dx, T dt, T dt_dx, T* out) {
-  constexpr int di = D == 0 ? 0 : 1, dj = D == 0 ? 1 : 0;  // B - A in (row, col)
-  const int rb = ra + di, cb = ca + dj;
-  const int rl = ra - di, cl = ca - dj;
-  const int rr2 = rb + di, cr2 = cb + dj;
-  constexpr int kRec = FluxTile<T, TY>::kRec;
-#pragma unroll
-  for (int k = 0; k < kRec; ++k) out[k] = T(0);
-  const int tA = s.ty[ra][ca], tB = s.ty[rb][cb];
-  if (tA == 0 && tB == 0) return;
-  constexpr T nA = T(D == 0 ? 1 : -1);  // A's outward normal component along the edge axis
-  if (tA != 0 && tB != 0) {
-    const T zref = Prec<T>::local_datum ? s.z[ra][ca] : T(0);
-    FrameCell<T> c = frame_cell_d<D>(s, ra, ca, zref);
-    if (Prec<T>::local_datum) c.z = T(0);  // its own datum: z - z is exactly 0, known here at compile time
-    const FrameCell<T> r = frame_cell_d<D>(s, rb, cb, zref);
-    const FrameCell<T> lc = frame_cell_d<D>(s, rl, cl, zref);
-    const FrameCell<T> rc = frame_cell_d<D>(s, rr2, cr2, zref);
-    const FrameCell<T> l = s.ty[rl][cl] ? lc : c;
-    const FrameCell<T> rr = s.ty[rr2][cr2] ? rc : r;
-    const EdgeOut<T> o = solve_edge<T, ORDER>(c, l, r, rr, false, c.h + c.z, r.h + r.z, dx, dt, dt_dx);
-    if (!o.active) return;
-    store_record<T, D, kRec>(out, o.fh, D == 0 ? o.fn : o.ft, D == 0 ? o.ft : -o.fn, o.bed_c * nA, o.bed_r * (-nA));
-  } else {
-    // boundary edge, solved from the valid side with its outward normal
-    const bool from_a = tA != 0;
-    const int rc = from_a ? ra : rb, cc = from_a ? ca : cb, d = from_a ? D : (D + 2) & 3;
-    const bool axis_x = D == 0;
-    const T zref = Prec<T>::local_datum ? s.z[rc][cc] : T(0);
-    const FrameCell<T> c = frame_cell(s, rc, cc, d, zref);
-    const BcValues<T> bv = bc_values<T>(a, from_a ? tA : tB, rows);
-    const FrameCell<T> g = bc_ghost<T>(bv.type, c, d, bv.gd, bv.gwl - zref, bv.gqx, bv.gqy);
-    const T etaG = ORDER == 1 ? g.h + g.z : ghost_wl<T>(bv.type, c.h + c.z, g, bv.gwl - zref);
-    const EdgeOut<T> o = solve_edge<T, ORDER>(c, c, g, g, true, c.h + c.z, etaG, dx, dt, dt_dx);
-    if (!o.active) return;
-    T gx, gy;
-    to_global(o.fn, o.ft, d, gx, gy);
-    const T bed = o.bed_c * T(axis_x ? nrm_x(d) : nrm_y(d));
-    if (from_a) store_record<T, D, kRec>(out, o.fh, gx, gy, bed, T(0));
-    else store_record<T, D, kRec>(out, -o.fh, -gx, -gy, T(0), bed);
-  }
 }
 
 // Fold a block's CFL minimum and FP64 sums into its partial slot.
@@ -360,306 +221,6 @@ __device__ inline void update_state(const CellIn<T>& in, T& h, T& qx, T& qy, T d
   rain_h = upd ? rdt : T(0);
 }
 
-// FUSED = false: write the flux accumulators dh/dqx/dqy (two-pass step).
-// FUSED = true: finish the step in the same block - rain, implicit friction
-// and update of the tile's own cells into h_out/qx_out/qy_out (the input
-// planes stay untouched for the neighbouring tiles' halos), h_max, and one
-// partial record (CFL minimum, FP64 sums) per tile.
-// time_control false (single-pass step of a frozen schedule, whose time
-// control never runs): no CFL candidates, sums or partial record.
-template <class T, int ORDER, int TY, bool FUSED>
-__device__ inline void flux_tile(const hp_grid_desc& a, int bx, int by, const Partials& part, int64_t pidx,
-                                 bool save_flux = false, bool time_control = true, bool force_copy = false) {
-  __shared__ FluxTile<T, TY> s;
-  __shared__ T s_rate[FUSED ? kRateCache : 1];
-  using Tile = FluxTile<T, TY>;
-  constexpr int LH = Tile::LH;
-  constexpr int CPT = TY * kTX / kThreads;  // own cells per thread
-  static_assert(TY * kTX % kThreads == 0, "tile cells per thread");
-  if (stopped(a.ctrl)) {
-    if (FUSED) {
-      if (threadIdx.x == 0) part.put(pidx, INFINITY, 0.0, 0.0, 0.0, a.mass_sums != 0);
-      // the state passes through to the output planes as well, so that a
-      // caller alternating the two sets of planes keeps the final state;
-      // once the time control has marked it done, both sets hold it (unless
-      // the caller asks for the copy: the first step of a call, after which
-      // the host may have written the state)
-      if (a.ctrl->stopped_synced != 0.0 && !force_copy) return;
-      const int gx = bx * kTX + (int)(threadIdx.x & (kTX - 1));
-#pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        const int gy = by * TY + (int)(threadIdx.x / kTX) + (kThreads / kTX) * k;
-        if (gx < a.nx && gy < a.ny) {
-          const int64_t gi = (int64_t)gy * a.pitch + gx;
-          ((T*)a.h_out)[gi] = ((const T*)a.h)[gi];
-          ((T*)a.qx_out)[gi] = ((const T*)a.qx)[gi];
-          ((T*)a.qy_out)[gi] = ((const T*)a.qy)[gi];
-        }
-      }
-    }
-    return;
-  }
-  const int tid = threadIdx.x;
-  const int lane = tid & (kTX - 1), wv = tid / kTX;
-  const int x0 = bx * kTX, y0 = by * TY;
-  const int nx = a.nx, ny = a.ny;
-  const int64_t pitch = a.pitch;
-  const T* __restrict__ h = (const T*)a.h;
-  const T* __restrict__ qx = (const T*)a.qx;
-  const T* __restrict__ qy = (const T*)a.qy;
-  const T* __restrict__ z = (const T*)a.z;
-  const uint8_t* __restrict__ ty = a.type_slot;
-
-  // the thread's own cells: column x0 + lane, rows y0 + wv + 4k
-  CellIn<T> cin[FUSED ? CPT : 1];
-  RainRows rr{};
-  if (FUSED) {
-    rr = rain_rows(a, a.ctrl->t);
-    if (a.rain_mode == HP_RAIN_STATION && tid < kRateCache) s_rate[tid] = station_rate<T>(rr, tid, a.rain_scale);
-    const int gx = x0 + lane;
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int gy = y0 + wv + 4 * k;
-      cin[k] = CellIn<T>{T(0), 0, T(0), T(0), T(0), 0, false};
-      if (gx < nx && gy < ny) {
-        const int64_t gi = (int64_t)gy * pitch + gx;
-        const int cls = a.landuse[gi];
-        cin[k].on = cls != 255;
-        cin[k].cls = cls;
-        // the class's Manning value from the (cached) table: no LDS copy, so
-        // that six blocks fit a CU; a class beyond the table (undefined in
-        // the reference) reads its last entry, never past it
-        if (cin[k].on) cin[k].n = ((const T*)a.manning)[cls < a.n_classes ? cls : a.n_classes - 1];
-        if (a.rain_mode == HP_RAIN_STATION) cin[k].st = a.station ? (int)a.station[gi] : 0;
-        else if (a.rain_mode == HP_RAIN_FIELD) cin[k].rain = T(a.rain_field[gi]) * T(a.rain_scale);
-        cin[k].hmax = ((const T*)a.h_max)[gi];
-        if (a.infil_ks) cin[k].F = ((const T*)a.infil_F)[gi];
-      }
-    }
-  }
-
-  // Stage the tile and a 2-cell halo: the 64 interior columns row by row
-  // (one wave per row, coalesced), then the 4 halo columns.
-  {
-    const int gx = x0 + lane;
-    for (int r = wv; r < LH; r += kThreads / kTX) {
-      const int gy = y0 - 2 + r;
-      const bool in = gx < nx && gy >= 0 && gy < ny;
-      T vh = T(0), vqx = T(0), vqy = T(0), vz = T(0);
-      uint8_t vt = 0;
-      if (in) {
-        const int64_t gi = (int64_t)gy * pitch + gx;
-        vt = ty[gi]; vh = h[gi]; vqx = qx[gi]; vqy = qy[gi]; vz = z[gi];
-      }
-      s.ty[r][lane + 2] = vt; s.h[r][lane + 2] = vh; s.qx[r][lane + 2] = vqx; s.qy[r][lane + 2] = vqy;
-      s.z[r][lane + 2] = vz;
-    }
-    static_assert(4 * LH <= kThreads, "halo staging");
-    if (tid < 4 * LH) {
-      const int r = tid >> 2, k = tid & 3;
-      const int c = k < 2 ? k : kTX + k;  // local columns 0, 1, 66, 67
-      const int gy = y0 - 2 + r, gxh = x0 - 2 + c;
-      const bool in = gxh >= 0 && gxh < nx && gy >= 0 && gy < ny;
-      T vh = T(0), vqx = T(0), vqy = T(0), vz = T(0);
-      uint8_t vt = 0;
-      if (in) {
-        const int64_t gi = (int64_t)gy * pitch + gxh;
-        vt = ty[gi]; vh = h[gi]; vqx = qx[gi]; vqy = qy[gi]; vz = z[gi];
-      }
-      s.ty[r][c] = vt; s.h[r][c] = vh; s.qx[r][c] = vqx; s.qy[r][c] = vqy; s.z[r][c] = vz;
-    }
-  }
-
-  const T t = T(a.ctrl->t);
-  const T dt = T(a.ctrl->dt);
-  const T dx = T(a.dx);
-  const T dt_dx = dt / dx;
-  SeriesRows rows;
-  rows.d = a.given_depth ? series_row<T>((const T*)a.given_depth, a.gd_rows, a.gd_w, t) : 0;
-  rows.w = a.given_wl ? series_row<T>((const T*)a.given_wl, a.gwl_rows, a.gwl_w, t) : 0;
-  rows.q = a.given_q ? series_row<T>((const T*)a.given_q, a.gq_rows, a.gq_w, t) : 0;
-  __syncthreads();
-
-  // Edges touching the tile: x-edges (row ly, between local columns lx-1 = A
-  // and lx = B, lx = 0..64) and y-edges (column lx, between local rows ly-1 =
-  // A and ly = B, ly = 0..TY).  The owner of cell (ly, lx) solves its west
-  // and north edges, in the same passes for every wave (one direction per
-  // pass); the last x-edge column runs in wave 0 and the last y-edge row in
-  // wave 1.  B parts stay in registers, A parts go to LDS.
-  constexpr int kRec = Tile::kRec, kSide = Tile::kSide;
-  T bw[CPT][kSide], bn[CPT][kSide];  // the own cells' parts of their west and north edges
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int ly = wv + 4 * k, lx = lane;
-    T rec[kRec];
-    solve_tile_edge<T, ORDER, TY, 0>(s, a, rows, ly + 2, lx + 1, dx, dt, dt_dx, rec);
-#pragma unroll
-    for (int w = 0; w < kSide; ++w) {
-      bw[k][w] = side_word<T, kRec>(rec, 1, w);
-      if (lx > 0) s.a[0][w][ly][lx - 1] = side_word<T, kRec>(rec, 0, w);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int ly = wv + 4 * k, lx = lane;
-    T rec[kRec];
-    solve_tile_edge<T, ORDER, TY, 3>(s, a, rows, ly + 1, lx + 2, dx, dt, dt_dx, rec);
-#pragma unroll
-    for (int w = 0; w < kSide; ++w) {
-      bn[k][w] = side_word<T, kRec>(rec, 1, w);
-      if (ly > 0) s.a[1][w][ly - 1][lx] = side_word<T, kRec>(rec, 0, w);
-    }
-  }
-  static_assert(TY <= kTX && kThreads >= 2 * kTX, "edge tail layout");
-  if (tid < TY) {
-    T rec[kRec];
-    solve_tile_edge<T, ORDER, TY, 0>(s, a, rows, tid + 2, kTX + 1, dx, dt, dt_dx, rec);
-#pragma unroll
-    for (int w = 0; w < kSide; ++w) s.a[0][w][tid][kTX - 1] = side_word<T, kRec>(rec, 0, w);
-  } else if (tid >= kTX && tid < 2 * kTX) {
-    const int lx = tid - kTX;
-    T rec[kRec];
-    solve_tile_edge<T, ORDER, TY, 3>(s, a, rows, TY + 1, lx + 2, dx, dt, dt_dx, rec);
-#pragma unroll
-    for (int w = 0; w < kSide; ++w) s.a[1][w][TY - 1][lx] = side_word<T, kRec>(rec, 0, w);
-  }
-  __syncthreads();
-
-  const bool t_zero = (t == T(0));
-  T* __restrict__ dh = (T*)a.dh;
-  T* __restrict__ dqx = (T*)a.dqx;
-  T* __restrict__ dqy = (T*)a.dqy;
-  const T cfl_dx = T(a.cfl) * T(a.dx);
-  const bool sums = a.mass_sums != 0;
-  T mn = T(INFINITY);
-  double vol = 0.0, fsum = 0.0, rsum = 0.0;
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int ly = wv + 4 * k, lx = lane;
-    const int gy = y0 + ly, gx = x0 + lx;
-    if (gy >= ny || gx >= nx) continue;
-    const int r = ly + 2, c = lx + 2;
-    T ah = T(0), aqx = T(0), aqy = T(0);
-    bool listed = false;
-    if (s.ty[r][c] != 0) {
-      // fluxMask rule: t == 0, wet, or a wet valid neighbour E, N, W, S that
-      // is not compact cell 0 (fluxMaskGenerator_Kernel.cu:36); the
-      // neighbours are looked at only for a dry cell (the four LDS reads of
-      // that case issue together)
-      listed = t_zero | gt_hs(s.h[r][c]);
-      if (!listed) {
-        const bool w_e = (s.ty[r][c + 1] != 0) & gt_hs(s.h[r][c + 1]) & !(gx + 1 == a.cell0_x && gy == a.cell0_y);
-        const bool w_n = (s.ty[r - 1][c] != 0) & gt_hs(s.h[r - 1][c]) & !(gx == a.cell0_x && gy - 1 == a.cell0_y);
-        const bool w_w = (s.ty[r][c - 1] != 0) & gt_hs(s.h[r][c - 1]) & !(gx - 1 == a.cell0_x && gy == a.cell0_y);
-        const bool w_s = (s.ty[r + 1][c] != 0) & gt_hs(s.h[r + 1][c]) & !(gx == a.cell0_x && gy + 1 == a.cell0_y);
-        listed = w_e | w_n | w_w | w_s;
-      }
-      if (listed) {
-        T eE[kSide], eS[kSide];  // this cell is A of its east and south edges
-#pragma unroll
-        for (int w = 0; w < kSide; ++w) {
-          eE[w] = s.a[0][w][ly][lx];
-          eS[w] = s.a[1][w][ly][lx];
-        }
-        const T* eN = bn[k];  // B of its north edge
-        const T* eW = bw[k];  // B of its west edge
-        // the reference's order: E, N, W, S; per edge HLLC terms then bed term
-        if (kRec == 5) {
-          ah -= eE[0]; aqx -= eE[1]; aqx -= eE[3]; aqy -= eE[2];
-          ah -= -eN[0]; aqx -= -eN[1]; aqy -= -eN[2]; aqy -= eN[3];
-          ah -= -eW[0]; aqx -= -eW[1]; aqx -= eW[3]; aqy -= -eW[2];
-          ah -= eS[0]; aqx -= eS[1]; aqy -= eS[2]; aqy -= eS[3];
-        } else {
-          ah -= eE[0]; aqx -= eE[2]; aqy -= eE[1];
-          ah += eN[0]; aqx += eN[1]; aqy += eN[2];
-          ah += eW[0]; aqx += eW[2]; aqy += eW[1];
-          ah -= eS[0]; aqx -= eS[1]; aqy -= eS[2];
-        }
-      }
-    }
-    const int64_t gi = (int64_t)gy * pitch + gx;
-    if (!FUSED) {
-      dh[gi] = ah;
-      dqx[gi] = aqx;
-      dqy[gi] = aqy;
-    } else {
-      if (save_flux) {  // the step's flux as well (a calibration run's saved steps)
-        dh[gi] = ah;
-        dqx[gi] = aqx;
-        dqy[gi] = aqy;
-      }
-      CellIn<T> in = cin[k];
-      if (a.rain_mode == HP_RAIN_STATION)
-        in.rain = (in.st >= 0 && in.st < kRateCache) ? s_rate[in.st] : station_rate<T>(rr, in.st, a.rain_scale);
-      T hn = s.h[r][c], qxn = s.qx[r][c], qyn = s.qy[r][c], hm = in.hmax;
-      // infiltration over the flux list (SWE_CUDA.py:439-443)
-      T dF = T(0);
-      if (a.infil_ks && listed) {
-        dF = green_ampt<T>(hn, in.F, ((const T*)a.infil_ks)[in.cls], ((const T*)a.infil_phi)[in.cls],
-                           ((const T*)a.infil_dtheta)[in.cls], dt);
-        ((T*)a.infil_F)[gi] = in.F + dF;
-      }
-      T cand, vh, fh, rh;
-      update_state<T>(in, hn, qxn, qyn, ah, aqx, aqy, dF, dt, cfl_dx, hm, cand, vh, fh, rh, time_control);
-      if (time_control) {
-        mn = fmin(mn, cand);
-        if (sums) {
-          vol += (double)vh;
-          fsum += (double)fh;
-          rsum += (double)rh;
-        }
-      }
-      ((T*)a.h_out)[gi] = hn;
-      ((T*)a.qx_out)[gi] = qxn;
-      ((T*)a.qy_out)[gi] = qyn;
-      if (hm != in.hmax) ((T*)a.h_max)[gi] = hm;
-    }
-  }
-  if (FUSED && time_control) block_partial<T>(mn, vol, fsum, rsum, part, pidx, sums);
-}
-
-template <class T, int ORDER, int TY>
-__global__ __launch_bounds__(kThreads) void k_flux(hp_grid_desc a, int ntx) {
-  const int tile = xcd_band(blockIdx.x, gridDim.x);
-  flux_tile<T, ORDER, TY, false>(a, tile % ntx, tile / ntx, Partials(nullptr, 0), 0);
-}
-
-template <class T, int ORDER, int TY>
-__global__ __launch_bounds__(kThreads) void k_flux_multi(const hp_grid_desc* __restrict__ doms,
-                                                         const int2* __restrict__ map) {
-  const int2 m = map[xcd_band(blockIdx.x, gridDim.x)];
-  const hp_grid_desc& a = doms[m.x];
-  const int ntx = (a.nx + kTX - 1) / kTX;
-  flux_tile<T, ORDER, TY, false>(a, m.y % ntx, m.y / ntx, Partials(nullptr, 0), 0);
-}
-
-// Single-pass step of every tile of every domain of an ensemble; map[i] =
-// (domain, tile), listed domain by domain, so the partial records of a domain
-// are one contiguous range.
-template <class T, int ORDER, int TY>
-__global__ __launch_bounds__(kThreads) void k_step_fused_multi(const hp_grid_desc* __restrict__ doms,
-                                                               const int2* __restrict__ map, void* parts,
-                                                               int n_total) {
-  const int slot = xcd_band(blockIdx.x, gridDim.x);
-  const int2 m = map[slot];
-  const hp_grid_desc& a = doms[m.x];
-  const int ntx = (a.nx + kTX - 1) / kTX;
-  flux_tile<T, ORDER, TY, true>(a, m.y % ntx, m.y / ntx, Partials(parts, n_total), slot);
-}
-
-// Single-pass step: reads (h, qx, qy), writes (h_out, qx_out, qy_out).
-template <class T, int ORDER, int TY>
-// flags: 1 also save the step's flux in dh, dqx, dqy; 2 no time-control
-// outputs (a frozen schedule); 4 a stopped domain copies its state to the
-// output planes even when the time control marked both sets in step.
-__global__ __launch_bounds__(kThreads) void k_step_fused(hp_grid_desc a, int ntx, int flags) {
-  // the partial record goes to the tile's own slot (tile order, as in an
-  // ensemble), not the block's
-  const int tile = xcd_band(blockIdx.x, gridDim.x);
-  flux_tile<T, ORDER, TY, true>(a, tile % ntx, tile / ntx, Partials(a.work, gridDim.x), tile, (flags & 1) != 0,
-                                (flags & 2) == 0, (flags & 4) != 0);
-}
-
 }  // namespace hp
 
 #include "swe_walk.hpp"
@@ -726,7 +287,7 @@ __device__ inline void update_chunk(const hp_grid_desc& a, int64_t chunk, const 
   const T dt = T(a.ctrl->dt);
   const T cfl_dx = T(a.cfl) * T(a.dx);
   for (int k = tid; k < a.n_classes; k += kThreads) s_man[k] = ((const T*)a.manning)[k];
-  const RainRows rr = rain_rows(a, a.ctrl->t);
+  const RainRows rr = wave_rain_rows(&a, a.ctrl->t);
   const int mode = a.rain_mode;
   if (mode == HP_RAIN_STATION && tid < kRateCache) s_rate[tid] = station_rate<T>(rr, tid, a.rain_scale);
   __syncthreads();
@@ -961,21 +522,55 @@ static int64_t update_blocks(const hp_grid_desc* g) {
   return (total + kChunk - 1) / kChunk;
 }
 
-// Rows per flux work unit: FP32 column-walk units of 60 columns x 2, 4, 6,
-// 8, 10, 12 or 16 rows (default 8); FP64 LDS tiles of 64 x 4 or 64 x 8 cells
-// (default 4).  Every launch of a domain's units takes its height from here.
-static int flux_rows(const hp_grid_desc* g) {
-  const int r = g->tile_rows;
-  if (g->dtype == HP_F32) return (r == 2 || r == 4 || r == 6 || r == 10 || r == 12 || r == 16) ? r : 8;
-  return r == 8 ? 8 : 4;
+static int64_t units(const hp_grid_desc* g, int cols, int rows) {
+  return (int64_t)((g->nx + cols - 1) / cols) * (int64_t)((g->ny + rows - 1) / rows);
 }
 
-static int flux_cols(const hp_grid_desc* g) { return g->dtype == HP_F32 ? kWalkOwn : kTX; }
+// Rows per flux work unit (60 columns wide): a height asked for by tile_rows
+// (2, 4, 6, 8, 10, 12 or 16 in float, 4 or 8 in double), else 0.
+static int asked_rows(const hp_grid_desc* g) {
+  const int r = g->tile_rows;
+  if (g->dtype == HP_F32) return (r == 2 || r == 4 || r == 6 || r == 8 || r == 10 || r == 12 || r == 16) ? r : 0;
+  return r == 4 || r == 8 ? r : 0;
+}
+
+// What a domain's height counts as where heights are compared and sizes are
+// checked (a domain that asks for none: 8 in float, 4 in double).
+static int nominal_rows(const hp_grid_desc* g) {
+  const int r = asked_rows(g);
+  return r ? r : (g->dtype == HP_F32 ? 8 : 4);
+}
+
+// The height where none is asked for, from the number of units of height 1
+// (of one domain, or of all the domains of an ensemble).  A taller unit
+// spreads its prologue (four rows loaded, an edge solved twice, the tables)
+// over more rows, but the launch ends with some units walking alone, at about
+// 2 us a row whatever else runs: doubling the height pays while enough
+// shorter units remain to hide that.  Measured per step, order 2 (height:
+// us), float 384^2 1: 13.9, 2: 15.0; 512^2 1: 17.1, 2: 16.4, 4: 19.5; 1024^2
+// 2: 31.5, 4: 29.9, 8: 34.5; 1536^2 4: 48.2, 8: 46.5, 16: 57.2; 2048^2
+// 4: 71.5, 8: 67.9, 16: 75.6; 4096^2 8: 228, 16: 219, 32: 230; 6000^2 16: 446,
+// 32: 439; double 384^2 1: 20.4, 2: 21.7; 1024^2 2: 63.3, 4: 60.8, 8: 64.9;
+// 2048^2 4: 166, 8: 157, 16: 172; 3000^2 8: 326, 16: 320.  The line below lies
+// between the two sides of each of these.
+static int chosen_rows(int64_t rows1) {
+  int r = 1;
+  while (r < 32 && rows1 / (2 * r) >= 1000 + 480 * (2 * r)) r *= 2;
+  return r;
+}
+
+static int flux_rows(const hp_grid_desc* g) {
+  const int r = asked_rows(g);
+  return r ? r : chosen_rows(units(g, kWalkOwn, 1));
+}
 
 // Flux work units of a domain: one partial record each in the single-pass step.
-static int64_t flux_tiles(const hp_grid_desc* g) {
-  const int ty = flux_rows(g), tx = flux_cols(g);
-  return (int64_t)((g->nx + tx - 1) / tx) * (int64_t)((g->ny + ty - 1) / ty);
+static int64_t flux_tiles(const hp_grid_desc* g) { return units(g, kWalkOwn, flux_rows(g)); }
+
+// Units a domain of its nominal height has had in every version (64-column
+// tiles in double): the records a workspace is sized for hold at least these.
+static int64_t nominal_tiles(const hp_grid_desc* g) {
+  return units(g, g->dtype == HP_F32 ? kWalkOwn : 64, nominal_rows(g));
 }
 
 static int check_desc(const hp_grid_desc* g) {
@@ -1022,64 +617,25 @@ static int check_desc(const hp_grid_desc* g) {
   return HP_OK;
 }
 
-template <class T, int ORDER, int TY>
-static int launch_flux_single(const hp_grid_desc* g, hipStream_t st) {
-  const int ntx = (g->nx + kTX - 1) / kTX, nty = (g->ny + TY - 1) / TY;
-  hipLaunchKernelGGL((k_flux<T, ORDER, TY>), dim3(ntx * nty), dim3(kThreads), 0, st, *g, ntx);
-  return check_launch("k_flux");
-}
-
-// FP32: column-walk units (k_walk), 64-lane workgroups.
-template <int ORDER, int R, bool FUSED>
-static int launch_walk_r(const hp_grid_desc* g, hipStream_t st, int flags) {
-  const int ns = (g->nx + kWalkOwn - 1) / kWalkOwn, nb = (g->ny + R - 1) / R;
-  hipLaunchKernelGGL((k_walk<ORDER, R, FUSED>), dim3(ns * nb), dim3(kWalkLanes), 0, st, *g, ns, flags);
+template <class T, int ORDER, bool FUSED>
+static int launch_walk_t(const hp_grid_desc* g, hipStream_t st, int flags) {
+  const int rows = flux_rows(g), ns = (g->nx + kWalkOwn - 1) / kWalkOwn;
+  hipLaunchKernelGGL((k_walk<T, ORDER, FUSED>), dim3((unsigned)units(g, kWalkOwn, rows)), dim3(kWalkLanes), 0, st, *g,
+                     Divisor::of(ns), rows, flags);
   return check_launch(FUSED ? "k_walk (single-pass step)" : "k_walk (flux pass)");
-}
-
-template <int ORDER, bool FUSED>
-static int launch_walk_o(const hp_grid_desc* g, hipStream_t st, int flags) {
-  switch (flux_rows(g)) {
-    case 2: return launch_walk_r<ORDER, 2, FUSED>(g, st, flags);
-    case 4: return launch_walk_r<ORDER, 4, FUSED>(g, st, flags);
-    case 6: return launch_walk_r<ORDER, 6, FUSED>(g, st, flags);
-    case 10: return launch_walk_r<ORDER, 10, FUSED>(g, st, flags);
-    case 12: return launch_walk_r<ORDER, 12, FUSED>(g, st, flags);
-    case 16: return launch_walk_r<ORDER, 16, FUSED>(g, st, flags);
-    default: return launch_walk_r<ORDER, 8, FUSED>(g, st, flags);
-  }
 }
 
 template <bool FUSED>
 static int launch_walk(const hp_grid_desc* g, hipStream_t st, int flags) {
-  return g->order == 2 ? launch_walk_o<2, FUSED>(g, st, flags) : launch_walk_o<1, FUSED>(g, st, flags);
+  if (g->dtype == HP_F32)
+    return g->order == 2 ? launch_walk_t<float, 2, FUSED>(g, st, flags) : launch_walk_t<float, 1, FUSED>(g, st, flags);
+  return g->order == 2 ? launch_walk_t<double, 2, FUSED>(g, st, flags) : launch_walk_t<double, 1, FUSED>(g, st, flags);
 }
 
-template <int ORDER>
-static int launch_flux_f64(const hp_grid_desc* g, hipStream_t st) {
-  return flux_rows(g) == 8 ? launch_flux_single<double, ORDER, 8>(g, st) : launch_flux_single<double, ORDER, 4>(g, st);
-}
-
-static int launch_flux(const hp_grid_desc* g, hipStream_t st) {
-  if (g->dtype == HP_F32) return launch_walk<false>(g, st, 0);
-  return g->order == 2 ? launch_flux_f64<2>(g, st) : launch_flux_f64<1>(g, st);
-}
-
-template <class T, int ORDER, int TY>
-static int launch_fused_t(const hp_grid_desc* g, hipStream_t st, int flags) {
-  const int ntx = (g->nx + kTX - 1) / kTX, nty = (g->ny + TY - 1) / TY;
-  hipLaunchKernelGGL((k_step_fused<T, ORDER, TY>), dim3(ntx * nty), dim3(kThreads), 0, st, *g, ntx, flags);
-  return check_launch("k_step_fused");
-}
-
-template <int ORDER>
-static int launch_fused_f64(const hp_grid_desc* g, hipStream_t st, int flags) {
-  return flux_rows(g) == 8 ? launch_fused_t<double, ORDER, 8>(g, st, flags) : launch_fused_t<double, ORDER, 4>(g, st, flags);
-}
+static int launch_flux(const hp_grid_desc* g, hipStream_t st) { return launch_walk<false>(g, st, 0); }
 
 static int launch_step_fused(const hp_grid_desc* g, hipStream_t st, int flags = 0) {
-  if (g->dtype == HP_F32) return launch_walk<true>(g, st, flags);
-  return g->order == 2 ? launch_fused_f64<2>(g, st, flags) : launch_fused_f64<1>(g, st, flags);
+  return launch_walk<true>(g, st, flags);
 }
 
 static int launch_finalize_fused(const hp_grid_desc* g, hipStream_t st, const StepRecord* rec = nullptr) {
@@ -1139,10 +695,22 @@ struct EnsembleLayout {
 };
 
 
+// The unit height of an ensemble: the one its domains ask for (all the same),
+// else by the units of all of them, which share one launch.
+static int ensemble_rows(int32_t n, const hp_grid_desc* d) {
+  int64_t rows1 = 0;
+  for (int k = 0; k < n; ++k) {
+    if (asked_rows(&d[k])) return asked_rows(&d[k]);
+    rows1 += units(&d[k], kWalkOwn, 1);
+  }
+  return chosen_rows(rows1);
+}
+
 static EnsembleLayout ensemble_layout(int32_t n, const hp_grid_desc* d) {
   EnsembleLayout L{};
+  const int rows = ensemble_rows(n, d);
   for (int k = 0; k < n; ++k) {
-    L.n_ftiles += flux_tiles(&d[k]);
+    L.n_ftiles += units(&d[k], kWalkOwn, rows);
     L.n_ublocks += update_blocks(&d[k]);
   }
   L.off_doms = 0;
@@ -1155,62 +723,31 @@ static EnsembleLayout ensemble_layout(int32_t n, const hp_grid_desc* d) {
   return L;
 }
 
-template <class T, int ORDER, int TY>
-static void launch_flux_multi(const hp_ensemble* e, hipStream_t st) {
-  hipLaunchKernelGGL((k_flux_multi<T, ORDER, TY>), dim3((unsigned)e->n_flux_tiles), dim3(kThreads), 0, st,
-                     (const hp_grid_desc*)e->doms, (const int2*)e->flux_map);
-}
-
 template <class T>
 static void launch_update_multi(const hp_ensemble* e, hipStream_t st) {
   hipLaunchKernelGGL((k_update_multi<T, HP_UPDATE_STEP>), dim3((unsigned)e->n_update_blocks), dim3(kThreads), 0, st,
                      (const hp_grid_desc*)e->doms, (const int2*)e->update_map, e->partials);
 }
 
-template <class T, int ORDER, int TY>
-static void launch_fused_multi(const hp_ensemble* e, int parity, hipStream_t st) {
-  hipLaunchKernelGGL((k_step_fused_multi<T, ORDER, TY>), dim3((unsigned)e->n_flux_tiles), dim3(kThreads), 0, st,
-                     (const hp_grid_desc*)e->doms + (parity ? e->n_domains : 0), (const int2*)e->flux_map,
-                     e->partials, (int)e->n_flux_tiles);
-}
-
-template <int ORDER, int R, bool FUSED>
+template <class T, int ORDER, bool FUSED>
 static void launch_walk_multi(const hp_ensemble* e, int parity, hipStream_t st) {
-  hipLaunchKernelGGL((k_walk_multi<ORDER, R, FUSED>), dim3((unsigned)e->n_flux_tiles), dim3(kWalkLanes), 0, st,
+  hipLaunchKernelGGL((k_walk_multi<T, ORDER, FUSED>), dim3((unsigned)e->n_flux_tiles), dim3(kWalkLanes), 0, st,
                      (const hp_grid_desc*)e->doms + (parity ? e->n_domains : 0), (const int2*)e->flux_map,
-                     e->partials, (int)e->n_flux_tiles);
-}
-
-template <int ORDER, bool FUSED>
-static void launch_walk_multi_o(const hp_ensemble* e, int parity, hipStream_t st) {
-  switch (e->tile_rows) {
-    case 2: return launch_walk_multi<ORDER, 2, FUSED>(e, parity, st);
-    case 4: return launch_walk_multi<ORDER, 4, FUSED>(e, parity, st);
-    case 6: return launch_walk_multi<ORDER, 6, FUSED>(e, parity, st);
-    case 10: return launch_walk_multi<ORDER, 10, FUSED>(e, parity, st);
-    case 12: return launch_walk_multi<ORDER, 12, FUSED>(e, parity, st);
-    case 16: return launch_walk_multi<ORDER, 16, FUSED>(e, parity, st);
-    default: return launch_walk_multi<ORDER, 8, FUSED>(e, parity, st);
-  }
+                     e->partials, (int)e->n_flux_tiles, (int)e->tile_rows);
 }
 
 template <bool FUSED>
 static void launch_walk_multi_any(const hp_ensemble* e, int parity, hipStream_t st) {
-  if (e->order == 2) launch_walk_multi_o<2, FUSED>(e, parity, st);
-  else launch_walk_multi_o<1, FUSED>(e, parity, st);
+  if (e->dtype == HP_F32)
+    (e->order == 2 ? launch_walk_multi<float, 2, FUSED> : launch_walk_multi<float, 1, FUSED>)(e, parity, st);
+  else (e->order == 2 ? launch_walk_multi<double, 2, FUSED> : launch_walk_multi<double, 1, FUSED>)(e, parity, st);
 }
 
 // One single-pass step of every domain: even steps read the domains' own
 // planes and write their second set, odd steps the reverse.
 static int ensemble_fused_step_once(const hp_ensemble* e, int parity, hipStream_t st) {
-  if (e->dtype == HP_F32) {
-    launch_walk_multi_any<true>(e, parity, st);
-  } else {
-    const bool t8 = e->tile_rows == 8;
-    if (e->order == 2) (t8 ? launch_fused_multi<double, 2, 8> : launch_fused_multi<double, 2, 4>)(e, parity, st);
-    else (t8 ? launch_fused_multi<double, 1, 8> : launch_fused_multi<double, 1, 4>)(e, parity, st);
-  }
-  int rc = check_launch("k_step_fused_multi");
+  launch_walk_multi_any<true>(e, parity, st);
+  int rc = check_launch("k_walk_multi (single-pass step)");
   if (rc) return rc;
   hipLaunchKernelGGL(k_finalize_multi, dim3((unsigned)e->n_domains), dim3(1024), 0, st,
                      (const hp_grid_desc*)e->doms, (const int2*)e->fused_finalize_map, e->partials,
@@ -1220,14 +757,8 @@ static int ensemble_fused_step_once(const hp_ensemble* e, int parity, hipStream_
 
 static int ensemble_step_once(const hp_ensemble* e, hipStream_t st) {
   const bool f32 = e->dtype == HP_F32;
-  if (f32) {
-    launch_walk_multi_any<false>(e, 0, st);
-  } else {
-    const bool t8 = e->tile_rows == 8;
-    if (e->order == 2) (t8 ? launch_flux_multi<double, 2, 8> : launch_flux_multi<double, 2, 4>)(e, st);
-    else (t8 ? launch_flux_multi<double, 1, 8> : launch_flux_multi<double, 1, 4>)(e, st);
-  }
-  int rc = check_launch("k_flux_multi");
+  launch_walk_multi_any<false>(e, 0, st);
+  int rc = check_launch("k_walk_multi (flux pass)");
   if (rc) return rc;
   if (f32) launch_update_multi<float>(e, st);
   else launch_update_multi<double>(e, st);
@@ -1311,8 +842,7 @@ static int scratch_ptr(void** out) {
 // Workspace of a domain: the partial records of the larger of the update
 // pass and the flux / single-pass step.
 static int64_t workspace_need(const hp_grid_desc* g) {
-  const int64_t nt = flux_tiles(g), nu = update_blocks(g);
-  return partials_bytes(nu > nt ? nu : nt);
+  return partials_bytes(std::max({flux_tiles(g), nominal_tiles(g), update_blocks(g)}));
 }
 
 // The checks every single-pass entry point makes.
@@ -1380,7 +910,7 @@ int64_t hp_grid_noalloc_max_bytes(void) { return kScratchBytes; }
 int hp_grid_step_fused_noalloc(const hp_grid_desc* g, int32_t nsteps, void* stream) {
   int rc = check_desc(g);
   if (rc) return rc;
-  const int64_t need = workspace_need(g);
+  const int64_t need = partials_bytes(std::max(nominal_tiles(g), update_blocks(g)));
   if (need > kScratchBytes)
     return fail(HP_ESPACE, "domain needs " + std::to_string(need) + " bytes of per-tile records; the allocation-free "
                            "step holds at most " + std::to_string(kScratchBytes) + " (use hp_grid_step_fused)");
@@ -1390,6 +920,9 @@ int hp_grid_step_fused_noalloc(const hp_grid_desc* g, int32_t nsteps, void* stre
   hp_grid_desc d = *g;
   d.work = p;
   d.work_bytes = kScratchBytes;
+  // (an asked height whose 60-column units have more records than its
+  // nominal tiles gives way to the chosen one, which has fewer)
+  if (workspace_need(&d) > kScratchBytes) d.tile_rows = 0;
   return hp_grid_step_fused(&d, nsteps, stream);
 }
 
@@ -1505,7 +1038,7 @@ int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, 
     if (single_pass && (!descs[k].h_out || !descs[k].qx_out || !descs[k].qy_out))
       return fail(HP_EINVAL, "domain " + std::to_string(k) + ": the single-pass step needs h_out, qx_out, qy_out");
     if (descs[k].dtype != descs[0].dtype || descs[k].order != descs[0].order ||
-        flux_rows(&descs[k]) != flux_rows(&descs[0]))
+        nominal_rows(&descs[k]) != nominal_rows(&descs[0]))
       return fail(HP_EINVAL, "every domain of an ensemble needs the same dtype, order and tile_rows");
   }
   const EnsembleLayout L = ensemble_layout(n, descs);
@@ -1525,8 +1058,9 @@ int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, 
   int32_t* fin = (int32_t*)(host.data() + L.off_fin);
   int32_t* fin1 = (int32_t*)(host.data() + L.off_fin1);
   int64_t fi = 0, ui = 0;
+  const int rows = ensemble_rows(n, descs);
   for (int k = 0; k < n; ++k) {
-    const int64_t nt = flux_tiles(&descs[k]), nu = update_blocks(&descs[k]);
+    const int64_t nt = units(&descs[k], kWalkOwn, rows), nu = update_blocks(&descs[k]);
     fin1[2 * k] = (int32_t)fi;
     fin1[2 * k + 1] = (int32_t)nt;
     for (int64_t j = 0; j < nt; ++j, ++fi) {
@@ -1547,7 +1081,7 @@ int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, 
   out->n_domains = n;
   out->dtype = descs[0].dtype;
   out->order = descs[0].order;
-  out->tile_rows = flux_rows(&descs[0]);
+  out->tile_rows = rows;
   out->n_flux_tiles = (int32_t)L.n_ftiles;
   out->n_update_blocks = (int32_t)L.n_ublocks;
   out->doms = w + L.off_doms;

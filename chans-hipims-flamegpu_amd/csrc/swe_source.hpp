@@ -44,27 +44,56 @@ struct RainRows {
   bool zero;         // every station rate is 0 (after the table, or one row)
 };
 
-// The descriptor through any pointer type (generic, or the kernel-argument
-// address space).
-template <class DP> __device__ inline RainRows rain_rows_at(DP a, double t_now) {
+// The smallest i in [from, to) for which hit(i), else `to`: the answer of a
+// loop from `from` upwards, found 64 candidates at a time by the whole wave
+// (all lanes active, the arguments the same in every lane).  Tables of a
+// storm hold hundreds of rows (289 rows of five minutes make a day), and a
+// loop pays a memory round trip for each: the 37th row of such a table cost a
+// block of the update pass about 12 us.
+template <class F> __device__ inline int wave_first(int from, int to, F hit) {
+  const int lane = (int)(threadIdx.x & 63);
+  for (int base = from; base < to; base += 64) {
+    const int i = base + lane;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(i < to && hit(i));
+    if (m) return __builtin_amdgcn_readfirstlane(base + (int)__builtin_ctzll(m));
+  }
+  return to;
+}
+
+// The bracketing rows at t_now, through any pointer type of the descriptor
+// (generic, or the kernel-argument address space); called by whole waves.
+template <class DP> __device__ inline RainRows wave_rain_rows(DP a, double t_now) {
   RainRows r{nullptr, nullptr, 0.0, 0, true};
   if (a->rain_mode != HP_RAIN_STATION || a->rain_table == nullptr || a->rain_rows <= 0) return r;
   const int rows = a->rain_rows, cols = a->rain_cols;
   const double* tab = a->rain_table;
   r.n_st = cols - 1;
-  const bool after = !(t_now < tab[(rows - 1) * cols]);
-  int i = 0;
-  while (i + 1 < rows - 1 && !(t_now < tab[(i + 1) * cols])) i++;
-  r.zero = after || rows <= 1;
-  if (!r.zero) {
-    r.lo = tab + i * cols + 1;
-    r.hi = tab + (i + 1) * cols + 1;
-    r.per = (t_now - tab[i * cols]) / (tab[(i + 1) * cols] - tab[i * cols]);
+  if (rows <= 1) return r;
+  int i;  // the last row whose successor lies after t_now (the table's last two rows at most)
+  double t0, t1;
+  if (rows <= 64) {
+    // a row per lane: one memory round trip
+    const int lane = (int)(threadIdx.x & 63);
+    const double t = tab[(int64_t)(lane < rows ? lane : 0) * cols];
+    const uint64_t later = __builtin_amdgcn_ballot_w64(lane < rows && t_now < t);
+    r.zero = !(later >> (rows - 1) & 1);
+    if (r.zero) return r;
+    const uint64_t inner = later & ((uint64_t(1) << (rows - 1)) - 2);  // rows 1 .. rows - 2
+    i = inner ? (int)__builtin_ctzll(inner) - 1 : rows - 2;
+    t0 = __shfl(t, i, 64);
+    t1 = __shfl(t, i + 1, 64);
+  } else {
+    r.zero = !(t_now < tab[(int64_t)(rows - 1) * cols]);
+    if (r.zero) return r;
+    i = wave_first(0, rows - 2, [&](int k) { return t_now < tab[(int64_t)(k + 1) * cols]; });
+    t0 = tab[(int64_t)i * cols];
+    t1 = tab[(int64_t)(i + 1) * cols];
   }
+  r.lo = tab + (int64_t)i * cols + 1;
+  r.hi = r.lo + cols;
+  r.per = (t_now - t0) / (t1 - t0);
   return r;
 }
-
-__device__ inline RainRows rain_rows(const hp_grid_desc& a, double t_now) { return rain_rows_at(&a, t_now); }
 
 // Rain rate of a cell whose station index is k.
 template <class T> __device__ inline T station_rate(const RainRows& rr, int k, double scale) {

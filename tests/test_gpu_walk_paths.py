@@ -56,3 +56,60 @@ def test_double_walk_matches_oracle(oracle_lib, cuda, ny, nx, order):
     for k, ref in (("h", o.h_c), ("qx", o.qx_c), ("qy", o.qy_c)):
         assert rel_err(compact(m, s.raster(getattr(s, k))), ref) <= 1e-10, k
     assert abs(s.dt - o.dt) <= 1e-12 * o.dt
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("ny,nx", [(6, 400), (520, 530), (1030, 1000)])
+def test_chosen_unit_height_changes_no_bits(cuda, ny, nx, dtype):
+    """The chosen height (1, 2 and 4 at these sizes) against one asked for."""
+    res = []
+    for rows in (0, 8):
+        s = GridSolver(*domain(ny, nx, 1, 1), 1.0, order=2, dtype=dtype, first_dt=0.02, t=1.0, manning=[0.03],
+                       tile_rows=rows)
+        s.step_fused(3)
+        res.append([getattr(s, k).clone() for k in ("h", "qx", "qy", "h_max")] + [s.ctrl[:2].clone()])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("rows", [1, 2, 3, 63, 64, 65, 129, 289])
+def test_rain_table_rows(cuda, rows, fused):
+    """The bracketing rows of a rain table, at, between and beyond them: a dry
+    flat box holds rate * dt after one step."""
+    rng = np.random.Generator(np.random.PCG64(rows))
+    tab = np.column_stack([300.0 * np.arange(rows), rng.uniform(1e-5, 2e-5, (rows, 3))])
+    mask = np.full((7, 72), -9999)
+    mask[1:-1, 1:-1] = 40
+    st = np.arange(mask.size).reshape(mask.shape) % 3
+    zero = np.zeros(mask.shape)
+    for t in sorted({0.0, 10.0, 300.0 * (rows // 2), 300.0 * (rows // 2) + 77.0, 300.0 * (rows - 2) + 299.0,
+                     300.0 * (rows - 1), 300.0 * rows}):
+        if t < 0:
+            continue
+        s = GridSolver(mask, zero, zero, zero, zero, 1.0, order=1, dtype=torch.float64, first_dt=1.0, t=t)
+        s.set_station_rain(tab, st)
+        s.step_fused(1) if fused else s.step(1)
+        want = np.zeros(3)
+        if t < tab[-1, 0]:
+            want = np.array([np.interp(t, tab[:, 0], tab[:, 1 + k]) for k in range(3)])
+        got = s.raster(s.h)[mask > 0]
+        assert np.abs(got - want[st[mask > 0]]).max() <= 1e-15, (rows, t)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 64, 65, 130])
+def test_boundary_series_rows(oracle_lib, cuda, rows):
+    """The row of a boundary series in force (the first whose time is not
+    before t), against the oracle."""
+    m, h, qx, qy, z = domain(12, 70, 1, 1)
+    m[2:8, 1] = 70
+    rng = np.random.Generator(np.random.PCG64(rows))
+    q = np.column_stack([100.0 * np.arange(rows), rng.uniform(0.1, 0.5, (rows, 2))])
+    for t in (1.0, 100.0 * (rows // 2), 100.0 * (rows // 2) + 1.0, 100.0 * rows + 5.0):
+        kw = dict(order=2, first_dt=0.02, t=t, manning=np.array([0.03]), given_q=q)
+        s = GridSolver(m, h, qx, qy, z, 1.0, dtype=torch.float64, **kw)
+        o = oracle_lib.OracleSim(m, h, qx, qy, z, 1.0, **kw)
+        s.step_fused(1)
+        o.run(1)
+        for k, ref in (("h", o.h_c), ("qx", o.qx_c), ("qy", o.qy_c)):
+            assert rel_err(compact(m, s.raster(getattr(s, k))), ref) <= 1e-10, (k, rows, t)
