@@ -79,35 +79,54 @@ template <class T> __device__ inline void to_global(T fn, T ft, int d, T& gx, T&
 }
 
 // --- reductions ------------------------------------------------------------
-// Time control of one domain from its step's folded CFL minimum and FP64
-// sums (one thread): dt = min of the candidates (kept when no cell was
-// listed, SWE_CUDA.py:818-822), capped at 10x the previous dt, clamped onto
-// the next export time, then t advanced by it (SWE_CUDA.py:824-831).
-// c: the control block as it was read at the start of the pass (nothing
-// else writes it meanwhile).
-__device__ inline void advance_ctrl(hp_ctrl* ctrl, const hp_ctrl& c, double mn, double vol, double fs, double rs,
-                                    double dx, bool sums) {
-  const double area = dx * dx;
-  const double t = c.t;
-  const double dt_old = c.dt;
-  double dt_new = isinf(mn) ? dt_old : mn;
-  const double upper = dt_old * 10.0;
-  dt_new = (upper < dt_new) ? upper : dt_new;
+// The fields of a control block that a step advances, and those they depend on.
+struct StepCtrl {
+  double t, dt, export_T, export_n, export_pending, steps, t_stop, synced;
+  template <class CP> static __device__ StepCtrl of(CP c) {
+    return StepCtrl{c->t, c->dt, c->export_T, c->export_n, c->export_pending, c->steps, c->t_stop, c->stopped_synced};
+  }
+  __device__ bool stopped() const { return t_stop > 0.0 && t >= t_stop; }
+  __device__ void put(hp_ctrl* c) const {
+    c->t = t;
+    c->dt = dt;
+    c->export_n = export_n;
+    c->export_pending = export_pending;
+    c->steps = steps;
+    c->stopped_synced = synced;
+  }
+};
+
+// Time control of one domain from its step's folded CFL minimum: dt = min of
+// the candidates (kept when no cell was listed, SWE_CUDA.py:818-822), capped at
+// 10x the previous dt, clamped onto the next export time, then t advanced by
+// it (SWE_CUDA.py:824-831).  The FP64 sums are the caller's.
+__device__ inline StepCtrl next_ctrl(const StepCtrl& c, double mn) {
+  double dt = isinf(mn) ? c.dt : mn;
+  const double upper = c.dt * 10.0;
+  dt = (upper < dt) ? upper : dt;
   const double next_export = (c.export_n + 1.0) * c.export_T;
-  if (dt_new + t >= next_export) {
-    dt_new = next_export - t;
-    ctrl->export_n = c.export_n + 1.0;
-    ctrl->export_pending = c.export_pending + 1.0;
-  }
-  ctrl->dt = dt_new;
-  ctrl->t = t + dt_new;
-  if (sums) {
-    ctrl->volume = vol * area;
-    ctrl->flux_volume = c.flux_volume + fs * area;
-    ctrl->rain_volume = c.rain_volume + rs * area;
-  }
-  ctrl->steps = c.steps + 1.0;
-  ctrl->stopped_synced = 0.0;
+  const bool at_export = dt + c.t >= next_export;
+  const double left = next_export - c.t;
+  dt = at_export ? left : dt;
+  const double one = at_export ? 1.0 : 0.0;
+  return StepCtrl{c.t + dt, dt, c.export_T, c.export_n + one, c.export_pending + one, c.steps + 1.0, c.t_stop, 0.0};
+}
+
+// The same for a step the single-pass kernel ran: on a stopped domain that
+// step left both sets of planes holding the state.
+__device__ inline StepCtrl next_ctrl_single_pass(const StepCtrl& c, double mn) {
+  const StepCtrl e = next_ctrl(c, mn);
+  const bool s = c.stopped();
+  return StepCtrl{s ? c.t : e.t, s ? c.dt : e.dt, c.export_T, s ? c.export_n : e.export_n,
+                  s ? c.export_pending : e.export_pending, s ? c.steps : e.steps, c.t_stop, s ? 1.0 : 0.0};
+}
+
+// A step's FP64 sums into the control block.
+__device__ inline void put_sums(hp_ctrl* ctrl, double vol, double fs, double rs, double dx) {
+  const double area = dx * dx;
+  ctrl->volume = vol * area;
+  ctrl->flux_volume += fs * area;
+  ctrl->rain_volume += rs * area;
 }
 
 // Per-block results of a pass that ends a step, in the workspace: the CFL
@@ -131,15 +150,132 @@ struct Partials {
   }
 };
 
-template <class T> __device__ inline T wave_min(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-  return v;
+// Minimum over the wave, the same in every lane (all lanes active): lane
+// shifts within rows of 16 (row_shr 1, 2, 4, 8: lane 15 holds its row's), then
+// row to row, into lane 63; the order does not matter.  A lane that has no
+// source keeps its value.  A fraction of the latency of six shuffles through
+// LDS, and in float one instruction each (s_nop: a lane shift reads what the
+// instruction before it wrote).
+template <int CTRL, int ROWS> __device__ inline double shifted(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const int l = (int)(uint32_t)u, h = (int)(uint32_t)(u >> 32);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(l, l, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(h, h, CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ inline double wave_min(double v) {
+  v = fmin(v, shifted<0x111, 0xf>(v));
+  v = fmin(v, shifted<0x112, 0xf>(v));
+  v = fmin(v, shifted<0x114, 0xf>(v));
+  v = fmin(v, shifted<0x118, 0xf>(v));
+  v = fmin(v, shifted<0x142, 0xa>(v));  // row_bcast 15 into rows 1 and 3
+  v = fmin(v, shifted<0x143, 0xc>(v));  // row_bcast 31 into rows 2 and 3
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, 63);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), 63);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ inline float wave_min(float v) {
+  asm("s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "+v"(v));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 __device__ inline double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
+}
+
+// --- time control inside the step kernel --------------------------------
+// A call of several single-pass steps runs no time-control launch between
+// them (a launch costs 4 to 5 us whatever it does, and the gap before it 1 to
+// 2; a 2048^2 float step takes 62).  Each unit of step k posts its CFL minimum
+// into one of kFoldSlots words by an atomic minimum (a non-negative double
+// orders like its bits, so the minimum does not depend on the order), and
+// every unit of step k + 1 folds the slots and advances the time control for
+// itself, from the control block of step k: one load per lane and one wave
+// reduction, in the shadow of the unit's first rows.  64 slots: at most one
+// load per lane, and 2048^2 posts 140 times to each at about 36 ns.
+// Step k posts to slots[k % 3], reads slots[(k - 1) % 3] and clears
+// slots[(k + 1) % 3]; its control block goes from ring[(k - 1) & 1] to
+// ring[k & 1], written by the unit 0.  Records of the FP64 sums take turns the
+// same way: kFoldSumBlocks further blocks of step k + 1 sum step k's as the
+// waves of the time-control kernel do, and the first of them in step k + 2
+// adds these up into the control block (one block for all the records took
+// longer than the step itself at 6 650 units: 30 us).
+constexpr int kFoldSlots = 64;
+constexpr int kFoldSumBlocks = 16;
+struct FoldState {
+  unsigned long long slots[3][kFoldSlots];
+  hp_ctrl ring[2];
+  double wave_sums[2][3][kFoldSumBlocks];  // of step k (k & 1): volume, flux, rain
+  double summed[2];                        // whether step k was one to sum (not stopped)
+};
+constexpr unsigned long long kNoMinimum = 0x7ff0000000000000ull;  // the bits of +infinity
+
+// What a unit of a folded step works on: st null, a step with a time-control
+// launch of its own.
+struct WalkFold {
+  FoldState* st;
+  int k;         // step of the call
+  Sums* records;  // this step's records of the domain's units
+};
+
+// The sum of n records as wave w of a 1024-thread block takes it (thread i adds
+// records i, i + 1024, ... in turn; a wave64 butterfly), by one wave.
+__device__ inline void wave_records(const Sums* __restrict__ part, int n, int w, double& vol, double& fs, double& rs) {
+  const int lane = threadIdx.x & 63;
+  vol = fs = rs = 0.0;
+  for (int k = w * 64 + lane; k < n; k += 1024) {
+    const Sums p = part[k];
+    vol += p.vol;
+    fs += p.flux;
+    rs += p.rain;
+  }
+  vol = wave_sum(vol);
+  fs = wave_sum(fs);
+  rs = wave_sum(rs);
+}
+
+// The sixteen waves' sums in turn (one thread).
+__device__ inline void add_waves(const double (&s)[3][kFoldSumBlocks], double& vol, double& fs, double& rs) {
+  vol = s[0][0];
+  fs = s[1][0];
+  rs = s[2][0];
+  for (int k = 1; k < kFoldSumBlocks; ++k) {
+    vol += s[0][k];
+    fs += s[1][k];
+    rs += s[2][k];
+  }
+}
+
+// Block w of the sum blocks in the launch of step k: wave w of step k - 1's
+// sum; block 0 also brings step k - 2's into the control block (nothing else
+// of the launch touches those fields).
+__device__ inline void fold_sums_block(hp_ctrl* ctrl, FoldState* f, int k, int w, const Sums* prev, int n, double dx) {
+  double vol, fs, rs;
+  if (w == 0 && k >= 2 && threadIdx.x == 0 && f->summed[k & 1] != 0.0) {
+    add_waves(f->wave_sums[k & 1], vol, fs, rs);
+    put_sums(ctrl, vol, fs, rs, dx);
+  }
+  if (k == 0) return;
+  const bool live = !stopped(&f->ring[(k + 1) & 1]);
+  if (live) wave_records(prev, n, w, vol, fs, rs);
+  if (threadIdx.x == 0) {
+    double(&to)[3][kFoldSumBlocks] = f->wave_sums[(k + 1) & 1];
+    if (live) {
+      to[0][w] = vol;
+      to[1][w] = fs;
+      to[2][w] = rs;
+    }
+    if (w == 0) f->summed[(k + 1) & 1] = live ? 1.0 : 0.0;
+  }
 }
 
 // Fold a block's CFL minimum and FP64 sums into its partial slot.
@@ -420,7 +556,7 @@ __device__ inline void finalize_domain(hp_ctrl* ctrl, const double* __restrict__
   constexpr int kU = 24;
   __shared__ double s_red[4][16];
   const int tid = threadIdx.x;
-  const hp_ctrl c = *ctrl;
+  const StepCtrl c = StepCtrl::of(ctrl);
   double mn = INFINITY, vol = 0.0, fs = 0.0, rs = 0.0;
   for (int base = tid; base < n; base += blockDim.x * kU) {
     double v[kU];
@@ -432,7 +568,7 @@ __device__ inline void finalize_domain(hp_ctrl* ctrl, const double* __restrict__
 #pragma unroll
     for (int u = 0; u < kU; ++u) mn = fmin(mn, v[u]);
   }
-  if (stopped(&c)) {
+  if (c.stopped()) {
     if (threadIdx.x == 0) ctrl->stopped_synced = single_pass ? 1.0 : 0.0;
     return;
   }
@@ -470,7 +606,8 @@ __device__ inline void finalize_domain(hp_ctrl* ctrl, const double* __restrict__
       fs += s_red[2][k];
       rs += s_red[3][k];
     }
-    advance_ctrl(ctrl, c, mn, vol, fs, rs, dx, sums);
+    next_ctrl(c, mn).put(ctrl);
+    if (sums) put_sums(ctrl, vol, fs, rs, dx);
   }
 }
 
@@ -478,6 +615,47 @@ __global__ __launch_bounds__(1024) void k_finalize(hp_ctrl* ctrl, void* work, in
                                                    int single_pass) {
   const Partials P(work, n);
   finalize_domain(ctrl, P.mins, P.sums, n, dx, sums != 0, single_pass != 0);
+}
+
+// Before and after the steps of a folded call: the control block into the
+// ring, and from it back to the caller's after the last step's fold.
+__global__ __launch_bounds__(64) void k_fold_begin(const hp_ctrl* __restrict__ ctrl, FoldState* f) {
+  const int lane = threadIdx.x;
+  for (int b = 0; b < 3; ++b) f->slots[b][lane] = kNoMinimum;
+  if (lane == 0) f->ring[1] = *ctrl;
+}
+// (k: the number of steps, at least 2; a 1024-thread block with sums)
+__device__ inline void fold_end(hp_ctrl* ctrl, const FoldState* f, int k, const Sums* prev, int n, double dx, bool sums) {
+  const StepCtrl c = StepCtrl::of(&f->ring[(k + 1) & 1]);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const double mn = wave_min(__builtin_bit_cast(double, (uint64_t)f->slots[(k + 2) % 3][lane]));
+  __shared__ double s_sum[3][kFoldSumBlocks];
+  const bool add = sums && !c.stopped();
+  double vol, fs, rs;
+  if (add) {
+    wave_records(prev, n, w, vol, fs, rs);
+    if (lane == 0) {
+      s_sum[0][w] = vol;
+      s_sum[1][w] = fs;
+      s_sum[2][w] = rs;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (sums && f->summed[k & 1] != 0.0) {
+      add_waves(f->wave_sums[k & 1], vol, fs, rs);
+      put_sums(ctrl, vol, fs, rs, dx);
+    }
+    next_ctrl_single_pass(c, mn).put(ctrl);
+    if (add) {
+      add_waves(s_sum, vol, fs, rs);
+      put_sums(ctrl, vol, fs, rs, dx);
+    }
+  }
+}
+__global__ __launch_bounds__(1024) void k_fold_end(hp_ctrl* ctrl, const FoldState* f, int k, const Sums* prev, int n,
+                                                   double dx, int sums) {
+  fold_end(ctrl, f, k, prev, n, dx, sums != 0);
 }
 
 // k_finalize followed by a calibration step's record (thread 0 wrote the
@@ -617,25 +795,34 @@ static int check_desc(const hp_grid_desc* g) {
   return HP_OK;
 }
 
+// A folded step: its place in the call and the record arrays of this step and
+// the one before (null without mass sums).
+struct FoldStep {
+  FoldState* st;
+  int k;
+  Sums *records, *prev;
+};
+
 template <class T, int ORDER, bool FUSED>
-static int launch_walk_t(const hp_grid_desc* g, hipStream_t st, int flags) {
+static int launch_walk_t(const hp_grid_desc* g, hipStream_t st, int flags, const FoldStep& f) {
   const int rows = flux_rows(g), ns = (g->nx + kWalkOwn - 1) / kWalkOwn;
-  hipLaunchKernelGGL((k_walk<T, ORDER, FUSED>), dim3((unsigned)units(g, kWalkOwn, rows)), dim3(kWalkLanes), 0, st, *g,
-                     Divisor::of(ns), rows, flags);
+  const int n = (int)units(g, kWalkOwn, rows), extra = f.st && f.records ? kFoldSumBlocks : 0;
+  hipLaunchKernelGGL((k_walk<T, ORDER, FUSED>), dim3((unsigned)(n + extra)), dim3(kWalkLanes), 0, st, *g,
+                     Divisor::of(ns), rows, flags, n, WalkFold{f.st, f.k, f.records}, f.prev);
   return check_launch(FUSED ? "k_walk (single-pass step)" : "k_walk (flux pass)");
 }
 
 template <bool FUSED>
-static int launch_walk(const hp_grid_desc* g, hipStream_t st, int flags) {
+static int launch_walk(const hp_grid_desc* g, hipStream_t st, int flags, const FoldStep& f = FoldStep{}) {
   if (g->dtype == HP_F32)
-    return g->order == 2 ? launch_walk_t<float, 2, FUSED>(g, st, flags) : launch_walk_t<float, 1, FUSED>(g, st, flags);
-  return g->order == 2 ? launch_walk_t<double, 2, FUSED>(g, st, flags) : launch_walk_t<double, 1, FUSED>(g, st, flags);
+    return (g->order == 2 ? launch_walk_t<float, 2, FUSED> : launch_walk_t<float, 1, FUSED>)(g, st, flags, f);
+  return (g->order == 2 ? launch_walk_t<double, 2, FUSED> : launch_walk_t<double, 1, FUSED>)(g, st, flags, f);
 }
 
 static int launch_flux(const hp_grid_desc* g, hipStream_t st) { return launch_walk<false>(g, st, 0); }
 
-static int launch_step_fused(const hp_grid_desc* g, hipStream_t st, int flags = 0) {
-  return launch_walk<true>(g, st, flags);
+static int launch_step_fused(const hp_grid_desc* g, hipStream_t st, int flags = 0, const FoldStep& f = FoldStep{}) {
+  return launch_walk<true>(g, st, flags, f);
 }
 
 static int launch_finalize_fused(const hp_grid_desc* g, hipStream_t st, const StepRecord* rec = nullptr) {
@@ -845,6 +1032,13 @@ static int64_t workspace_need(const hp_grid_desc* g) {
   return partials_bytes(std::max({flux_tiles(g), nominal_tiles(g), update_blocks(g)}));
 }
 
+// Workspace of a call with folded time control: the fold's state, and two
+// arrays of sum records when they are kept.  Asked for beside workspace_need;
+// where a caller brings less, the time control keeps its own launches.
+static int64_t fold_need(const hp_grid_desc* g) {
+  return align256(sizeof(FoldState)) + (g->mass_sums ? 2 * flux_tiles(g) * (int64_t)sizeof(Sums) : 0);
+}
+
 // The checks every single-pass entry point makes.
 static int check_fused(const hp_grid_desc* g) {
   int rc = check_desc(g);
@@ -855,12 +1049,49 @@ static int check_fused(const hp_grid_desc* g) {
   return HP_OK;
 }
 
-// One single-pass step and its time control.  first: the first step of a
-// call (a stopped domain copies its state through even when marked in step).
-static int single_pass_step(const hp_grid_desc* d, hipStream_t st, bool first) {
-  int rc = launch_step_fused(d, st, first ? 4 : 0);
-  if (rc) return rc;
-  return launch_finalize_fused(d, st);
+// Calls of at least this many steps fold the time control into the step
+// kernel: begin and end are launches too, so below it nothing is saved.
+constexpr int kFoldSteps = 3;
+
+// nsteps single-pass steps, each with its time control; the buffers swap every
+// step.  before / after are called around every step's kernel.
+template <class Before, class After>
+static int single_pass_steps(const hp_grid_desc* g, int32_t nsteps, hipStream_t st, Before before, After after) {
+  hp_grid_desc d = *g;
+  // (a negative CFL number would give negative minima, whose bits do not order)
+  const bool fold = nsteps >= kFoldSteps && g->cfl >= 0.0 && g->work_bytes >= fold_need(g);
+  FoldState* fs = fold ? (FoldState*)g->work : nullptr;
+  const int64_t n = flux_tiles(g);
+  Sums* rec = fold && g->mass_sums ? (Sums*)((char*)g->work + align256(sizeof(FoldState))) : nullptr;
+  auto records = [&](int k) { return rec ? rec + (k & 1) * n : nullptr; };
+  int rc = HP_OK;
+  if (fold) {
+    hipLaunchKernelGGL(k_fold_begin, dim3(1), dim3(64), 0, st, (const hp_ctrl*)g->ctrl, fs);
+    rc = check_launch("k_fold_begin");
+    if (rc) return rc;
+  }
+  for (int32_t k = 0; k < nsteps; ++k) {
+    before(k);
+    // the first step of a call copies a stopped domain's state through even
+    // if an earlier call left both sets in step: the host may have written
+    // the state in between
+    rc = launch_step_fused(&d, st, k == 0 ? 4 : 0, FoldStep{fs, k, records(k), records(k + 1)});
+    if (rc) return rc;
+    after(k);
+    if (!fold) {
+      rc = launch_finalize_fused(&d, st);
+      if (rc) return rc;
+    }
+    std::swap(d.h, d.h_out);
+    std::swap(d.qx, d.qx_out);
+    std::swap(d.qy, d.qy_out);
+  }
+  if (fold) {
+    hipLaunchKernelGGL(k_fold_end, dim3(1), dim3(rec ? 1024 : 64), 0, st, g->ctrl, (const FoldState*)fs, (int)nsteps,
+                       (const Sums*)records(nsteps - 1), (int)n, g->dx, rec ? 1 : 0);
+    rc = check_launch("k_fold_end");
+  }
+  return rc;
 }
 
 // After an odd number of single-pass steps the state sits in the second set
@@ -882,7 +1113,7 @@ extern "C" {
 
 int64_t hp_grid_workspace_bytes(const hp_grid_desc* g) {
   if (!g || g->pitch <= 0 || g->ny <= 0 || g->nx <= 0) return 0;
-  return workspace_need(g);
+  return std::max(workspace_need(g), fold_need(g));
 }
 
 int hp_grid_step_fused(const hp_grid_desc* g, int32_t nsteps, void* stream) {
@@ -890,17 +1121,8 @@ int hp_grid_step_fused(const hp_grid_desc* g, int32_t nsteps, void* stream) {
   if (rc) return rc;
   if (nsteps < 0) return fail(HP_EINVAL, "nsteps must be >= 0");
   hipStream_t st = (hipStream_t)stream;
-  hp_grid_desc d = *g;
-  for (int32_t k = 0; k < nsteps; ++k) {
-    // the first step of a call copies a stopped domain's state through even
-    // if an earlier call left both sets in step: the host may have written
-    // the state in between
-    rc = single_pass_step(&d, st, k == 0);
-    if (rc) return rc;
-    std::swap(d.h, d.h_out);
-    std::swap(d.qx, d.qx_out);
-    std::swap(d.qy, d.qy_out);
-  }
+  rc = single_pass_steps(g, nsteps, st, [](int) {}, [](int) {});
+  if (rc) return rc;
   if (nsteps & 1) return copy_state_back(g, st);
   return HP_OK;
 }
@@ -947,21 +1169,15 @@ int hp_grid_step_fused_timed(const hp_grid_desc* g, int32_t nsteps, int32_t samp
       return fail(HP_ELAUNCH, "hipEventCreate failed");
     }
   }
-  hp_grid_desc d = *g;
   (void)hipEventRecord(ev[0], st);
-  for (int32_t k = 0; k < nsteps && rc == HP_OK; ++k) {
-    const bool sample = k % sample_every == 0;
-    const size_t j = 2 + 2 * (size_t)(k / sample_every);
-    if (sample) (void)hipEventRecord(ev[j], st);
-    rc = launch_step_fused(&d, st, k == 0 ? 4 : 0);
-    if (rc == HP_OK) {
-      if (sample) (void)hipEventRecord(ev[j + 1], st);
-      rc = launch_finalize_fused(&d, st);
-    }
-    std::swap(d.h, d.h_out);
-    std::swap(d.qx, d.qx_out);
-    std::swap(d.qy, d.qy_out);
-  }
+  rc = single_pass_steps(
+      g, nsteps, st,
+      [&](int k) {
+        if (k % sample_every == 0) (void)hipEventRecord(ev[2 + 2 * (size_t)(k / sample_every)], st);
+      },
+      [&](int k) {
+        if (k % sample_every == 0) (void)hipEventRecord(ev[3 + 2 * (size_t)(k / sample_every)], st);
+      });
   if (rc == HP_OK) {
     (void)hipEventRecord(ev[1], st);
     if (nsteps & 1) rc = copy_state_back(g, st);  // after the timed steps

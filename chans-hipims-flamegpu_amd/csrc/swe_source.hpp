@@ -60,9 +60,19 @@ template <class F> __device__ inline int wave_first(int from, int to, F hit) {
   return to;
 }
 
+// The times of a rain table of at most 64 rows, a row per lane (all the lanes
+// of a wave call it): one memory round trip, which a kernel can start before
+// it knows its own time.
+template <class DP> __device__ inline double wave_rain_times(DP a) {
+  if (a->rain_mode != HP_RAIN_STATION || a->rain_table == nullptr || a->rain_rows <= 1 || a->rain_rows > 64) return 0.0;
+  const int lane = (int)(threadIdx.x & 63);
+  return a->rain_table[(int64_t)(lane < a->rain_rows ? lane : 0) * a->rain_cols];
+}
+
 // The bracketing rows at t_now, through any pointer type of the descriptor
 // (generic, or the kernel-argument address space); called by whole waves.
-template <class DP> __device__ inline RainRows wave_rain_rows(DP a, double t_now) {
+// times: wave_rain_times.
+template <class DP> __device__ inline RainRows wave_rain_rows(DP a, double t_now, double times) {
   RainRows r{nullptr, nullptr, 0.0, 0, true};
   if (a->rain_mode != HP_RAIN_STATION || a->rain_table == nullptr || a->rain_rows <= 0) return r;
   const int rows = a->rain_rows, cols = a->rain_cols;
@@ -72,16 +82,14 @@ template <class DP> __device__ inline RainRows wave_rain_rows(DP a, double t_now
   int i;  // the last row whose successor lies after t_now (the table's last two rows at most)
   double t0, t1;
   if (rows <= 64) {
-    // a row per lane: one memory round trip
     const int lane = (int)(threadIdx.x & 63);
-    const double t = tab[(int64_t)(lane < rows ? lane : 0) * cols];
-    const uint64_t later = __builtin_amdgcn_ballot_w64(lane < rows && t_now < t);
+    const uint64_t later = __builtin_amdgcn_ballot_w64(lane < rows && t_now < times);
     r.zero = !(later >> (rows - 1) & 1);
     if (r.zero) return r;
     const uint64_t inner = later & ((uint64_t(1) << (rows - 1)) - 2);  // rows 1 .. rows - 2
     i = inner ? (int)__builtin_ctzll(inner) - 1 : rows - 2;
-    t0 = __shfl(t, i, 64);
-    t1 = __shfl(t, i + 1, 64);
+    t0 = __shfl(times, i, 64);
+    t1 = __shfl(times, i + 1, 64);
   } else {
     r.zero = !(t_now < tab[(int64_t)(rows - 1) * cols]);
     if (r.zero) return r;
@@ -93,6 +101,10 @@ template <class DP> __device__ inline RainRows wave_rain_rows(DP a, double t_now
   r.hi = r.lo + cols;
   r.per = (t_now - t0) / (t1 - t0);
   return r;
+}
+
+template <class DP> __device__ inline RainRows wave_rain_rows(DP a, double t_now) {
+  return wave_rain_rows(a, t_now, wave_rain_times(a));
 }
 
 // Rain rate of a cell whose station index is k.

@@ -480,6 +480,39 @@ __device__ inline WalkFlux<T> walk_edges(const WalkEnv<T>& env, DP a, const WRow
   return o;
 }
 
+// The time control a unit steps by (the same for the whole wave).
+struct WalkClock {
+  double t, dt;
+  bool stopped, synced;
+};
+// From the domain's control block, which no launch of this kernel writes:
+// constant memory, scalar loads.
+__device__ inline WalkClock walk_clock(KCtrl c) {
+  return WalkClock{c->t, c->dt, c->t_stop > 0.0 && c->t >= c->t_stop, c->stopped_synced != 0.0};
+}
+// Folded: the minima of the step before, advanced from its control block; the
+// lead unit hands the result on and clears the slots of the next step.
+template <class T> __device__ inline WalkClock walk_fold(const WalkFold& f, bool lead) {
+  const int lane = (int)threadIdx.x;
+  const KCtrl b = (KCtrl)&f.st->ring[(f.k + 1) & 1];
+  StepCtrl e = StepCtrl::of(b);
+  if (f.k > 0) {
+    const uint64_t m = f.st->slots[(f.k + 2) % 3][lane];
+    // (the minima of a float step are floats)
+    e = next_ctrl_single_pass(e, (double)wave_min(T(__builtin_bit_cast(double, m))));
+  }
+  if (lead) {
+    f.st->slots[(f.k + 1) % 3][lane] = kNoMinimum;
+    if (lane == 0) {
+      hp_ctrl* to = &f.st->ring[f.k & 1];
+      e.put(to);
+      to->export_T = e.export_T;
+      to->t_stop = e.t_stop;
+    }
+  }
+  return WalkClock{uniform(e.t), uniform(e.dt), uniform((int)e.stopped()) != 0, uniform((int)(e.synced != 0.0)) != 0};
+}
+
 // What a unit does besides the step itself (the same for the whole launch).
 struct WalkMode {
   bool save_flux;     // also write the flux increments to dh, dqx, dqy
@@ -555,9 +588,12 @@ __device__ __forceinline__ void walk_row(const WalkEnv<T>& env, DP a, const Walk
 // makes a stopped domain copy its state through even when marked in step.
 // (inlined into each kernel: the launder needs the descriptor pointer known
 // uniform, which a call shared by two kernels would not let the compiler see)
+// fold: where the step's time control comes from and its minimum goes, when
+// no launch of its own runs it (lead: the unit that carries the domain's
+// control block on).
 template <class T, int ORDER, bool FUSED, class DP>
 __device__ __forceinline__ void walk_unit(DP a, int bx, int by, int R, const Partials& part, int64_t pidx, bool save_flux,
-                                 bool time_control, bool force_copy) {
+                                          bool time_control, bool force_copy, const WalkFold& fold, bool lead) {
   __shared__ T s_rate[FUSED ? kMaxStations : 1], s_man[FUSED ? 256 : 1];
   __shared__ double s_sums[FUSED ? 3 * kWalkLanes : 1];
   const int lane = (int)threadIdx.x;
@@ -569,15 +605,22 @@ __device__ __forceinline__ void walk_unit(DP a, int bx, int by, int R, const Par
   // east of them (the last owned cell's east edge)
   const bool need_x = lane >= 2 && lane <= 2 + kWalkOwn && gx <= a->nx;
   const int y0 = by * R;
-  // the control block, which no launch of this kernel writes, as constant
-  // memory: scalar loads
-  const KCtrl ctrl = (KCtrl)a->ctrl;
-  if (ctrl->t_stop > 0.0 && ctrl->t >= ctrl->t_stop) {
+  // The unit's first rows y0 - 2 .. y0 + 1 are asked for before anything
+  // else: the time control and the tables below take memory round trips of
+  // their own meanwhile.
+  const WalkPlanes p(a);
+  WRow<T> A = walk_load<T>(p, cx, y0 - 2, col_in), B = walk_load<T>(p, cx, y0 - 1, col_in);
+  WRow<T> C = walk_load<T>(p, cx, y0, col_in), D = walk_load<T>(p, cx, y0 + 1, col_in);
+  // (the rain table's times too)
+  const double rain_times = FUSED ? wave_rain_times(a) : 0.0;
+  const bool folded = FUSED && fold.st != nullptr;
+  const WalkClock clock = folded ? walk_fold<T>(fold, lead) : walk_clock((KCtrl)a->ctrl);
+  if (clock.stopped) {
     if (FUSED) {
-      if (lane == 0) part.put(pidx, INFINITY, 0.0, 0.0, 0.0, a->mass_sums != 0);
+      if (lane == 0 && !folded) part.put(pidx, INFINITY, 0.0, 0.0, 0.0, a->mass_sums != 0);
       // (once the time control has marked the copy done, both sets of planes
       // hold the state)
-      if (ctrl->stopped_synced != 0.0 && !force_copy) return;
+      if (clock.synced && !force_copy) return;
       if (own) {
         for (int r = 0; r < R; ++r) {
           const int gy = y0 + r;
@@ -591,14 +634,9 @@ __device__ __forceinline__ void walk_unit(DP a, int bx, int by, int R, const Par
     }
     return;
   }
-  // The unit's first rows y0 - 2 .. y0 + 1 are asked for before anything
-  // else: the tables below take memory round trips of their own meanwhile.
-  const WalkPlanes p(a);
-  WRow<T> A = walk_load<T>(p, cx, y0 - 2, col_in), B = walk_load<T>(p, cx, y0 - 1, col_in);
-  WRow<T> C = walk_load<T>(p, cx, y0, col_in), D = walk_load<T>(p, cx, y0 + 1, col_in);
-  const double t_now = ctrl->t;
+  const double t_now = clock.t;
   WalkEnv<T> env;
-  env.dt = uniform(T(ctrl->dt));
+  env.dt = uniform(T(clock.dt));
   env.dx = uniform(T(a->dx));
   env.dt_dx = uniform(env.dt / env.dx);
   env.cfl_dx = uniform(T(a->cfl) * T(a->dx));
@@ -625,7 +663,7 @@ __device__ __forceinline__ void walk_unit(DP a, int bx, int by, int R, const Par
       // naming another station, or any cell once the table has ended, gets
       // no rain, as station_rate gives); without a station plane every cell
       // takes station 0
-      const RainRows rr = wave_rain_rows(a, t_now);
+      const RainRows rr = wave_rain_rows(a, t_now, rain_times);
       if (env.rain == 0) {
         env.rate = uniform(station_rate<T>(rr, 0, a->rain_scale));
       } else {
@@ -680,7 +718,17 @@ __device__ __forceinline__ void walk_unit(DP a, int bx, int by, int R, const Par
       fs = wave_sum(fs);
       rs = wave_sum(rs);
     }
-    if (lane == 0) part.put(pidx, (double)mn, vol, fs, rs, sums);
+    if (lane == 0) {
+      if (folded) {
+        // (another unit's minimum may land first: order does not matter)
+        __hip_atomic_fetch_min(&fold.st->slots[fold.k % 3][pidx % kFoldSlots],
+                               (unsigned long long)__builtin_bit_cast(uint64_t, (double)mn), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        if (sums) fold.records[pidx] = Sums{vol, fs, rs, 0.0};
+      } else {
+        part.put(pidx, (double)mn, vol, fs, rs, sums);
+      }
+    }
   }
 }
 
@@ -693,14 +741,22 @@ template <class T> constexpr int walk_waves() { return sizeof(T) == 4 ? 5 : 3; }
 // flags: 1 also save the step's flux in dh, dqx, dqy; 2 no time-control
 // outputs (a frozen schedule); 4 a stopped domain copies its state through
 // even when marked in step.
+// With fold.st set, the grid may begin with blocks that fold the FP64 sums of
+// the step before (n_units: the blocks that walk).
 template <class T, int ORDER, bool FUSED>
 __global__ __launch_bounds__(kWalkLanes, walk_waves<T>()) void k_walk(hp_grid_desc a, Divisor strips, int rows,
-                                                                       int flags) {
+                                                                       int flags, int n_units, WalkFold fold,
+                                                                       const Sums* prev) {
   const KDesc pa = kernarg_desc();
-  const int unit = xcd_band(blockIdx.x, gridDim.x);
+  const int extra = (int)gridDim.x - n_units;
+  if (FUSED && (int)blockIdx.x < extra) {
+    fold_sums_block(pa->ctrl, fold.st, fold.k, (int)blockIdx.x, prev, n_units, pa->dx);
+    return;
+  }
+  const int unit = xcd_band((int)blockIdx.x - extra, n_units);
   const int by = strips.div(unit);
-  walk_unit<T, ORDER, FUSED>(pa, unit - by * strips.n, by, rows, Partials(a.work, gridDim.x), unit,
-                             (flags & 1) != 0, (flags & 2) == 0, (flags & 4) != 0);
+  walk_unit<T, ORDER, FUSED>(pa, unit - by * strips.n, by, rows, Partials(a.work, n_units), unit, (flags & 1) != 0,
+                             (flags & 2) == 0, (flags & 4) != 0, fold, unit == 0);
 }
 
 // Every unit of every domain of an ensemble; map[i] = (domain, unit), domain
@@ -717,7 +773,8 @@ __global__ __launch_bounds__(kWalkLanes, walk_waves<T>()) void k_walk_multi(cons
   const KDesc a = (KDesc)(doms + dom);
   const int nstrips = (a->nx + kWalkOwn - 1) / kWalkOwn;
   const int by = uniform(unit / nstrips);
-  walk_unit<T, ORDER, FUSED>(a, unit - by * nstrips, by, rows, Partials(parts, n_total), slot, false, true, false);
+  walk_unit<T, ORDER, FUSED>(a, unit - by * nstrips, by, rows, Partials(parts, n_total), slot, false, true, false,
+                             WalkFold{nullptr, 0, nullptr}, false);
 }
 
 }  // namespace hp
