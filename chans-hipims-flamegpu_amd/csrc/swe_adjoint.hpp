@@ -22,19 +22,18 @@ template <class T> __host__ __device__ inline FrameAdj<T> zero_adj() {
   return a;
 }
 
-// Which argument minmod(x, y) returned: 0 none (opposite signs), 1 x, 2 y.
-template <class T> __host__ __device__ inline int minmod_pick(T x, T y) {
-  if (x * y <= T(0)) return 0;
-  return fabs(x) < fabs(y) ? 1 : 2;
-}
+// v where on, else 0 (a select; v may be anything where it is dropped).
+template <class T> __host__ __device__ inline T only(bool on, T v) { return on ? v : T(0); }
 
-// Cotangent of e = c + 0.5 * minmod(c - l, r - c) pushed to (c, l, r).
+// Cotangent of e = c + 0.5 * minmod(c - l, r - c) pushed to (c, l, r): half of
+// it goes to the two cells of the difference that minmod returned, if any.
 template <class T> __host__ __device__ inline void muscl_adj(T c, T l, T r, T a_e, T& a_c, T& a_l, T& a_r) {
-  a_c += a_e;
-  const int p = minmod_pick<T>(c - l, r - c);
-  const T m = T(0.5) * a_e;
-  if (p == 1) { a_c += m; a_l -= m; }
-  else if (p == 2) { a_r += m; a_c -= m; }
+  const T x = c - l, y = r - c, m = T(0.5) * a_e;
+  const bool some = x * y > T(0), first = fabs(x) < fabs(y);
+  const T mx = only(both(some, first), m), my = only(both(some, !first), m);
+  a_c += a_e + (mx - my);
+  a_l -= mx;
+  a_r += my;
 }
 
 // VJP of solve_edge (swe_physics.hpp) with cotangents (v_fh, v_fn, v_ft,
@@ -58,10 +57,10 @@ __host__ __device__ inline bool solve_edge_vjp(const FrameCell<T>& c, const Fram
     eL = c;
     eR = r;
     if (ORDER == 1 && !r_is_ghost) {
-      T rb = Prec<T>::limit(c.z - l.z, r.z - c.z);
-      if (gt_hs(r.h)) eL.z += T(0.5) * rb;
-      rb = Prec<T>::limit(r.z - rr.z, c.z - r.z);
-      if (gt_hs(c.h)) eR.z += T(0.5) * rb;
+      const T zl = eL.z + T(0.5) * Prec<T>::limit(c.z - l.z, r.z - c.z);
+      const T zr = eR.z + T(0.5) * Prec<T>::limit(r.z - rr.z, c.z - r.z);
+      eL.z = gt_hs(r.h) ? zl : eL.z;
+      eR.z = gt_hs(c.h) ? zr : eR.z;
     }
   } else {
     eL.h = c.h + T(0.5) * Prec<T>::limit(c.h - l.h, r.h - c.h);
@@ -70,22 +69,25 @@ __host__ __device__ inline bool solve_edge_vjp(const FrameCell<T>& c, const Fram
     eR.z = r.z + T(0.5) * Prec<T>::limit(r.z - rr.z, c.z - r.z);
     zeroL = lt_hs(c.h);
     zeroR = lt_hs(r.h);
-    if (zeroL) { eL.qn = T(0); eL.qt = T(0); }
-    else {
-      eL.qn = c.qn + T(0.5) * Prec<T>::limit(c.qn - l.qn, r.qn - c.qn);
-      eL.qt = c.qt + T(0.5) * Prec<T>::limit(c.qt - l.qt, r.qt - c.qt);
-    }
-    if (zeroR) { eR.qn = T(0); eR.qt = T(0); }
-    else {
-      eR.qn = r.qn + T(0.5) * Prec<T>::limit(r.qn - rr.qn, c.qn - r.qn);
-      eR.qt = r.qt + T(0.5) * Prec<T>::limit(r.qt - rr.qt, c.qt - r.qt);
-    }
+    const T nL = c.qn + T(0.5) * Prec<T>::limit(c.qn - l.qn, r.qn - c.qn);
+    const T tL = c.qt + T(0.5) * Prec<T>::limit(c.qt - l.qt, r.qt - c.qt);
+    const T nR = r.qn + T(0.5) * Prec<T>::limit(r.qn - rr.qn, c.qn - r.qn);
+    const T tR = r.qt + T(0.5) * Prec<T>::limit(r.qt - rr.qt, c.qt - r.qt);
+    eL.qn = only(!zeroL, nL);
+    eL.qt = only(!zeroL, tL);
+    eR.qn = only(!zeroR, nR);
+    eR.qt = only(!zeroR, tR);
   }
+  // From here on straight-line code with selects, as in hllc_edge: the
+  // branches of the forward step become masks on the cotangents, and what a
+  // mask drops may hold anything.  (With the branches, a wave whose edges fell
+  // in different regions ran each in turn and copied some twenty values at
+  // every join: 62 -> 52.8 us per reverse step of 1024^2 cells, order 1, float.)
   // ---- forward: velocities and hydrostatic reconstruction ----
   const bool dryL0 = lt_hs(eL.h), dryR0 = lt_hs(eR.h);
   const T rhL = P::div(T(1), eL.h), rhR = P::div(T(1), eR.h);  // as hllc_edge forms them
-  const T uL0 = dryL0 ? T(0) : eL.qn * rhL, vL0 = dryL0 ? T(0) : eL.qt * rhL;
-  const T uR0 = dryR0 ? T(0) : eR.qn * rhR, vR0 = dryR0 ? T(0) : eR.qt * rhR;
+  const T uL0 = dryL0 ? T(0) : mul_alone(eL.qn, rhL), vL0 = dryL0 ? T(0) : mul_alone(eL.qt, rhL);
+  const T uR0 = dryR0 ? T(0) : mul_alone(eR.qn, rhR), vR0 = dryR0 ? T(0) : mul_alone(eR.qt, rhR);
   const T wL0 = eL.h + eL.z, wR0 = eR.h + eR.z;
   const bool maxC = etaC >= etaR;  // fmax(etaC, etaR) took etaC
   const bool minC = etaC <= etaR;  // fmin(etaC, etaR) took etaC
@@ -98,177 +100,153 @@ __host__ __device__ inline bool solve_edge_vjp(const FrameCell<T>& c, const Fram
   bool avg = false, liftL = false, takeL = false;
   if (ORDER == 1) {
     avg = (etaC - etaR) * (wL2 - wR2) < T(0);
-    if (avg) { wL3 = wR3 = (wL2 + wR2) / T(2); }
+    const T m = (wL2 + wR2) / T(2);
+    wL3 = avg ? m : wL2;
+    wR3 = avg ? m : wR2;
   } else {
     liftL = etaC > etaR;
     takeL = wL2 >= wR2;
     const T m = takeL ? wL2 : wR2;
-    if (liftL) wL3 = m; else wR3 = m;
+    wL3 = liftL ? m : wL2;
+    wR3 = liftL ? wR2 : m;
   }
   const T zL0 = wL3 - eL.h, zR0 = wR3 - eR.h;
   const bool zbL = zL0 >= zR0;
   const T zbm = zbL ? zL0 : zR0;
-  const bool posL = wL3 - zbm > T(0), posR = wR3 - zbm > T(0);
-  const T hL = posL ? wL3 - zbm : T(0), hR = posR ? wR3 - zbm : T(0);
+  const T dL = wL3 - zbm, dR = wR3 - zbm;
+  const bool posL = dL > T(0), posR = dR > T(0);
+  const T hL = only(posL, dL), hR = only(posR, dR);
   const T zL = wL3 - hL, zR = wR3 - hR;
-  const bool flux_on = !(lt_hs(hL) && lt_hs(hR));
+  const bool flux_on = !both(lt_hs(hL), lt_hs(hR));
 
   const T s = dt / dx;
   const T Gb = T(0.5) * g * s;
-  // cotangents of intermediates
-  T a_hL = T(0), a_hR = T(0), a_zL = T(0), a_zR = T(0);
-  T a_uL0 = T(0), a_vL0 = T(0), a_uR0 = T(0), a_vR0 = T(0);
-
   // ---- reverse: bed terms ----
-  a_hL += v_bc * Gb * (zL - c.z);
-  a_zL += v_bc * Gb * (hL + c.h);
+  T a_hL = v_bc * Gb * (zL - c.z), a_zL = v_bc * Gb * (hL + c.h);
   ac.h += v_bc * Gb * (zL - c.z);
-  a_hR += v_br * Gb * (zR - r.z);
-  a_zR += v_br * Gb * (hR + r.h);
+  T a_hR = v_br * Gb * (zR - r.z), a_zR = v_br * Gb * (hR + r.h);
   ar.h += v_br * Gb * (zR - r.z);
 
   // ---- reverse: HLLC ----
-  if (flux_on) {
-    const T qnL = uL0 * hL, qtL = vL0 * hL, qnR = uR0 * hR, qtR = vR0 * hR;
-    const T aL = Prec<T>::sqrt_(g * hL), aR = Prec<T>::sqrt_(g * hR);
-    const T base = (aL + aR) / T(2) + (uL0 - uR0) / T(4);
-    const T u_star = (uL0 + uR0) / T(2) + aL - aR;
-    const T a_star = P::star_celerity(base, g);
-    const bool sLdry = le_hs(hL), sRdry = le_hs(hR);
-    const T x1 = uL0 - aL, x2 = u_star - a_star;
-    const T y1 = uR0 + aR, y2 = u_star + a_star;
-    const bool sLx1 = x1 <= x2, sRy1 = y1 >= y2;
-    const T sL = sLdry ? uR0 - T(2) * aR : (sLx1 ? x1 : x2);
-    const T sR = sRdry ? uL0 + T(2) * aL : (sRy1 ? y1 : y2);
-    const T sM = P::div(sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), hR * (uR0 - sR) - hL * (uL0 - sL));
-    const T b_fh = v_fh * s, b_fn = v_fn * s, b_ft = v_ft * s;
-    T a_qnL = T(0), a_qtL = T(0), a_qnR = T(0), a_qtR = T(0), a_sL = T(0), a_sR = T(0);
-    if (T(0) <= sL) {
-      a_qnL += b_fh + b_fn * uL0;
-      a_uL0 += b_fn * qnL + b_ft * qtL;
-      a_hL += b_fn * g * hL;
-      a_qtL += b_ft * uL0;
-    } else if ((sL < T(0) && T(0) <= sM) || (sM < T(0) && T(0) <= sR)) {
-      const bool useL = (sL < T(0) && T(0) <= sM);
-      const T vstar = useL ? vL0 : vR0;
-      const T D = sR - sL;
-      const T qnfL = uL0 * qnL + T(0.5) * g * hL * hL;
-      const T qnfR = uR0 * qnR + T(0.5) * g * hR * hR;
-      const T Nh = sR * qnL - sL * qnR + sL * sR * (hR - hL);
-      const T Nn = sR * qnfL - sL * qnfR + sL * sR * (qnR - qnL);
-      const T rD = P::div(T(1), D);
-      const T fh = Nh * rD, fn = Nn * rD;
-      const T b_fh_tot = b_fh + b_ft * vstar;
-      if (useL) a_vL0 += b_ft * fh; else a_vR0 += b_ft * fh;
-      T a_D = P::div(-(b_fh_tot * fh + b_fn * fn), D);
-      const T a_Nh = P::div(b_fh_tot, D), a_Nn = P::div(b_fn, D);
-      a_sR += a_Nh * (qnL + sL * (hR - hL));
-      a_sL += a_Nh * (-qnR + sR * (hR - hL));
-      a_qnL += a_Nh * sR;
-      a_qnR -= a_Nh * sL;
-      a_hR += a_Nh * sL * sR;
-      a_hL -= a_Nh * sL * sR;
-      T a_qnfL = a_Nn * sR, a_qnfR = -a_Nn * sL;
-      a_sR += a_Nn * (qnfL + sL * (qnR - qnL));
-      a_sL += a_Nn * (-qnfR + sR * (qnR - qnL));
-      a_qnR += a_Nn * sL * sR;
-      a_qnL -= a_Nn * sL * sR;
-      a_qnL += a_qnfL * uL0; a_uL0 += a_qnfL * qnL; a_hL += a_qnfL * g * hL;
-      a_qnR += a_qnfR * uR0; a_uR0 += a_qnfR * qnR; a_hR += a_qnfR * g * hR;
-      a_sR += a_D;
-      a_sL -= a_D;
-    } else {
-      a_qnR += b_fh + b_fn * uR0;
-      a_uR0 += b_fn * qnR + b_ft * qtR;
-      a_hR += b_fn * g * hR;
-      a_qtR += b_ft * uR0;
-    }
-    // wave speeds
-    T a_aL = T(0), a_aR = T(0), a_ustar = T(0), a_astar = T(0);
-    if (sLdry) { a_uR0 += a_sL; a_aR -= T(2) * a_sL; }
-    else if (sLx1) { a_uL0 += a_sL; a_aL -= a_sL; }
-    else { a_ustar += a_sL; a_astar -= a_sL; }
-    if (sRdry) { a_uL0 += a_sR; a_aL += T(2) * a_sR; }
-    else if (sRy1) { a_uR0 += a_sR; a_aR += a_sR; }
-    else { a_ustar += a_sR; a_astar += a_sR; }
-    const T a_base = P::star_celerity_adj(base, g, a_star, a_astar);
-    a_uL0 += a_ustar / T(2); a_uR0 += a_ustar / T(2); a_aL += a_ustar; a_aR -= a_ustar;
-    a_aL += a_base / T(2); a_aR += a_base / T(2); a_uL0 += a_base / T(4); a_uR0 -= a_base / T(4);
-    if (aL > T(0)) a_hL += P::div(a_aL * g, T(2) * aL);
-    if (aR > T(0)) a_hR += P::div(a_aR * g, T(2) * aR);
-    a_uL0 += a_qnL * hL; a_hL += a_qnL * uL0;
-    a_vL0 += a_qtL * hL; a_hL += a_qtL * vL0;
-    a_uR0 += a_qnR * hR; a_hR += a_qnR * uR0;
-    a_vR0 += a_qtR * hR; a_hR += a_qtR * vR0;
-  }
+  const T qnL = uL0 * hL, qtL = vL0 * hL, qnR = uR0 * hR, qtR = vR0 * hR;
+  const T aL = P::sqrt_(g * hL), aR = P::sqrt_(g * hR);
+  const T base = (aL + aR) / T(2) + (uL0 - uR0) / T(4);
+  const T u_star = (uL0 + uR0) / T(2) + aL - aR;
+  const T a_star = P::star_celerity(base, g);
+  const bool sLdry = le_hs(hL), sRdry = le_hs(hR);
+  const T x1 = uL0 - aL, x2 = u_star - a_star;
+  const T y1 = uR0 + aR, y2 = u_star + a_star;
+  const bool sLx1 = x1 <= x2, sRy1 = y1 >= y2;
+  const T sLd = uR0 - T(2) * aR, sLw = sLx1 ? x1 : x2;
+  const T sRd = uL0 + T(2) * aL, sRw = sRy1 ? y1 : y2;
+  const T sL = sLdry ? sLd : sLw, sR = sRdry ? sRd : sRw;
+  // the sign of the contact speed, as hllc_edge takes it
+  const T num = sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), den = hR * (uR0 - sR) - hL * (uL0 - sL);
+  const T sM = num * den;
+  const bool left = T(0) <= sL, useL = both(sL < T(0), T(0) <= sM);
+  const bool star = both(!left, either(useL, both(sM < T(0), T(0) <= sR)));
+  const bool inL = both(flux_on, left), inS = both(flux_on, star), inR = both(flux_on, !either(left, star));
+  const T b_fh = v_fh * s, b_fn = v_fn * s, b_ft = v_ft * s;
+  // the outer regions: the flux of one side
+  const T lh = only(inL, b_fh), ln = only(inL, b_fn), lt = only(inL, b_ft);
+  const T rh = only(inR, b_fh), rn = only(inR, b_fn), rt = only(inR, b_ft);
+  T a_qnL = lh + ln * uL0, a_qtL = lt * uL0, a_uL0 = ln * qnL + lt * qtL;
+  T a_qnR = rh + rn * uR0, a_qtR = rt * uR0, a_uR0 = rn * qnR + rt * qtR;
+  a_hL += ln * g * hL;
+  a_hR += rn * g * hR;
+  // the star region
+  const T sh = only(inS, b_fh), sn = only(inS, b_fn), st = only(inS, b_ft);
+  const T D = inS ? sR - sL : T(1), rD = P::div(T(1), D);
+  const T dh = hR - hL, dq = qnR - qnL, sLR = sL * sR;
+  const T qnfL = uL0 * qnL + T(0.5) * g * hL * hL;
+  const T qnfR = uR0 * qnR + T(0.5) * g * hR * hR;
+  const T fh = (sR * qnL - sL * qnR + sLR * dh) * rD, fn = (sR * qnfL - sL * qnfR + sLR * dq) * rD;
+  const T vstar = useL ? vL0 : vR0;
+  const T tot = sh + st * vstar;
+  const T a_D = -(tot * fh + sn * fn) * rD, a_Nh = tot * rD, a_Nn = sn * rD;
+  T a_vL0 = only(useL, st * fh), a_vR0 = only(!useL, st * fh);
+  const T a_sL = a_Nh * (sR * dh - qnR) + a_Nn * (sR * dq - qnfR) - a_D;
+  const T a_sR = a_Nh * (qnL + sL * dh) + a_Nn * (qnfL + sL * dq) + a_D;
+  const T a_qnfL = a_Nn * sR, a_qnfR = -a_Nn * sL;
+  a_qnL += a_Nh * sR - a_Nn * sLR + a_qnfL * uL0;
+  a_qnR += a_Nn * sLR - a_Nh * sL + a_qnfR * uR0;
+  a_hL += a_qnfL * g * hL - a_Nh * sLR;
+  a_hR += a_qnfR * g * hR + a_Nh * sLR;
+  a_uL0 += a_qnfL * qnL;
+  a_uR0 += a_qnfR * qnR;
+  // wave speeds
+  const T sl_d = only(sLdry, a_sL), sl_x = only(both(!sLdry, sLx1), a_sL), sl_s = only(!either(sLdry, sLx1), a_sL);
+  const T sr_d = only(sRdry, a_sR), sr_y = only(both(!sRdry, sRy1), a_sR), sr_s = only(!either(sRdry, sRy1), a_sR);
+  const T a_ustar = sl_s + sr_s, a_astar = sr_s - sl_s;
+  const T a_base = P::star_celerity_adj(base, g, a_star, a_astar);
+  const T a_aL = T(2) * sr_d - sl_x + a_ustar + a_base / T(2);
+  const T a_aR = sr_y - T(2) * sl_d - a_ustar + a_base / T(2);
+  a_uL0 += sl_x + sr_d + a_ustar / T(2) + a_base / T(4);
+  a_uR0 += sl_d + sr_y + a_ustar / T(2) - a_base / T(4);
+  const T c_aL = P::div(a_aL * g, T(2) * aL), c_aR = P::div(a_aR * g, T(2) * aR);
+  a_hL += only(aL > T(0), c_aL);
+  a_hR += only(aR > T(0), c_aR);
+  a_uL0 += a_qnL * hL;
+  a_vL0 += a_qtL * hL;
+  a_hL += a_qnL * uL0 + a_qtL * vL0;
+  a_uR0 += a_qnR * hR;
+  a_vR0 += a_qtR * hR;
+  a_hR += a_qnR * uR0 + a_qtR * vR0;
 
   // ---- reverse: hydrostatic reconstruction ----
-  T a_wL3 = a_zL, a_wR3 = a_zR;
   a_hL -= a_zL;
   a_hR -= a_zR;
-  T a_zbm = T(0);
-  if (posL) { a_wL3 += a_hL; a_zbm -= a_hL; }
-  if (posR) { a_wR3 += a_hR; a_zbm -= a_hR; }
-  T a_zL0 = zbL ? a_zbm : T(0), a_zR0 = zbL ? T(0) : a_zbm;
-  a_wL3 += a_zL0;
-  a_wR3 += a_zR0;
+  const T pL = only(posL, a_hL), pR = only(posR, a_hR);
+  const T a_zbm = -(pL + pR);
+  const T a_zL0 = only(zbL, a_zbm), a_zR0 = only(!zbL, a_zbm);
+  const T a_wL3 = a_zL + pL + a_zL0, a_wR3 = a_zR + pR + a_zR0;
   T a_eLh = -a_zL0, a_eRh = -a_zR0;
-  T a_wL2 = T(0), a_wR2 = T(0);
+  T a_wL2, a_wR2;
   if (ORDER == 1) {
-    if (avg) {
-      const T m = (a_wL3 + a_wR3) / T(2);
-      a_wL2 += m; a_wR2 += m;
-    } else {
-      a_wL2 += a_wL3; a_wR2 += a_wR3;
-    }
+    const T m = (a_wL3 + a_wR3) / T(2);
+    a_wL2 = avg ? m : a_wL3;
+    a_wR2 = avg ? m : a_wR3;
   } else {
+    // the lifted side took the higher of the two levels
     const T a_m = liftL ? a_wL3 : a_wR3;
-    if (liftL) a_wR2 += a_wR3; else a_wL2 += a_wL3;
-    if (takeL) a_wL2 += a_m; else a_wR2 += a_m;
+    a_wL2 = only(!liftL, a_wL3) + only(takeL, a_m);
+    a_wR2 = only(liftL, a_wR3) + only(!takeL, a_m);
   }
-  T a_emax = T(0), a_emin = T(0);
-  T a_wL1 = L2a ? a_wL2 : T(0), a_wR1 = R2a ? a_wR2 : T(0);
-  if (!L2a) a_emin += a_wL2;
-  if (!R2a) a_emin += a_wR2;
-  T a_wL0 = L1a ? a_wL1 : T(0), a_wR0 = R1a ? a_wR1 : T(0);
-  if (!L1a) a_emax += a_wL1;
-  if (!R1a) a_emax += a_wR1;
-  if (maxC) a_etaC += a_emax; else a_etaR += a_emax;
-  if (minC) a_etaC += a_emin; else a_etaR += a_emin;
+  const T a_emin = only(!L2a, a_wL2) + only(!R2a, a_wR2);
+  const T a_wL1 = only(L2a, a_wL2), a_wR1 = only(R2a, a_wR2);
+  const T a_emax = only(!L1a, a_wL1) + only(!R1a, a_wR1);
+  const T a_wL0 = only(L1a, a_wL1), a_wR0 = only(R1a, a_wR1);
+  a_etaC += only(maxC, a_emax) + only(minC, a_emin);
+  a_etaR += only(!maxC, a_emax) + only(!minC, a_emin);
   a_eLh += a_wL0;
   a_eRh += a_wR0;
-  T a_eLqn = T(0), a_eLqt = T(0), a_eRqn = T(0), a_eRqt = T(0);
-  if (!dryL0) {
-    a_eLqn += P::div(a_uL0, eL.h);
-    a_eLqt += P::div(a_vL0, eL.h);
-    a_eLh -= P::div(a_uL0 * uL0 + a_vL0 * vL0, eL.h);
-  }
-  if (!dryR0) {
-    a_eRqn += P::div(a_uR0, eR.h);
-    a_eRqt += P::div(a_vR0, eR.h);
-    a_eRh -= P::div(a_uR0 * uR0 + a_vR0 * vR0, eR.h);
-  }
+  T a_eLqn = a_uL0 * rhL, a_eLqt = a_vL0 * rhL, a_eRqn = a_uR0 * rhR, a_eRqt = a_vR0 * rhR;
+  const T c_hL = (a_uL0 * uL0 + a_vL0 * vL0) * rhL, c_hR = (a_uR0 * uR0 + a_vR0 * vR0) * rhR;
+  a_eLqn = only(!dryL0, a_eLqn);
+  a_eLqt = only(!dryL0, a_eLqt);
+  a_eLh -= only(!dryL0, c_hL);
+  a_eRqn = only(!dryR0, a_eRqn);
+  a_eRqt = only(!dryR0, a_eRqt);
+  a_eRh -= only(!dryR0, c_hR);
 
   // ---- reverse: edge states ----
   if (ORDER == 1 || r_is_ghost || frozen_slopes) {
     // (with frozen slopes the limited slope terms are constants)
     if (ORDER == 2 && !r_is_ghost) {
-      if (zeroL) a_eLqn = a_eLqt = T(0);
-      if (zeroR) a_eRqn = a_eRqt = T(0);
+      a_eLqn = only(!zeroL, a_eLqn);
+      a_eLqt = only(!zeroL, a_eLqt);
+      a_eRqn = only(!zeroR, a_eRqn);
+      a_eRqt = only(!zeroR, a_eRqt);
     }
     ac.h += a_eLh; ac.qn += a_eLqn; ac.qt += a_eLqt;
     ar.h += a_eRh; ar.qn += a_eRqn; ar.qt += a_eRqt;
   } else {
     muscl_adj<T>(c.h, l.h, r.h, a_eLh, ac.h, al.h, ar.h);
     muscl_adj<T>(r.h, rr.h, c.h, a_eRh, ar.h, arr.h, ac.h);
-    if (!zeroL) {
-      muscl_adj<T>(c.qn, l.qn, r.qn, a_eLqn, ac.qn, al.qn, ar.qn);
-      muscl_adj<T>(c.qt, l.qt, r.qt, a_eLqt, ac.qt, al.qt, ar.qt);
-    }
-    if (!zeroR) {
-      muscl_adj<T>(r.qn, rr.qn, c.qn, a_eRqn, ar.qn, arr.qn, ac.qn);
-      muscl_adj<T>(r.qt, rr.qt, c.qt, a_eRqt, ar.qt, arr.qt, ac.qt);
-    }
+    muscl_adj<T>(c.qn, l.qn, r.qn, only(!zeroL, a_eLqn), ac.qn, al.qn, ar.qn);
+    muscl_adj<T>(c.qt, l.qt, r.qt, only(!zeroL, a_eLqt), ac.qt, al.qt, ar.qt);
+    muscl_adj<T>(r.qn, rr.qn, c.qn, only(!zeroR, a_eRqn), ar.qn, arr.qn, ac.qn);
+    muscl_adj<T>(r.qt, rr.qt, c.qt, only(!zeroR, a_eRqt), ar.qt, arr.qt, ac.qt);
   }
   return true;
 }
@@ -316,57 +294,46 @@ template <class T>
 __host__ __device__ inline void friction_vjp(T h, T n, T dt, T qx, T qy, T a_ox, T a_oy, T& a_qx, T& a_qy, T& a_h,
                                              T& a_n) {
   const T g = T(kG);
-  if (!(n > T(0))) {
-    a_qx += a_ox;
-    a_qy += a_oy;
-    return;
-  }
   using P = Prec<T>;
   const T h13 = P::rcbrt_friction(h);
   const T C_f = g * n * n * h13;
   const T qn2 = qx * qx + qy * qy;
   const T q_norm = P::sqrt_(qn2);
   const T lim = T(5) * h * P::sqrt_(h * g);
-  const T x = P::div(T(4) * dt * C_f, h * h) * q_norm;
+  const T coef = P::div(T(4) * dt, h * h);
+  const T x = coef * C_f * q_norm;
   const T S = P::sqrt_(T(1) + x);
   const T k = P::div(T(2), T(1) + S);
-  T a_k = T(0);
+  // per component: q' = k q, past the Froude limit the reflected 2 q' - q
+  // (nothing once that changes sign); |q| <= 1e-10 passes unchanged
+  T a_k = T(0), aq[2];
   const T qc[2] = {qx, qy};
   const T ac_[2] = {a_ox, a_oy};
-  T aq[2] = {T(0), T(0)};
+#pragma unroll
   for (int m = 0; m < 2; ++m) {
-    const T q = qc[m];
-    if (!(fabs(q) > T(1.0e-10))) {
-      aq[m] += ac_[m];
-      continue;
-    }
-    const T tmp = k * q;
-    T a_tmp;
-    if (fabs(tmp) > lim) {
-      const T out = T(2) * tmp - q;
-      if (out * tmp <= T(0)) continue;  // clipped to 0
-      a_tmp = T(2) * ac_[m];
-      aq[m] -= ac_[m];
-    } else {
-      a_tmp = ac_[m];
-    }
+    const T q = qc[m], tmp = k * q, out = T(2) * tmp - q;
+    const bool moves = fabs(q) > T(1.0e-10), over = fabs(tmp) > lim, clipped = both(over, out * tmp <= T(0));
+    const bool live = both(moves, !clipped);
+    const T twice = T(2) * ac_[m];
+    const T a_tmp = only(live, over ? twice : ac_[m]);
+    const T direct = only(both(live, over), -ac_[m]);
     a_k += a_tmp * q;
-    aq[m] += a_tmp * k;
+    aq[m] = (moves ? direct : ac_[m]) + a_tmp * k;
   }
   const T dk_dx = P::div(-T(1), (T(1) + S) * (T(1) + S) * S);
   const T a_x = a_k * dk_dx;
-  const T coef = P::div(T(4) * dt, h * h);
   const T a_Cf = a_x * coef * q_norm;
-  T a_qnorm = a_x * coef * C_f;
-  a_h += a_x * P::div(T(-2) * x, h);
-  if (q_norm > T(0)) {
-    aq[0] += P::div(a_qnorm * qx, q_norm);
-    aq[1] += P::div(a_qnorm * qy, q_norm);
-  }
-  a_n += P::div(a_Cf * T(2) * C_f, n);
-  a_h += P::div(a_Cf * (T(-1.0 / 3.0)) * C_f, h);
-  a_qx += aq[0];
-  a_qy += aq[1];
+  const T a_qnorm = a_x * coef * C_f;
+  const T over_q = P::div(a_qnorm, q_norm);
+  const bool flows = q_norm > T(0);
+  const T ax = aq[0] + only(flows, over_q * qx), ay = aq[1] + only(flows, over_q * qy);
+  const T hx = P::div(a_x * (T(-2) * x) + a_Cf * (T(-1.0 / 3.0)) * C_f, h);
+  const T nx = P::div(a_Cf * T(2) * C_f, n);
+  const bool rough = n > T(0);  // without friction the momenta pass through
+  a_qx += rough ? ax : a_ox;
+  a_qy += rough ? ay : a_oy;
+  a_h += only(rough, hx);
+  a_n += only(rough, nx);
 }
 
 }  // namespace hp
