@@ -704,6 +704,34 @@ static int64_t units(const hp_grid_desc* g, int cols, int rows) {
   return (int64_t)((g->nx + cols - 1) / cols) * (int64_t)((g->ny + rows - 1) / rows);
 }
 
+// Expected time in us of a launch of u units of r rows.  n units on a SIMD
+// take row[n - 1] for a row of each (one or two of them run at the latency of
+// a row, five in float and three in double fill the SIMD), after start[n - 1]
+// for their prologues.  More units than fit at once go in rounds; up to four
+// of them, a last round that is nearly empty takes as long as a full one, and
+// tall units spread uneven rows (dry ones, nodata) worse, by 0.25 % a row; the
+// dispatcher begins a second round some 5 % before every slot is taken.  Over
+// many rounds only the prologues and a short tail count.  Measured, float,
+// order 2, height: us (units per SIMD): 256^2 1: 10.1 (1.3), 2: 10.6 (0.6);
+// 500^2 1: 20.1 (4.4), 2: 16.4 (2.2), 3: 15.4 (1.5), 5: 17.2 (0.9); 1024^2
+// 3: 33.6 (6.0), 4: 28.4 (4.5), 5: 27.0 (3.6), 8: 28.4 (2.3); 2048^2 8: 63.2
+// (8.8), 13: 67.4 (5.4), 15: 59.0 (4.7), 18: 61.6 (3.9), 24: 68.8 (2.9);
+// 3000^2 15: 119 (9.8), 30: 141 (4.9), 31: 122 (4.7), with a flood in
+// a dry plain, order 1, 15: 102, 28: 123, 32: 119; 8192^2 8: 814, 16: 752, 24: 744,
+// 32: 737; double, order 2: 256^2 1: 12.7 (1.3), 2: 13.8 (0.6); 700^2 2: 33.0
+// (4.1), 3: 27.3 (2.7), 5: 29.1 (1.6), 8: 41.3 (1.0); 2048^2 8: 145 (8.8),
+// 14: 158 (5.0), 24: 141 (2.9).
+template <class T> static double walk_cost(int64_t u, int r) {
+  static const double kRowF[] = {2.05, 2.4, 2.45, 2.85, 3.0}, kStartF[] = {6.3, 8.0, 10.5, 12.0, 16.0};
+  static const double kRowD[] = {3.35, 4.1, 5.25}, kStartD[] = {6.7, 8.6, 11.5};
+  const double *row = sizeof(T) == 4 ? kRowF : kRowD, *start = sizeof(T) == 4 ? kStartF : kStartD;
+  const double x = (double)u / walk_slots<T>();
+  const bool many = x > 4.0;
+  const double rounds = many ? x + 0.25 : std::ceil(x + (x > 1.0 ? 0.02 : 0.05));
+  const int i = (int)(rounds > 1.0 ? walk_waves<T>() : (u + kSimds - 1) / kSimds) - 1;
+  return start[i] + rounds * row[i] * r * (many ? 1.0 : 1.0 + 0.0025 * r) + 5.0 * (rounds - 1.0);
+}
+
 // Rows per flux work unit (60 columns wide): a height asked for by tile_rows
 // (2, 4, 6, 8, 10, 12 or 16 in float, 4 or 8 in double), else 0.
 static int asked_rows(const hp_grid_desc* g) {
@@ -719,27 +747,29 @@ static int nominal_rows(const hp_grid_desc* g) {
   return r ? r : (g->dtype == HP_F32 ? 8 : 4);
 }
 
-// The height where none is asked for, from the number of units of height 1
-// (of one domain, or of all the domains of an ensemble).  A taller unit
-// spreads its prologue (four rows loaded, an edge solved twice, the tables)
-// over more rows, but the launch ends with some units walking alone, at about
-// 2 us a row whatever else runs: doubling the height pays while enough
-// shorter units remain to hide that.  Measured per step, order 2 (height:
-// us), float 384^2 1: 13.9, 2: 15.0; 512^2 1: 17.1, 2: 16.4, 4: 19.5; 1024^2
-// 2: 31.5, 4: 29.9, 8: 34.5; 1536^2 4: 48.2, 8: 46.5, 16: 57.2; 2048^2
-// 4: 71.5, 8: 67.9, 16: 75.6; 4096^2 8: 228, 16: 219, 32: 230; 6000^2 16: 446,
-// 32: 439; double 384^2 1: 20.4, 2: 21.7; 1024^2 2: 63.3, 4: 60.8, 8: 64.9;
-// 2048^2 4: 166, 8: 157, 16: 172; 3000^2 8: 326, 16: 320.  The line below lies
-// between the two sides of each of these.
-static int chosen_rows(int64_t rows1) {
-  int r = 1;
-  while (r < 32 && rows1 / (2 * r) >= 1000 + 480 * (2 * r)) r *= 2;
-  return r;
+// The height where none is asked for: the one that a launch of all the n
+// domains together is expected to finish first with (see walk_cost).
+template <class T> static int chosen_rows(int n, const hp_grid_desc* d) {
+  int best = 1;
+  double least = 0.0;
+  for (int r = 1; r <= 32; ++r) {
+    int64_t u = 0;
+    for (int k = 0; k < n; ++k) u += units(&d[k], kWalkOwn, r);
+    const double c = walk_cost<T>(u, r);
+    if (r == 1 || c < least) {
+      best = r;
+      least = c;
+    }
+  }
+  return best;
+}
+static int chosen_height(int n, const hp_grid_desc* d) {
+  return d->dtype == HP_F32 ? chosen_rows<float>(n, d) : chosen_rows<double>(n, d);
 }
 
 static int flux_rows(const hp_grid_desc* g) {
   const int r = asked_rows(g);
-  return r ? r : chosen_rows(units(g, kWalkOwn, 1));
+  return r ? r : chosen_height(1, g);
 }
 
 // Flux work units of a domain: one partial record each in the single-pass step.
@@ -885,12 +915,9 @@ struct EnsembleLayout {
 // The unit height of an ensemble: the one its domains ask for (all the same),
 // else by the units of all of them, which share one launch.
 static int ensemble_rows(int32_t n, const hp_grid_desc* d) {
-  int64_t rows1 = 0;
-  for (int k = 0; k < n; ++k) {
+  for (int k = 0; k < n; ++k)
     if (asked_rows(&d[k])) return asked_rows(&d[k]);
-    rows1 += units(&d[k], kWalkOwn, 1);
-  }
-  return chosen_rows(rows1);
+  return chosen_height(n, d);
 }
 
 static EnsembleLayout ensemble_layout(int32_t n, const hp_grid_desc* d) {
