@@ -93,9 +93,13 @@ template <class T> struct Prec;
 template <> struct Prec<double> {
   static constexpr bool local_datum = false;
   __host__ __device__ static inline double limit(double x, double y) { return minmod<double>(x, y); }
-  __host__ __device__ static inline double clamp(double x, double lo, double hi) { return fmax(fmin(x, hi), lo); }
+  // clamp to the range between a and b, in either order
+  __host__ __device__ static inline double between(double x, double a, double b) {
+    return fmax(fmin(x, fmax(a, b)), fmin(a, b));
+  }
   __host__ __device__ static inline double max2(double x, double y) { return fmax(x, y); }
   __host__ __device__ static inline double min2(double x, double y) { return fmin(x, y); }
+  __host__ __device__ static inline double max_abs(double x, double y) { return fmax(fabs(x), fabs(y)); }
   __host__ __device__ static inline double div(double a, double b) { return a / b; }
   __host__ __device__ static inline double sqrt_(double x) { return __builtin_sqrt(x); }
   // h^(-1/3) for a wet depth (h > 1e-6): a single-precision seed (relative
@@ -128,10 +132,11 @@ template <> struct Prec<float> {
   // and two selects (it differs from the product form only when x * y
   // underflows to zero)
   __device__ static inline float limit(float x, float y) { return __builtin_amdgcn_fmed3f(x, y, 0.0f); }
-  // clamp to [lo, hi] (lo <= hi) as one median-of-three
-  __device__ static inline float clamp(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
+  // clamp to the range between a and b, in either order: the median of the three
+  __device__ static inline float between(float x, float a, float b) { return __builtin_amdgcn_fmed3f(x, a, b); }
   // max / min as the bare instruction: fmaxf / fminf first quiet an input that
-  // was loaded or came through a lane shift (one more instruction each)
+  // was loaded, came through a lane shift or has its sign taken off (one more
+  // instruction each)
   __device__ static inline float max2(float x, float y) {
     float r;
     asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
@@ -140,6 +145,11 @@ template <> struct Prec<float> {
   __device__ static inline float min2(float x, float y) {
     float r;
     asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+  }
+  __device__ static inline float max_abs(float x, float y) {
+    float r;
+    asm("v_max_f32 %0, |%1|, |%2|" : "=v"(r) : "v"(x), "v"(y));
     return r;
   }
   __device__ static inline float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
@@ -258,9 +268,12 @@ template <class T> struct EdgeOut {
 // from these.  etaC / etaR: the cells' water levels used by the clamp.
 // On return eL.h/eL.z and eR.h/eR.z hold the reconstructed depth and bed.
 // off: no flux passes (both cells dry).
+// stillL / stillR: that side's momentum counts as zero (a reconstructed face
+// of a dry cell); one select of the velocity then serves both this and a dry
+// face.
 template <class T, int ORDER>
 __host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T etaC, T etaR, T& fh, T& fn, T& ft,
-                                          bool off = false) {
+                                          bool off = false, bool stillL = false, bool stillR = false) {
   // Written as straight-line code with selects: a wave whose edges fall in
   // different wave-speed regions evaluates one path instead of all three
   // under divergent branches.  Each alternative is a value of its own before
@@ -273,7 +286,7 @@ __host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T 
   // one reciprocal per face serves both velocities (in FP64 two IEEE
   // divisions become one; in FP32 the hardware reciprocal was shared anyway)
   const T rhL = P::div(T(1), eL.h), rhR = P::div(T(1), eR.h);
-  const bool dryL = lt_hs(eL.h), dryR = lt_hs(eR.h);
+  const bool dryL = either(stillL, lt_hs(eL.h)), dryR = either(stillR, lt_hs(eR.h));
   const T uLw = mul_alone(eL.qn, rhL), vLw = mul_alone(eL.qt, rhL);
   const T uRw = mul_alone(eR.qn, rhR), vRw = mul_alone(eR.qt, rhR);
   const T uL0 = dryL ? T(0) : uLw, vL0 = dryL ? T(0) : vLw;
@@ -282,9 +295,8 @@ __host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T 
   // hydrostatic reconstruction
   T wL = eL.h + eL.z;
   T wR = eR.h + eR.z;
-  const T emax = P::max2(etaC, etaR), emin = P::min2(etaC, etaR);
-  wL = P::clamp(wL, emin, emax);
-  wR = P::clamp(wR, emin, emax);
+  wL = P::between(wL, etaC, etaR);
+  wR = P::between(wR, etaC, etaR);
   if (ORDER == 1) {
     const T m = (wL + wR) / T(2);
     const bool avg = (etaC - etaR) * (wL - wR) < T(0);
@@ -486,7 +498,7 @@ __device__ inline T cfl_candidate(T h, T qx, T qy, T cfl_dx) {
   if (!gt_hs(h)) return T(60.0);
   const float gh = (float)(T(kG) * h);
   const float a = sizeof(T) == 4 ? __builtin_amdgcn_sqrtf(gh) : __builtin_sqrtf(gh);
-  return Prec<T>::div(cfl_dx, T(a) + Prec<T>::div(fmax(fabs(qx), fabs(qy)), h));
+  return Prec<T>::div(cfl_dx, T(a) + Prec<T>::div(Prec<T>::max_abs(qx, qy), h));
 }
 
 // Mask-code decode (fluxCal_jh_modified_surface_Kernel.cu:528-535): leading

@@ -43,10 +43,10 @@
 // ahead and before the row's stores, no load sits under a condition (where
 // paths join, its register would be copied, and waited for), and boundary
 // edges share the interior edges' solver call.  Measured on one MI355X, single
-// pass, order 2, per step at the chosen unit height: float 64^2 14.4 (height
-// 2) -> 11.1 us (height 1), 2048^2 72.7 -> 67.9, 8192^2 with a rain field and
-// mass sums 921 -> 824; double 2048^2 216 (an LDS tile of 64 x 4 cells per
-// block) -> 157, 256^2 17.1 (tile) -> 16.2.
+// pass, order 2, per step at the chosen unit height, from the two-row-prologue
+// walk (double: an LDS tile of 64 x 4 cells per block) to this one: float 64^2
+// 14.4 -> 8.3 us, 2048^2 72.7 -> 60.5, 8192^2 with a rain field and mass sums
+// 921 -> 814; double 2048^2 216 -> 147, 256^2 17.1 -> 12.0.
 //
 // Geometry: a unit is (strip bx, row block by); 60 columns x R rows.  Each
 // interior x edge is solved once, except the one between two strips (solved
@@ -217,7 +217,8 @@ struct WMask {
   uint64_t valid, wet;
 };
 template <class T> __device__ inline WMask walk_mask(const WRow<T>& w) {
-  return WMask{__builtin_amdgcn_ballot_w64(w.ty != 0), __builtin_amdgcn_ballot_w64(both(w.ty != 0, gt_hs(w.h)))};
+  const uint64_t valid = __builtin_amdgcn_ballot_w64(w.ty != 0);
+  return WMask{valid, valid & __builtin_amdgcn_ballot_w64(gt_hs(w.h))};
 }
 // Whether every lane is dry: no wet one, and none that is neither (a NaN).
 template <class T> __device__ inline bool walk_dry(const WMask& m, T h) {
@@ -276,6 +277,9 @@ __device__ inline void walk_edge(const WalkEnv<T>& env, DP a, const WRow<T>& A, 
   T etaC = local ? A.h : A.h + zA, etaR = B.h + zB;
   const bool vA = either(FULL, A.ty != 0), vB = either(FULL, B.ty != 0);
   const bool rim = both(need, vA != vB);
+  // (order 2: a dry cell's faces carry no momentum; a ghost's and its cell's
+  // are taken as they are)
+  bool stillA = both(ORDER == 2, lt_hs(A.h)), stillB = both(ORDER == 2, lt_hs(B.h));
   if (!FULL && __builtin_amdgcn_ballot_w64(rim) != 0) {
     if (rim) {
       const int d = vA ? D : (D + 2) & 3;
@@ -297,11 +301,12 @@ __device__ inline void walk_edge(const WalkEnv<T>& env, DP a, const WRow<T>& A, 
       hA = c.h;
       hB = gh.h;
       zA = c.z;
+      stillA = stillB = false;
     }
   }
   const bool off = both(lt_hs(hA), lt_hs(hB));
   T fh, fn, ft;
-  hllc_edge<T, ORDER>(eL, eR, etaC, etaR, fh, fn, ft, off);
+  hllc_edge<T, ORDER>(eL, eR, etaC, etaR, fh, fn, ft, off, stillA, stillB);
   // raw fluxes: the cell scales its summed increments by dt / dx once
   const T bA = T(0.5) * g * (eL.h + hA), dzA = local && FULL ? eL.z : eL.z - zA;
   const T bB = T(0.5) * g * (eR.h + hB), dzB = eR.z - zB;
@@ -333,10 +338,8 @@ __device__ inline FrameCell<T> walk_face(const WRow<T>& c, const WSlope<T>& s, T
   if (ORDER == 2) {
     f.h = fma(T(0.5) * side, s.h, c.h);
     const T fqx = fma(T(0.5) * side, s.qx, c.qx), fqy = fma(T(0.5) * side, s.qy, c.qy);
-    const bool dry = lt_hs(c.h);
-    const T fn = D == 0 ? fqx : -fqy, ft = D == 0 ? fqy : fqx;
-    f.qn = dry ? T(0) : fn;
-    f.qt = dry ? T(0) : ft;
+    f.qn = D == 0 ? fqx : -fqy;
+    f.qt = D == 0 ? fqy : fqx;
   } else {
     f.h = c.h;
     f.qn = D == 0 ? c.qx : -c.qy;
