@@ -24,6 +24,13 @@ inline int check_launch(const char* what) {
   return HP_OK;
 }
 
+// Depths at n plane offsets to copy into `row` (grid dtype).
+struct WalkGauges {
+  const int64_t* off;
+  void* row;
+  int n;
+};
+
 // What a calibration step records once its time control has run: the depths
 // at n plane offsets into `row` (grid dtype) and, when sched is set, (t, dt)
 // of the next step into sched[k_next].

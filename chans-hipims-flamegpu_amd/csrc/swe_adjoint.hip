@@ -42,13 +42,13 @@
 namespace hp {
 
 constexpr int kAThreads = 256;
-constexpr int kAChunk = 1024;  // plane elements per block of the pointwise passes
+constexpr int kAChunk = 1024;  // plane elements per block of the class sums
 constexpr int kGradStride = 16;  // doubles per block: classes 0..14, rain at 15
 constexpr int kARateCache = 64;  // station rates kept in LDS per block
 
 int grid_flux_launch(const hp_grid_desc* g, hipStream_t st);                   // swe_grid.hip
 int grid_fused_launch(const hp_grid_desc* g, bool save_flux, bool finalize, hipStream_t st,
-                      const StepRecord* rec, bool time_control);  // swe_grid.hip
+                      const StepRecord* rec, bool time_control, const WalkGauges& gauges);  // swe_grid.hip
 
 // Records (t, dt) of the control block as step k of a schedule [K+1][2].
 __global__ void k_schedule_save(const hp_ctrl* ctrl, double* sched, int k) {
@@ -134,21 +134,95 @@ __device__ inline bool adj_update_cell(int cls, T h0, T qx, T qy, T dh, T dqx, T
   return true;
 }
 
-// Reverse of rain + friction + update, kVec consecutive elements per thread
-// per access.  The derivative w.r.t. the Manning value of a cell's class goes
-// into the cell's FP64 running sum gn (folded per class once, by
-// hp_adjoint_finish); the rain-multiplier derivative is summed per block.
+// flux_listed with every load issued at once: taken one by one, the depths and
+// types of the neighbours are a chain of memory round trips.
 template <class T>
+__device__ inline bool flux_listed_flat(const hp_grid_desc& a, const T* h, T hc, int x, int y, T t) {
+  const int P = (int)a.pitch, i = y * P + x;
+  const bool in[4] = {x + 1 < a.nx, y > 0, x > 0, y + 1 < a.ny};
+  const int nb[4] = {i + 1, i - P, i - 1, i + P};
+  const int dx[4] = {1, 0, -1, 0}, dy[4] = {0, -1, 0, 1};
+  T hn[4];
+  int ty[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int j = in[k] ? nb[k] : i;
+    hn[k] = h[j];
+    ty[k] = a.type_slot[j];
+  }
+  bool on = either(t == T(0), gt_hs(hc));
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const bool other = either(x + dx[k] != a.cell0_x, y + dy[k] != a.cell0_y);
+    on = either(on, both(both(in[k], ty[k] != 0), both(gt_hs(hn[k]), other)));
+  }
+  return on;
+}
+
+// The cotangents that the edges of the valid cell (x, y) left for it.
+template <class T, int ORDER>
+__device__ inline void adj_gathered(const AdjPlanes<T>& p, int x, int y, T& sh, T& sx, T& sy) {
+  // x-edges j = x-1 (this cell is rr), x (B), x+1 (A), x+2 (l); y-edges alike
+  const int64_t C = p.cpitch;
+  const int64_t xs[4] = {(int64_t)y * C + (x + 2), (int64_t)y * C + (x + 1), (int64_t)y * C + x,
+                         (int64_t)y * C + (x - 1)};
+  const int64_t ys[4] = {(int64_t)(y + 2) * C + x, (int64_t)(y + 1) * C + x, (int64_t)y * C + x,
+                         (int64_t)(y - 1) * C + x};
+  sh = sx = sy = T(0);
+#pragma unroll
+  for (int role = ORDER == 1 ? 1 : 0; role < (ORDER == 1 ? 3 : 4); ++role) {
+    const T* bx = p.xc + (int64_t)(role * 3) * p.cplane;
+    const T* by = p.yc + (int64_t)(role * 3) * p.cplane;
+    sh += bx[xs[role]] + by[ys[role]];
+    sx += bx[p.cplane + xs[role]] + by[p.cplane + ys[role]];
+    sy += bx[2 * p.cplane + xs[role]] + by[2 * p.cplane + ys[role]];
+  }
+}
+
+// Reverse of rain + friction + update, one plane element per thread.  The
+// derivative w.r.t. the Manning value of a cell's class goes into the cell's
+// FP64 running sum gn (folded per class once, by hp_adjoint_finish); the
+// rain-multiplier derivative is summed per block.
+// GATHER (1 or 2, the order; 0: none): the cells first take what the edges of
+// the reverse step before left for them, which saves that step's own gather
+// launch and a pass over the cotangents.
+// A small domain sees the latency of one thread's loads, so they are all asked
+// for before any is used (a thread had four elements, each a chain of
+// conditional loads: 193x161 in double 10.6 us, and 4.3 for the gather; this
+// one takes about 8 with it).
+template <class T, int GATHER>
 __global__ __launch_bounds__(kAThreads) void k_adj_update(hp_grid_desc a, AdjPlanes<T> p, double* grads,
                                                           double* gn) {
   __shared__ T s_man[256];
   __shared__ T s_rb[kARateCache], s_rs[kARateCache];  // station rates: unscaled, scaled
   __shared__ double s_r[kAThreads / 64];
   const int tid = threadIdx.x;
+  const int total = (int)(a.pitch * (int64_t)a.ny);  // below 2^31
+  const int64_t at = (int64_t)blockIdx.x * kAThreads + tid;
+  const bool in = at < total;
+  const int i = in ? (int)at : 0;
+  const int y = (int)((unsigned)i / (unsigned)a.pitch), x = i - y * (int)a.pitch;
+  const int mode = a.rain_mode;
+  const T* __restrict__ h = (const T*)a.h;
+  const int cls = in ? (int)a.landuse[i] : 255;
+  const T h0 = h[i], qx0 = ((const T*)a.qx)[i], qy0 = ((const T*)a.qy)[i];
+  const T dh = ((const T*)a.dh)[i], dqx = ((const T*)a.dqx)[i], dqy = ((const T*)a.dqy)[i];
+  T lh = p.lh[i], lqx = p.lqx[i], lqy = p.lqy[i];
+  double g = gn[i];
+  const int gauge = p.gauge_of ? p.gauge_of[i] : -1;
+  const int st = mode == HP_RAIN_STATION && a.station ? (int)a.station[i] : 0;
+  const float rain = mode == HP_RAIN_FIELD ? a.rain_field[i] : 0.0f;
   const double t_now = a.ctrl->t;
   const T dt = T(a.ctrl->dt);
-  const T t_T = T(t_now);
-  const int mode = a.rain_mode;
+  const bool listed = flux_listed_flat<T>(a, h, h0, x, y, T(t_now));
+  if (GATHER != 0) {
+    const bool valid = both(in, a.type_slot[i] != 0);
+    T sh, sx, sy;
+    adj_gathered<T, GATHER == 1 ? 1 : 2>(p, valid ? x : 1, valid ? y : 1, sh, sx, sy);
+    lh = valid ? lh + sh : lh;
+    lqx = valid ? lqx + sx : lqx;
+    lqy = valid ? lqy + sy : lqy;
+  }
   for (int k = tid; k < a.n_classes; k += kAThreads) s_man[k] = ((const T*)a.manning)[k];
   const RainRows rr = wave_rain_rows(&a, t_now);
   if (mode == HP_RAIN_STATION && tid < kARateCache) {
@@ -156,70 +230,30 @@ __global__ __launch_bounds__(kAThreads) void k_adj_update(hp_grid_desc a, AdjPla
     s_rs[tid] = station_rate<T>(rr, tid, a.rain_scale);
   }
   __syncthreads();
-  const unsigned pitch32 = (unsigned)a.pitch;  // the plane has fewer than 2^31 elements
-  const T* __restrict__ h = (const T*)a.h;
-  const T* __restrict__ qx = (const T*)a.qx;
-  const T* __restrict__ qy = (const T*)a.qy;
-  const T* __restrict__ dh = (const T*)a.dh;
-  const T* __restrict__ dqx = (const T*)a.dqx;
-  const T* __restrict__ dqy = (const T*)a.dqy;
-  const T scale = T(a.rain_scale);
   double rsum = 0.0;
-  const int64_t total = a.pitch * (int64_t)a.ny;  // a multiple of 64
-  const int64_t base = (int64_t)blockIdx.x * kAChunk;
-  for (int it = 0; it < kAChunk / (kAThreads * kVec); ++it) {
-    const int64_t i0 = base + ((int64_t)it * kAThreads + tid) * kVec;
-    if (i0 >= total) break;
-    const VecU8 vl = ldv<VecU8>(a.landuse + i0);
-    const VecT<T> vh = ldv<VecT<T>>(h + i0), vqx = ldv<VecT<T>>(qx + i0), vqy = ldv<VecT<T>>(qy + i0);
-    const VecT<T> vdh = ldv<VecT<T>>(dh + i0), vdqx = ldv<VecT<T>>(dqx + i0), vdqy = ldv<VecT<T>>(dqy + i0);
-    VecT<T> lh = ldv<VecT<T>>(p.lh + i0), lqx = ldv<VecT<T>>(p.lqx + i0), lqy = ldv<VecT<T>>(p.lqy + i0);
-    if (p.gauge_of) {  // the loss cotangent of the depths after the step
-      const VecI32 vg = ldv<VecI32>(p.gauge_of + i0);
-#pragma unroll
-      for (int j = 0; j < kVec; ++j)
-        if (vg.x[j] >= 0) lh.x[j] += T(2.0 * (p.loss_h[vg.x[j]] - p.loss_obs[vg.x[j]]));
-    }
-    VecD vg = ldv<VecD>(gn + i0);
-    VecT<T> ch{}, cqx{}, cqy{}, rbv{}, rsc{};
+  if (in) {
+    if (gauge >= 0) lh += T(2.0 * (p.loss_h[gauge] - p.loss_obs[gauge]));  // the loss cotangent of the depths after the step
+    T rb = T(0), rs = T(0), c[3] = {T(0), T(0), T(0)};
     if (mode == HP_RAIN_STATION) {
-      VecI16 vs{};
-      if (a.station) vs = ldv<VecI16>(a.station + i0);
-#pragma unroll
-      for (int j = 0; j < kVec; ++j) {
-        const int st = vs.x[j];
-        const bool cached = st >= 0 && st < kARateCache;
-        rbv.x[j] = cached ? s_rb[st] : station_rate<T>(rr, st, 1.0);
-        rsc.x[j] = cached ? s_rs[st] : station_rate<T>(rr, st, a.rain_scale);
-      }
+      const bool cached = st >= 0 && st < kARateCache;
+      rb = cached ? s_rb[st] : station_rate<T>(rr, st, 1.0);
+      rs = cached ? s_rs[st] : station_rate<T>(rr, st, a.rain_scale);
     } else if (mode == HP_RAIN_FIELD) {
-      const VecF32 vf = ldv<VecF32>(a.rain_field + i0);
-#pragma unroll
-      for (int j = 0; j < kVec; ++j) {
-        rbv.x[j] = T(vf.x[j]);
-        rsc.x[j] = T(vf.x[j]) * scale;
-      }
+      rb = T(rain);
+      rs = T(rain) * T(a.rain_scale);
     }
-#pragma unroll
-    for (int j = 0; j < kVec; ++j) {
-      if (!adj_update_cell<T>(vl.x[j], vh.x[j], vqx.x[j], vqy.x[j], vdh.x[j], vdqx.x[j], vdqy.x[j], rbv.x[j], rsc.x[j],
-                              dt, s_man, lh.x[j], lqx.x[j], lqy.x[j], vg.x[j], rsum))
-        continue;
-      // the kVec elements share a row (pitch is a multiple of kVec)
-      const int y = (int)((unsigned)i0 / pitch32), x = (int)((unsigned)i0 - (unsigned)y * pitch32) + j;
-      if (flux_listed<T>(&a, h, x, y, t_T)) {
-        ch.x[j] = lh.x[j];
-        cqx.x[j] = lqx.x[j];
-        cqy.x[j] = lqy.x[j];
-      }
+    if (adj_update_cell<T>(cls, h0, qx0, qy0, dh, dqx, dqy, rb, rs, dt, s_man, lh, lqx, lqy, g, rsum) && listed) {
+      c[0] = lh;
+      c[1] = lqx;
+      c[2] = lqy;
     }
-    stv(p.lh + i0, lh);
-    stv(p.lqx + i0, lqx);
-    stv(p.lqy + i0, lqy);
-    stv(p.ch + i0, ch);
-    stv(p.cqx + i0, cqx);
-    stv(p.cqy + i0, cqy);
-    stv(gn + i0, vg);
+    p.lh[i] = lh;
+    p.lqx[i] = lqx;
+    p.lqy[i] = lqy;
+    p.ch[i] = c[0];
+    p.cqx[i] = c[1];
+    p.cqy[i] = c[2];
+    gn[i] = g;
   }
   const int lane = tid & 63, w = tid >> 6;
   for (int off = 32; off > 0; off >>= 1) rsum += __shfl_xor(rsum, off, 64);
@@ -405,13 +439,11 @@ __device__ inline void edge_adj(DP a, bool frozen_slopes, int col, int row, Cot 
   }
 }
 
-// One edge per thread.  Edges [0, nxe) are x-edges (row y, between columns
-// j-1 = A and j = B, j in [0, nx]); the rest are y-edges (column x, between
-// rows i-1 = A and i = B, i in [0, ny]).  Writes 12 cotangents per edge.
+// One edge per thread, writing 12 cotangents.  DIR 0: x-edges (row y, between
+// columns j-1 = A and j = B, j in [0, nx]); DIR 3: y-edges (column x, between
+// rows i-1 = A and i = B, i in [0, ny]).
 template <class T, int ORDER, int DIR>
-__global__ __launch_bounds__(kAThreads) void k_adj_edges(hp_grid_desc a, AdjPlanes<T> p) {
-  // DIR 0: x-edges, grid (ceil((nx+1)/256), ny); DIR 3: y-edges, grid
-  // (ceil(nx/256), ny+1).
+__device__ __forceinline__ void adj_edge_thread(const hp_grid_desc& a, const AdjPlanes<T>& p) {
   const int col = blockIdx.x * kAThreads + threadIdx.x, row = blockIdx.y;
   constexpr bool xe = DIR == 0;
   if (col >= (xe ? a.nx + 1 : a.nx) || row >= (xe ? a.ny : a.ny + 1)) return;
@@ -436,6 +468,15 @@ __global__ __launch_bounds__(kAThreads) void k_adj_edges(hp_grid_desc a, AdjPlan
   }
 }
 
+// Both directions in one launch, grid (ceil((nx+1)/256), ny+1, 2): on a small
+// domain each is bound by latency (two launches, 193x161 in double: 8.0 + 6.6
+// us), and the two fill the chip together.
+template <class T, int ORDER>
+__global__ __launch_bounds__(kAThreads) void k_adj_edges(hp_grid_desc a, AdjPlanes<T> p) {
+  if (blockIdx.z == 0) adj_edge_thread<T, ORDER, 0>(a, p);
+  else adj_edge_thread<T, ORDER, 3>(a, p);
+}
+
 template <class T, int ORDER>
 __global__ __launch_bounds__(kAThreads) void k_adj_gather(hp_grid_desc a, AdjPlanes<T> p) {
   const int64_t i = (int64_t)blockIdx.x * kAThreads + threadIdx.x;
@@ -443,21 +484,8 @@ __global__ __launch_bounds__(kAThreads) void k_adj_gather(hp_grid_desc a, AdjPla
   if (i >= total) return;
   if (a.type_slot[i] == 0) return;
   const int y = (int)(i / a.pitch), x = (int)(i - (int64_t)y * a.pitch);
-  // x-edges j = x-1 (this cell is rr), x (B), x+1 (A), x+2 (l); y-edges alike
-  const int64_t C = p.cpitch;
-  const int64_t xs[4] = {(int64_t)y * C + (x + 2), (int64_t)y * C + (x + 1), (int64_t)y * C + x,
-                         (int64_t)y * C + (x - 1)};
-  const int64_t ys[4] = {(int64_t)(y + 2) * C + x, (int64_t)(y + 1) * C + x, (int64_t)y * C + x,
-                         (int64_t)(y - 1) * C + x};
-  T sh = T(0), sx = T(0), sy = T(0);
-#pragma unroll
-  for (int role = ORDER == 1 ? 1 : 0; role < (ORDER == 1 ? 3 : 4); ++role) {
-    const T* bx = p.xc + (int64_t)(role * 3) * p.cplane;
-    const T* by = p.yc + (int64_t)(role * 3) * p.cplane;
-    sh += bx[xs[role]] + by[ys[role]];
-    sx += bx[p.cplane + xs[role]] + by[p.cplane + ys[role]];
-    sy += bx[2 * p.cplane + xs[role]] + by[2 * p.cplane + ys[role]];
-  }
+  T sh, sx, sy;
+  adj_gathered<T, ORDER>(p, x, y, sh, sx, sy);
   p.lh[i] += sh;
   p.lqx[i] += sx;
   p.lqy[i] += sy;
@@ -728,8 +756,11 @@ __global__ void k_adj_loss(T* lam_h, const int64_t* __restrict__ off, const doub
   if (k < n) lam_h[off[k]] += T(weight * 2.0 * (h_rec[k] - obs[k]));
 }
 
-template <class T>
-static int launch_adjoint(const hp_grid_desc* g, const hp_adjoint_desc* ad, hipStream_t st) {
+// One reverse step in separate passes.  gather_first: the step before this one
+// left its gather to this one's update; gather_last: this step's is done here.
+template <class T, int ORDER>
+static int launch_adjoint_order(const hp_grid_desc* g, const hp_adjoint_desc* ad, hipStream_t st, bool gather_first,
+                                bool gather_last) {
   AdjPlanes<T> p;
   p.lh = (T*)ad->lam_h; p.lqx = (T*)ad->lam_qx; p.lqy = (T*)ad->lam_qy;
   p.ch = (T*)ad->cot_h; p.cqx = (T*)ad->cot_qx; p.cqy = (T*)ad->cot_qy;
@@ -741,25 +772,27 @@ static int launch_adjoint(const hp_grid_desc* g, const hp_adjoint_desc* ad, hipS
   p.loss_h = ad->loss_h;
   p.loss_obs = ad->loss_obs;
   const int64_t total = g->pitch * (int64_t)g->ny;
-  const unsigned nbu = (unsigned)((total + kAChunk - 1) / kAChunk);
-  hipLaunchKernelGGL((k_adj_update<T>), dim3(nbu), dim3(kAThreads), 0, st, *g, p, ad->grads, ad->gn);
+  const unsigned nbu = (unsigned)((total + kAThreads - 1) / kAThreads);
+  if (gather_first)
+    hipLaunchKernelGGL((k_adj_update<T, ORDER>), dim3(nbu), dim3(kAThreads), 0, st, *g, p, ad->grads, ad->gn);
+  else hipLaunchKernelGGL((k_adj_update<T, 0>), dim3(nbu), dim3(kAThreads), 0, st, *g, p, ad->grads, ad->gn);
   int rc = check_launch("k_adj_update");
   if (rc) return rc;
-  const dim3 gx((unsigned)((g->nx + 1 + kAThreads - 1) / kAThreads), (unsigned)g->ny);
-  const dim3 gy((unsigned)((g->nx + kAThreads - 1) / kAThreads), (unsigned)(g->ny + 1));
-  if (g->order == 2) {
-    hipLaunchKernelGGL((k_adj_edges<T, 2, 0>), gx, dim3(kAThreads), 0, st, *g, p);
-    hipLaunchKernelGGL((k_adj_edges<T, 2, 3>), gy, dim3(kAThreads), 0, st, *g, p);
-  } else {
-    hipLaunchKernelGGL((k_adj_edges<T, 1, 0>), gx, dim3(kAThreads), 0, st, *g, p);
-    hipLaunchKernelGGL((k_adj_edges<T, 1, 3>), gy, dim3(kAThreads), 0, st, *g, p);
-  }
+  const dim3 ge((unsigned)((g->nx + 1 + kAThreads - 1) / kAThreads), (unsigned)(g->ny + 1), 2);
+  hipLaunchKernelGGL((k_adj_edges<T, ORDER>), ge, dim3(kAThreads), 0, st, *g, p);
   rc = check_launch("k_adj_edges");
-  if (rc) return rc;
+  if (rc || !gather_last) return rc;
   const unsigned nbg = (unsigned)((total + kAThreads - 1) / kAThreads);
-  if (g->order == 2) hipLaunchKernelGGL((k_adj_gather<T, 2>), dim3(nbg), dim3(kAThreads), 0, st, *g, p);
-  else hipLaunchKernelGGL((k_adj_gather<T, 1>), dim3(nbg), dim3(kAThreads), 0, st, *g, p);
+  hipLaunchKernelGGL((k_adj_gather<T, ORDER>), dim3(nbg), dim3(kAThreads), 0, st, *g, p);
   return check_launch("k_adj_gather");
+}
+static int launch_adjoint(const hp_grid_desc* g, const hp_adjoint_desc* ad, hipStream_t st, bool gather_first = false,
+                          bool gather_last = true) {
+  if (g->dtype == HP_F32)
+    return (g->order == 2 ? launch_adjoint_order<float, 2> : launch_adjoint_order<float, 1>)(g, ad, st, gather_first,
+                                                                                             gather_last);
+  return (g->order == 2 ? launch_adjoint_order<double, 2> : launch_adjoint_order<double, 1>)(g, ad, st, gather_first,
+                                                                                             gather_last);
 }
 
 }  // namespace hp
@@ -771,7 +804,7 @@ extern "C" {
 int64_t hp_adjoint_grad_blocks(const hp_grid_desc* g) {
   if (!g || g->pitch <= 0 || g->ny <= 0) return 0;
   // rows for the blocks of k_adj_update and for those of the tiled step
-  const int64_t nu = (g->pitch * (int64_t)g->ny + kAChunk - 1) / kAChunk;
+  const int64_t nu = (g->pitch * (int64_t)g->ny + kAThreads - 1) / kAThreads;
   const int64_t nt = g->dtype == HP_F32 ? adj_tile_count<float>(g) : adj_tile_count<double>(g);
   return nu > nt ? nu : nt;
 }
@@ -800,8 +833,7 @@ int hp_adjoint_step(const hp_grid_desc* g, const hp_adjoint_desc* ad, void* stre
     int rc = grid_flux_launch(g, (hipStream_t)stream);  // recompute the step's flux on U_k
     if (rc) return rc;
   }
-  if (g->dtype == HP_F32) return launch_adjoint<float>(g, ad, (hipStream_t)stream);
-  return launch_adjoint<double>(g, ad, (hipStream_t)stream);
+  return launch_adjoint(g, ad, (hipStream_t)stream);
 }
 
 int hp_adjoint_finish(const hp_grid_desc* g, const hp_adjoint_desc* ad, void* stream) {
@@ -908,15 +940,17 @@ int hp_calib_forward(const hp_grid_desc* g, double* sched, const hp_ctrl* frozen
     const int n = gauges ? n_gauges : 0;
     char* row = gauges ? (char*)hist + (int64_t)(k + 1) * n_gauges * esz : nullptr;
     // with time control the record rides on its kernel; a frozen schedule
-    // has none, so the gauges then take a small kernel of their own
+    // has none: the gauges of a state then ride on the step that starts from
+    // it, those of the last one take a small kernel of their own
     const StepRecord rec{out[0], gauge_off, n, row, save, k + 1, g->dtype == HP_F32};
     const bool ride = !frozen && (gauges || save);
-    // a frozen segment (the reverse sweep's recomputation, or a frozen run's
-    // last segment) needs no CFL candidates: no time control follows
-    const bool time_control = !(frozen && seg_u);
-    if ((rc = grid_fused_launch(&d, seg_u != nullptr, frozen == nullptr, st, ride ? &rec : nullptr, time_control)))
+    WalkGauges before{};
+    if (frozen && gauges && j > 0) before = WalkGauges{gauge_off, row - n * esz, n};
+    // (a frozen schedule needs no CFL candidates: no time control follows)
+    if ((rc = grid_fused_launch(&d, seg_u != nullptr, frozen == nullptr, st, ride ? &rec : nullptr, frozen == nullptr,
+                                before)))
       return rc;
-    if (frozen && gauges) {
+    if (frozen && gauges && j + 1 == nsteps) {
       const unsigned nb = (unsigned)((n > 0 ? n : 1) + 255) / 256;
       if (g->dtype == HP_F32)
         hipLaunchKernelGGL(k_step_record<float>, dim3(nb), dim3(256), 0, st, (const float*)out[0], gauge_off, n,
@@ -977,7 +1011,11 @@ int hp_calib_reverse(const hp_grid_desc* g, const hp_adjoint_desc* ad, const hp_
       cur = nxt;
       nxt = t;
     } else {
-      rc = hp_adjoint_step(&d, &a, stream);
+      // the cotangents of a step's edges are gathered by the next step's
+      // update (a loss added between the two needs them gathered before)
+      const bool defer = a.gauge_of || n_gauges <= 0;
+      if (int e = check_adjoint(&d, &a)) return e;
+      rc = launch_adjoint(&d, &a, st, defer && k + 1 < k_hi, !defer || k == k_lo);
     }
     if (rc) return rc;
   }

@@ -727,7 +727,7 @@ template <class T> static double walk_cost(int64_t u, int r) {
   const double *row = sizeof(T) == 4 ? kRowF : kRowD, *start = sizeof(T) == 4 ? kStartF : kStartD;
   const double x = (double)u / walk_slots<T>();
   const bool many = x > 4.0;
-  const double rounds = many ? x + 0.25 : std::ceil(x + (x > 1.0 ? 0.02 : 0.05));
+  const double rounds = many ? x + 0.25 : (double)(1 + (int)(x + (x > 1.0 ? 0.02 : 0.05)));
   const int i = (int)(rounds > 1.0 ? walk_waves<T>() : (u + kSimds - 1) / kSimds) - 1;
   return start[i] + rounds * row[i] * r * (many ? 1.0 : 1.0 + 0.0025 * r) + 5.0 * (rounds - 1.0);
 }
@@ -754,7 +754,7 @@ template <class T> static int chosen_rows(int n, const hp_grid_desc* d) {
   double least = 0.0;
   for (int r = 1; r <= 32; ++r) {
     int64_t u = 0;
-    for (int k = 0; k < n; ++k) u += units(&d[k], kWalkOwn, r);
+    for (int k = 0; k < n; ++k) u += (int64_t)((d[k].nx + kWalkOwn - 1) / kWalkOwn) * ((d[k].ny + r - 1) / r);
     const double c = walk_cost<T>(u, r);
     if (r == 1 || c < least) {
       best = r;
@@ -826,19 +826,22 @@ static int check_desc(const hp_grid_desc* g) {
 }
 
 // A folded step: its place in the call and the record arrays of this step and
-// the one before (null without mass sums).
+// the one before (null without mass sums).  A step that is not folded (st
+// null) may take the gauge depths of the state that it starts from.
 struct FoldStep {
   FoldState* st;
   int k;
   Sums *records, *prev;
+  WalkGauges gauges;
 };
 
 template <class T, int ORDER, bool FUSED>
 static int launch_walk_t(const hp_grid_desc* g, hipStream_t st, int flags, const FoldStep& f) {
   const int rows = flux_rows(g), ns = (g->nx + kWalkOwn - 1) / kWalkOwn;
-  const int n = (int)units(g, kWalkOwn, rows), extra = f.st && f.records ? kFoldSumBlocks : 0;
+  const int n = (int)units(g, kWalkOwn, rows);
+  const int extra = f.st && f.records ? kFoldSumBlocks : (f.gauges.n + kWalkLanes - 1) / kWalkLanes;
   hipLaunchKernelGGL((k_walk<T, ORDER, FUSED>), dim3((unsigned)(n + extra)), dim3(kWalkLanes), 0, st, *g,
-                     Divisor::of(ns), rows, flags, n, WalkFold{f.st, f.k, f.records}, f.prev);
+                     Divisor::of(ns), rows, flags, n, WalkFold{f.st, f.k, f.records}, f.prev, f.gauges);
   return check_launch(FUSED ? "k_walk (single-pass step)" : "k_walk (flux pass)");
 }
 
@@ -999,9 +1002,10 @@ __global__ void k_scatter(T* __restrict__ plane, const int64_t* __restrict__ off
 // step's flux also into dh, dqx, dqy) and, with finalize, its time control,
 // followed by rec when given; without time_control the step computes no
 // CFL candidates, sums or partial records (no time control may follow).
+// gauges: those of the state before the step.
 // Shared with the calibration runs.
 int grid_fused_launch(const hp_grid_desc* g, bool save_flux, bool finalize, hipStream_t st, const StepRecord* rec,
-                      bool time_control) {
+                      bool time_control, const WalkGauges& gauges) {
   int rc = check_desc(g);
   if (rc) return rc;
   if (!g->h_out || !g->qx_out || !g->qy_out) return fail(HP_EINVAL, "the fused step needs h_out, qx_out, qy_out");
@@ -1009,7 +1013,9 @@ int grid_fused_launch(const hp_grid_desc* g, bool save_flux, bool finalize, hipS
   if (!g->work || g->work_bytes < partials_bytes(flux_tiles(g)))
     return fail(HP_ESPACE, "workspace smaller than hp_grid_workspace_bytes()");
   if (finalize && !time_control) return fail(HP_EINVAL, "a time control needs the step's CFL candidates");
-  rc = launch_step_fused(g, st, (save_flux ? 1 : 0) | (time_control ? 0 : 2));
+  FoldStep f{};
+  f.gauges = gauges;
+  rc = launch_step_fused(g, st, (save_flux ? 1 : 0) | (time_control ? 0 : 2), f);
   if (rc || !finalize) return rc;
   return launch_finalize_fused(g, st, rec);
 }

@@ -770,14 +770,21 @@ template <class T> constexpr int walk_slots() { return kSimds * walk_waves<T>();
 // outputs (a frozen schedule); 4 a stopped domain copies its state through
 // even when marked in step.
 // With fold.st set, the grid may begin with blocks that fold the FP64 sums of
-// the step before (n_units: the blocks that walk).
+// the step before (n_units: the blocks that walk); without it, with blocks
+// that copy the gauge depths of the state the step starts from (a launch of
+// its own for those cost a calibration step 3 us).
 template <class T, int ORDER, bool FUSED>
 __global__ __launch_bounds__(kWalkLanes, walk_waves<T>()) void k_walk(hp_grid_desc a, Divisor strips, int rows,
                                                                        int flags, int n_units, WalkFold fold,
-                                                                       const Sums* prev) {
+                                                                       const Sums* prev, WalkGauges gauges) {
   const KDesc pa = kernarg_desc();
   const int extra = (int)gridDim.x - n_units;
   if (FUSED && (int)blockIdx.x < extra) {
+    if (fold.st == nullptr) {
+      const int i = (int)(blockIdx.x * kWalkLanes + threadIdx.x);
+      if (i < gauges.n) ((T*)gauges.row)[i] = ((const T*)pa->h)[gauges.off[i]];
+      return;
+    }
     fold_sums_block(pa->ctrl, fold.st, fold.k, (int)blockIdx.x, prev, n_units, pa->dx);
     return;
   }
