@@ -43,7 +43,6 @@
 namespace hp {
 
 constexpr int kThreads = 256;
-constexpr int kChunk = 2048;  // plane elements per update block
 constexpr int kMaxStations = 1024;
 constexpr int kRateCache = 64;  // station rates kept in LDS per block; further stations are evaluated per cell
 
@@ -380,15 +379,25 @@ __global__ __launch_bounds__(kThreads) void k_infiltration(hp_grid_desc a) {
   const int row = (int)(i / pitch), col = (int)(i - row * pitch);
   T dF = T(0);
   if (col < a.nx && ty[i] != 0) {
-    bool listed = T(a.ctrl->t) == T(0) || gt_hs(h[i]);
+    // (every neighbour is asked for before any is used: in turn, each would
+    // wait for the one before)
     const int nr[4] = {row, row - 1, row, row + 1};
     const int nc[4] = {col + 1, col, col - 1, col};
+    bool in[4];
+    T hn[4];
+    int tn[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      if (nr[k] < 0 || nr[k] >= a.ny || nc[k] < 0 || nc[k] >= a.nx) continue;
-      const int64_t j = (int64_t)nr[k] * pitch + nc[k];
-      const bool is0 = nc[k] == a.cell0_x && nr[k] == a.cell0_y;
-      listed = listed || (ty[j] != 0 && !is0 && gt_hs(h[j]));
+      in[k] = both(both(nr[k] >= 0, nr[k] < a.ny), both(nc[k] >= 0, nc[k] < a.nx));
+      const int64_t j = in[k] ? (int64_t)nr[k] * pitch + nc[k] : i;
+      hn[k] = h[j];
+      tn[k] = ty[j];
+    }
+    bool listed = either(T(a.ctrl->t) == T(0), gt_hs(h[i]));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool other = either(nc[k] != a.cell0_x, nr[k] != a.cell0_y);
+      listed = either(listed, both(both(in[k], tn[k] != 0), both(other, gt_hs(hn[k]))));
     }
     if (listed) {
       const int cls = a.landuse[i];
@@ -409,138 +418,181 @@ __global__ __launch_bounds__(kThreads) void k_infiltration(hp_grid_desc a) {
 //                       h > 1e-6; q += dq without friction; no CFL
 //   HP_UPDATE_CFL       time_update_cuda (:726-764): cells with h > 1e-6; no
 //                       state change and no rain; h_max, CFL + dt/t
-// Processes plane elements [chunk*kChunk, (chunk+1)*kChunk) and writes one
-// partial record.
-template <class T, int MODE>
-__device__ inline void update_chunk(const hp_grid_desc& a, int64_t chunk, const Partials& part, int64_t pidx) {
-  __shared__ T s_man[256];
-  __shared__ T s_rate[kRateCache];
-  const int tid = threadIdx.x;
+// Processes a chunk of kThreads * update_loops() plane elements and writes one
+// partial record.  On a small domain a launch lasts as long as one thread's
+// chain of loads, divisions and square roots, so a thread has one element
+// (with eight, in vectors of four, a 75x75 domain in double took 13.2 us and
+// takes 5.6).  Past 1024 blocks the elements per thread grow to eight, so that
+// one block can fold the records: one at a time in double (2048^2 with the
+// time control: 75 -> 68 us), in vectors of four in float, which moves half
+// the bytes per access (3000^2: 74 us one at a time, 69 in vectors).
+__host__ __device__ inline int update_loops(int64_t total) {
+  int n = 1;
+  while (n < 8 && total > (int64_t)n * kThreads * 1024) n *= 2;
+  return n;
+}
+
+// W consecutive elements of the planes.
+template <class T, int W> struct UpdateIn {
+  T h[W], qx[W], qy[W], hm[W], dh[W], dqx[W], dqy[W], df[W];
+  float rain[W];
+  uint8_t cls[W];
+  int16_t st[W];
+};
+template <int W, class V> __device__ inline void load_w(V (&to)[W], const V* p) {
+  struct alignas(W * sizeof(V)) Vec {
+    V x[W];
+  };
+  const Vec v = *reinterpret_cast<const Vec*>(p);
+#pragma unroll
+  for (int j = 0; j < W; ++j) to[j] = v.x[j];
+}
+template <int W, class V> __device__ inline void store_w(V* p, const V (&from)[W]) {
+  struct alignas(W * sizeof(V)) Vec {
+    V x[W];
+  } v;
+#pragma unroll
+  for (int j = 0; j < W; ++j) v.x[j] = from[j];
+  *reinterpret_cast<Vec*>(p) = v;
+}
+
+template <class T, int MODE, int W>
+__device__ inline void update_elements(const hp_grid_desc& a, int64_t base, int rounds, int64_t total,
+                                       const Partials& part, int64_t pidx, T* s_man, T* s_rate) {
+  const int tid = threadIdx.x, mode = a.rain_mode;
+  // (past the end: the last elements again, with the class of no cell)
+  auto load = [&](int it) {
+    const int64_t at = base + ((int64_t)it * kThreads + tid) * W, i = at < total ? at : total - W;
+    UpdateIn<T, W> c{};
+    load_w(c.cls, a.landuse + i);
+    if (at >= total) {
+#pragma unroll
+      for (int j = 0; j < W; ++j) c.cls[j] = 255;
+    }
+    load_w(c.h, (const T*)a.h + i);
+    load_w(c.qx, (const T*)a.qx + i);
+    load_w(c.qy, (const T*)a.qy + i);
+    load_w(c.hm, (const T*)a.h_max + i);
+    if (MODE != HP_UPDATE_CFL) {
+      if (a.infil_dF) load_w(c.df, (const T*)a.infil_dF + i);
+      load_w(c.dh, (const T*)a.dh + i);
+      load_w(c.dqx, (const T*)a.dqx + i);
+      load_w(c.dqy, (const T*)a.dqy + i);
+      if (mode == HP_RAIN_STATION && a.station) load_w(c.st, a.station + i);
+      else if (mode == HP_RAIN_FIELD) load_w(c.rain, a.rain_field + i);
+    }
+    return c;
+  };
+  UpdateIn<T, W> c = load(0);  // before the tables, whose round trips it overlaps
   if (stopped(a.ctrl)) {
     if (tid == 0) part.put(pidx, INFINITY, 0.0, 0.0, 0.0, a.mass_sums != 0);
     return;
   }
   const T dt = T(a.ctrl->dt);
-  const T cfl_dx = T(a.cfl) * T(a.dx);
+  const T cfl_dx = T(a.cfl) * T(a.dx), rscale = T(a.rain_scale);
   for (int k = tid; k < a.n_classes; k += kThreads) s_man[k] = ((const T*)a.manning)[k];
   const RainRows rr = wave_rain_rows(&a, a.ctrl->t);
-  const int mode = a.rain_mode;
   if (mode == HP_RAIN_STATION && tid < kRateCache) s_rate[tid] = station_rate<T>(rr, tid, a.rain_scale);
   __syncthreads();
-
-  const T* __restrict__ dhp = (const T*)a.dh;
-  const T* __restrict__ dqxp = (const T*)a.dqx;
-  const T* __restrict__ dqyp = (const T*)a.dqy;
-  T* __restrict__ hp_ = (T*)a.h;
-  T* __restrict__ qxp = (T*)a.qx;
-  T* __restrict__ qyp = (T*)a.qy;
-  T* __restrict__ hmp = (T*)a.h_max;
-  const uint8_t* __restrict__ lu = a.landuse;
-  const int16_t* __restrict__ st = a.station;
-  const float* __restrict__ rf = a.rain_field;
-  const T* __restrict__ dfp = (const T*)a.infil_dF;
-  const T rscale = T(a.rain_scale);
-
   const bool sums = a.mass_sums != 0;
   T mn = T(INFINITY);
   double vol = 0.0, fsum = 0.0, rsum = 0.0;
-  const int64_t total = a.pitch * (int64_t)a.ny;  // a multiple of 64
-  const int64_t base = chunk * kChunk;
-  for (int it = 0; it < kChunk / (kThreads * kVec); ++it) {
-    const int64_t i0 = base + ((int64_t)it * kThreads + tid) * kVec;
-    if (i0 >= total) break;
-    const VecU8 vl = ldv<VecU8>(lu + i0);
-    VecT<T> vh = ldv<VecT<T>>(hp_ + i0);
-    VecT<T> vqx = ldv<VecT<T>>(qxp + i0);
-    VecT<T> vqy = ldv<VecT<T>>(qyp + i0);
-    VecT<T> vhm = ldv<VecT<T>>(hmp + i0);
-    VecT<T> vdh{}, vdqx{}, vdqy{}, vr{}, vdf{};
-    if (MODE != HP_UPDATE_CFL) {
-      if (dfp) vdf = ldv<VecT<T>>(dfp + i0);
-      vdh = ldv<VecT<T>>(dhp + i0);
-      vdqx = ldv<VecT<T>>(dqxp + i0);
-      vdqy = ldv<VecT<T>>(dqyp + i0);
-      if (mode == HP_RAIN_STATION) {
-        VecI16 vs{};
-        if (st) vs = ldv<VecI16>(st + i0);
+  for (int it = 0;; ++it) {
+    const bool more = it + 1 < rounds;
+    UpdateIn<T, W> next{};
+    if (W == 1 && more) next = load(it + 1);  // (vectors ahead would halve the waves in flight)
+    const int64_t i = base + ((int64_t)it * kThreads + tid) * W;
 #pragma unroll
-        for (int j = 0; j < kVec; ++j) {
-          const int k = vs.x[j];
-          vr.x[j] = (k >= 0 && k < kRateCache) ? s_rate[k] : station_rate<T>(rr, k, a.rain_scale);
-        }
-      } else if (mode == HP_RAIN_FIELD) {
-        const VecF32 vf = ldv<VecF32>(rf + i0);
-#pragma unroll
-        for (int j = 0; j < kVec; ++j) vr.x[j] = T(vf.x[j]) * rscale;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kVec; ++j) {
-      const int cls = vl.x[j];
-      if (cls == 255) continue;
-      T h = vh.x[j];
+    for (int j = 0; j < W; ++j) {
+      if (c.cls[j] == 255) continue;
+      T h = c.h[j];
       if (MODE == HP_UPDATE_CFL) {
         if (gt_hs(h)) {
-          vhm.x[j] = fmax(h, vhm.x[j]);
-          mn = fmin(mn, cfl_candidate<T>(h, vqx.x[j], vqy.x[j], cfl_dx));
+          c.hm[j] = fmax(h, c.hm[j]);
+          mn = fmin(mn, cfl_candidate<T>(h, c.qx[j], c.qy[j], cfl_dx));
         }
-        if (sums) vol += (double)h;
-        continue;
-      }
-      const T dhf = vdh.x[j];
-      const T rdt = vr.x[j] * dt;
-      const T dht = (dhf + rdt) - vdf.x[j];  // flux, + rain, - infiltration (the reference's order)
-      const bool listed = (MODE == HP_UPDATE_EULER) ? (fabs(dht) > T(0) || gt_hs(h)) : (fabs(dht) > T(0) || h >= T(0));
-      if (!listed) {
-        if (sums) vol += (double)h;
-        continue;
-      }
-      const bool dry = new_depth_dry(h, dht);
-      T qx, qy;
-      if (MODE == HP_UPDATE_EULER) {
-        qx = vqx.x[j] + vdqx.x[j];
-        qy = vqy.x[j] + vdqy.x[j];
-      } else if (dry) {
-        qx = T(0);
-        qy = T(0);
       } else {
-        qx = vqx.x[j] + vdqx.x[j];
-        qy = vqy.x[j] + vdqy.x[j];
-        implicit_friction<T>(h, s_man[cls], dt, qx, qy);
+        T rate = T(0);
+        if (mode == HP_RAIN_STATION) {
+          const int k = c.st[j];
+          rate = (k >= 0 && k < kRateCache) ? s_rate[k] : station_rate<T>(rr, k, a.rain_scale);
+        } else if (mode == HP_RAIN_FIELD) {
+          rate = T(c.rain[j]) * rscale;
+        }
+        const T rdt = rate * dt;
+        const T dht = (c.dh[j] + rdt) - c.df[j];  // flux, + rain, - infiltration (the reference's order)
+        const bool listed =
+            (MODE == HP_UPDATE_EULER) ? (fabs(dht) > T(0) || gt_hs(h)) : (fabs(dht) > T(0) || h >= T(0));
+        if (listed) {
+          const bool dry = new_depth_dry(h, dht);
+          T qx = T(0), qy = T(0);
+          if (MODE == HP_UPDATE_EULER || !dry) {
+            qx = c.qx[j] + c.dqx[j];
+            qy = c.qy[j] + c.dqy[j];
+            if (MODE != HP_UPDATE_EULER) implicit_friction<T>(h, s_man[c.cls[j]], dt, qx, qy);
+          }
+          c.h[j] = h;
+          c.qx[j] = qx;
+          c.qy[j] = qy;
+          if (MODE == HP_UPDATE_STEP) {
+            c.hm[j] = fmax(h, c.hm[j]);
+            mn = fmin(mn, cfl_candidate<T>(h, qx, qy, cfl_dx));
+          }
+          if (sums) {
+            fsum += (double)c.dh[j];
+            rsum += (double)rdt;
+          }
+        }
       }
-      vh.x[j] = h;
-      vqx.x[j] = qx;
-      vqy.x[j] = qy;
-      if (MODE == HP_UPDATE_STEP) {
-        vhm.x[j] = fmax(h, vhm.x[j]);
-        mn = fmin(mn, cfl_candidate<T>(h, qx, qy, cfl_dx));
-      }
-      if (sums) {
-        vol += (double)h;
-        fsum += (double)dhf;
-        rsum += (double)rdt;
-      }
+      if (sums) vol += (double)h;
     }
-    if (MODE != HP_UPDATE_CFL) {
-      stv(hp_ + i0, vh);
-      stv(qxp + i0, vqx);
-      stv(qyp + i0, vqy);
+    if (i < total) {
+      if (MODE != HP_UPDATE_CFL) {
+        store_w((T*)a.h + i, c.h);
+        store_w((T*)a.qx + i, c.qx);
+        store_w((T*)a.qy + i, c.qy);
+      }
+      if (MODE == HP_UPDATE_STEP || MODE == HP_UPDATE_CFL) store_w((T*)a.h_max + i, c.hm);
     }
-    if (MODE == HP_UPDATE_STEP || MODE == HP_UPDATE_CFL) stv(hmp + i0, vhm);
+    if (!more) break;
+    c = W == 1 ? next : load(it + 1);
   }
   block_partial<T>(mn, vol, fsum, rsum, part, pidx, sums);
 }
 
-template <class T, int MODE>
-__global__ __launch_bounds__(kThreads) void k_update(hp_grid_desc a) {
-  update_chunk<T, MODE>(a, blockIdx.x, Partials(a.work, gridDim.x), blockIdx.x);
+// Elements per access of a domain's update.
+template <class T> __host__ __device__ inline int update_width(int64_t total) {
+  return sizeof(T) == 4 && update_loops(total) == 8 ? kVec : 1;
 }
 
+template <class T, int MODE, int W>
+__device__ inline void update_chunk(const hp_grid_desc& a, int64_t chunk, const Partials& part, int64_t pidx, T* s_man,
+                                    T* s_rate) {
+  const int64_t total = a.pitch * (int64_t)a.ny;  // a multiple of kVec
+  const int loops = update_loops(total);
+  update_elements<T, MODE, W>(a, chunk * kThreads * loops, loops / W, total, part, pidx, s_man, s_rate);
+}
+
+template <class T, int MODE, int W>
+__global__ __launch_bounds__(kThreads) void k_update(hp_grid_desc a) {
+  __shared__ T s_man[256];
+  __shared__ T s_rate[kRateCache];
+  update_chunk<T, MODE, W>(a, blockIdx.x, Partials(a.work, gridDim.x), blockIdx.x, s_man, s_rate);
+}
+
+// (the domains of an ensemble differ in size: each as it runs alone, so that
+// its sums keep their bits)
 template <class T, int MODE>
 __global__ __launch_bounds__(kThreads) void k_update_multi(const hp_grid_desc* __restrict__ doms,
                                                            const int2* __restrict__ map, void* parts) {
+  __shared__ T s_man[256];
+  __shared__ T s_rate[kRateCache];
   const int2 m = map[blockIdx.x];
-  update_chunk<T, MODE>(doms[m.x], m.y, Partials(parts, gridDim.x), blockIdx.x);
+  const hp_grid_desc& a = doms[m.x];
+  const Partials part(parts, gridDim.x);
+  if (update_width<T>(a.pitch * (int64_t)a.ny) != 1)
+    update_chunk<T, MODE, kVec>(a, m.y, part, blockIdx.x, s_man, s_rate);
+  else update_chunk<T, MODE, 1>(a, m.y, part, blockIdx.x, s_man, s_rate);
 }
 
 // Fold a domain's partials in a fixed order and advance its time control.
@@ -697,7 +749,8 @@ __global__ __launch_bounds__(1024) void k_finalize_multi(const hp_grid_desc* __r
 // --- host side -------------------------------------------------------------
 static int64_t update_blocks(const hp_grid_desc* g) {
   const int64_t total = g->pitch * (int64_t)g->ny;
-  return (total + kChunk - 1) / kChunk;
+  const int64_t chunk = (int64_t)kThreads * update_loops(total);
+  return (total + chunk - 1) / chunk;
 }
 
 static int64_t units(const hp_grid_desc* g, int cols, int rows) {
@@ -879,8 +932,10 @@ static int launch_infiltration(const hp_grid_desc* g, hipStream_t st) {
 
 template <int MODE>
 static void launch_update_mode(const hp_grid_desc* g, int64_t nb, hipStream_t st) {
-  if (g->dtype == HP_F32) hipLaunchKernelGGL((k_update<float, MODE>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
-  else hipLaunchKernelGGL((k_update<double, MODE>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
+  const bool wide = g->dtype == HP_F32 && update_width<float>(g->pitch * (int64_t)g->ny) != 1;
+  if (wide) hipLaunchKernelGGL((k_update<float, MODE, kVec>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
+  else if (g->dtype == HP_F32) hipLaunchKernelGGL((k_update<float, MODE, 1>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
+  else hipLaunchKernelGGL((k_update<double, MODE, 1>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
 }
 
 static int launch_update(const hp_grid_desc* g, int mode, hipStream_t st) {

@@ -422,7 +422,8 @@ __host__ __device__ inline void implicit_friction(T h, T n, T dt, T& qx, T& qy) 
   using P = Prec<T>;
   const T g = T(kG);
   const T C_f = g * n * n * Prec<T>::rcbrt_friction(h);
-  const T q_norm = P::sqrt_(qx * qx + qy * qy);
+  // (which of the two products is the fused one must not depend on the caller)
+  const T q_norm = P::sqrt_(fma(qx, qx, mul_alone(qy, qy)));
   const T lim = T(5) * h * P::sqrt_(h * g);
   if (P::local_datum) {
     // cancellation-free: (1 - sqrt(1 + x)) / (-(x/2) / q_k) == 2 q_k / (1 + sqrt(1 + x))
@@ -439,27 +440,19 @@ __host__ __device__ inline void implicit_friction(T h, T n, T dt, T& qx, T& qy) 
     qx = both(rough, fabs(qx) > T(1.0e-10)) ? ox : qx;
     qy = both(rough, fabs(qy) > T(1.0e-10)) ? oy : qy;
   } else {
-    if (!(n > T(0))) return;
-    if (fabs(qx) > T(1.0e-10)) {
-      const T tmp = (T(1) - P::sqrt_(T(1) + (T(4) * dt * C_f) / (h * h) * q_norm)) /
-                    (T(-2) * dt * C_f / (h * h) * (q_norm / qx));
-      if (fabs(tmp) > lim) {
-        qx = T(2) * tmp - qx;
-        if (qx * tmp <= T(0)) qx = T(0);
-      } else {
-        qx = tmp;
-      }
-    }
-    if (fabs(qy) > T(1.0e-10)) {
-      const T tmp = (T(1) - P::sqrt_(T(1) + (T(4) * dt * C_f) / (h * h) * q_norm)) /
-                    (T(-2) * dt * C_f / (h * h) * (q_norm / qy));
-      if (fabs(tmp) > lim) {
-        qy = T(2) * tmp - qy;
-        if (qy * tmp <= T(0)) qy = T(0);
-      } else {
-        qy = tmp;
-      }
-    }
+    // both components side by side, as selects: one's chain of division and
+    // square root hides the other's (a component left as it is may form
+    // anything on the way).  -2 dt C_f / h^2 is exactly -1/2 of 4 dt C_f / h^2.
+    const T x4 = (T(4) * dt * C_f) / (h * h), x2 = T(-0.5) * x4;
+    const T num = T(1) - P::sqrt_(T(1) + x4 * q_norm);
+    const T tx = num / (x2 * (q_norm / qx)), ty = num / (x2 * (q_norm / qy));
+    const T rx = T(2) * tx - qx, ry = T(2) * ty - qy;
+    const T zx = rx * tx <= T(0) ? T(0) : rx, zy = ry * ty <= T(0) ? T(0) : ry;
+    const T ox = fabs(tx) > lim ? zx : tx;
+    const T oy = fabs(ty) > lim ? zy : ty;
+    const bool rough = n > T(0);
+    qx = both(rough, fabs(qx) > T(1.0e-10)) ? ox : qx;
+    qy = both(rough, fabs(qy) > T(1.0e-10)) ? oy : qy;
   }
 }
 
