@@ -35,6 +35,33 @@ __device__ inline T c_series_at(const T* tab, int rows, int w, int row, int col)
   return tab[row * w + col];
 }
 
+// Boundary ghost of cell c (outward direction d) and its water level.  Only the
+// series that the type uses is searched.
+template <class T, int ORDER>
+__device__ inline FrameCell<T> c_ghost(int32_t code, const FrameCell<T>& c, int d, T c_wl, T zref, T t, const T* gd,
+                                       int gd_rows, int gd_w, const T* gwl, int gwl_rows, int gwl_w, const T* gq,
+                                       int gq_rows, int gq_w, T& eta) {
+  int type, id;
+  decode_code(code, type, id);
+  T bd = T(0), bw = T(0), bqx = T(0), bqy = T(0);
+  if (type == 6) bd = c_series_at(gd, gd_rows, gd_w, c_series_row(gd, gd_rows, gd_w, t), id + 1);
+  if (type == 8) bw = c_series_at(gwl, gwl_rows, gwl_w, c_series_row(gwl, gwl_rows, gwl_w, t), id + 1) - zref;
+  if (type == 7) {
+    const int rq = c_series_row(gq, gq_rows, gq_w, t);
+    bqx = c_series_at(gq, gq_rows, gq_w, rq, 1 + 2 * id);
+    bqy = c_series_at(gq, gq_rows, gq_w, rq, 2 + 2 * id);
+  }
+  const FrameCell<T> g = bc_ghost<T>(type, c, d, bd, bw, bqx, bqy);
+  eta = ORDER == 1 ? g.h + g.z : ghost_wl<T>(type, c_wl, g, bw);
+  return g;
+}
+
+// The flux of one listed cell: its four edges, each solved from the cell's own
+// side.  The loads form three round trips (the cell's neighbours, theirs
+// beyond, the states), each asked for as a whole before the first edge: edge
+// by edge they were twelve in turn.  Interior and boundary edges share the
+// solver call.  1500x1301 cells, order 2, float: 80 -> 45 us; 701x503, a basin,
+// order 1, double: 21.8 -> 16.4.
 template <class T, int ORDER>
 __global__ __launch_bounds__(kCThreads) void k_flux_compact(
     int64_t M, int64_t N, const int32_t* __restrict__ wet, T* __restrict__ dh, T* __restrict__ dqx,
@@ -47,47 +74,53 @@ __global__ __launch_bounds__(kCThreads) void k_flux_compact(
   const T dx = dxp[0], t = tp[0], dt = dtp[0];
   const T dt_dx = dt / dx;
   const int32_t i = wet[w];
+  struct Cell {
+    T h, qx, qy, z;
+  };
+  int32_t rid[4], rrid[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) rid[d] = index[(int64_t)(d + 1) * N + i];
   const int32_t code = index[i];
-  const T zref = Prec<T>::local_datum ? z[i] : T(0);
+  const Cell self{h[i], qx[i], qy[i], z[i]};
+  const T self_wl = ORDER == 1 ? T(0) : wl[i];
   T ah = dh[i], aqx = dqx[i], aqy = dqy[i];
+  // nb: the neighbours (the cell itself for a missing one), bey: those beyond
+  // (order 1 reads only their bed)
+  Cell nb[4], bey[4];
+  T nb_wl[4];
+#pragma unroll
   for (int d = 0; d < 4; ++d) {
-    const int32_t rid = index[(int64_t)(d + 1) * N + i];
-    const int32_t lid = index[(int64_t)(((d + 2) & 3) + 1) * N + i];
-    FrameCell<T> c;
-    c.h = h[i]; c.qn = rot_n(qx[i], qy[i], d); c.qt = rot_t(qx[i], qy[i], d); c.z = z[i] - zref;
-    const T c_wl = wl[i] - zref;
-    EdgeOut<T> o;
-    if (rid == -1) {
-      int type, id;
-      decode_code(code, type, id);
-      const T bd = c_series_at(gd, gd_rows, gd_w, c_series_row(gd, gd_rows, gd_w, t), id + 1);
-      const T bw = c_series_at(gwl, gwl_rows, gwl_w, c_series_row(gwl, gwl_rows, gwl_w, t), id + 1) - zref;
-      const int rq = c_series_row(gq, gq_rows, gq_w, t);
-      const T bqx = c_series_at(gq, gq_rows, gq_w, rq, 1 + 2 * id);
-      const T bqy = c_series_at(gq, gq_rows, gq_w, rq, 2 + 2 * id);
-      const FrameCell<T> g = bc_ghost<T>(type, c, d, bd, bw, bqx, bqy);
-      const T etaC = ORDER == 1 ? c.h + c.z : c_wl;
-      const T etaR = ORDER == 1 ? g.h + g.z : ghost_wl<T>(type, c_wl, g, bw);
-      o = solve_edge<T, ORDER>(c, c, g, g, true, etaC, etaR, dx, dt, dt_dx);
-    } else {
-      const int32_t rrid = index[(int64_t)(d + 1) * N + rid];
-      FrameCell<T> r, l, rr;
-      r.h = h[rid]; r.qn = rot_n(qx[rid], qy[rid], d); r.qt = rot_t(qx[rid], qy[rid], d); r.z = z[rid] - zref;
-      if (lid == -1) {
-        l = c;
-      } else {
-        l.h = h[lid]; l.qn = rot_n(qx[lid], qy[lid], d); l.qt = rot_t(qx[lid], qy[lid], d); l.z = z[lid] - zref;
-      }
-      if (rrid == -1) {
-        rr = r;
-      } else {
-        rr.h = h[rrid]; rr.qn = rot_n(qx[rrid], qy[rrid], d); rr.qt = rot_t(qx[rrid], qy[rrid], d);
-        rr.z = z[rrid] - zref;
-      }
-      const T etaC = ORDER == 1 ? c.h + c.z : c_wl;
-      const T etaR = ORDER == 1 ? r.h + r.z : wl[rid] - zref;
-      o = solve_edge<T, ORDER>(c, l, r, rr, false, etaC, etaR, dx, dt, dt_dx);
+    const int32_t j = rid[d] < 0 ? i : rid[d];
+    rrid[d] = index[(int64_t)(d + 1) * N + j];
+    nb[d] = Cell{h[j], qx[j], qy[j], z[j]};
+    nb_wl[d] = ORDER == 1 ? T(0) : wl[j];
+  }
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int32_t k = rid[d] < 0 ? i : (rrid[d] < 0 ? rid[d] : rrid[d]);
+    bey[d].z = z[k];
+    bey[d].h = ORDER == 1 ? T(0) : h[k];
+    bey[d].qx = ORDER == 1 ? T(0) : qx[k];
+    bey[d].qy = ORDER == 1 ? T(0) : qy[k];
+  }
+  const T zref = Prec<T>::local_datum ? self.z : T(0);
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    auto frame = [&](const Cell& s) {
+      return FrameCell<T>{s.h, rot_n(s.qx, s.qy, d), rot_t(s.qx, s.qy, d), s.z - zref};
+    };
+    const FrameCell<T> c = frame(self);
+    const T c_wl = self_wl - zref;
+    const bool ghost = rid[d] == -1;
+    FrameCell<T> l = frame(nb[(d + 2) & 3]), r = frame(nb[d]), rr = frame(bey[d]);
+    T etaR = ORDER == 1 ? r.h + r.z : nb_wl[d] - zref;
+    if (ghost) {
+      l = c;
+      r = rr = c_ghost<T, ORDER>(code, c, d, c_wl, zref, t, gd, gd_rows, gd_w, gwl, gwl_rows, gwl_w, gq, gq_rows, gq_w,
+                                 etaR);
     }
+    const T etaC = ORDER == 1 ? c.h + c.z : c_wl;
+    const EdgeOut<T> o = solve_edge<T, ORDER>(c, l, r, rr, ghost, etaC, etaR, dx, dt, dt_dx);
     if (!o.active) continue;
     T gx, gy;
     switch (d) {
