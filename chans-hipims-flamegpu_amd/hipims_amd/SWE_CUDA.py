@@ -195,17 +195,24 @@ class Godunov:
         self.solver.update(mode, rain=rain)
 
     def _export_if_due(self):
-        if self._ctrl[4].item() > 0:
+        """Returns the clock (t, dt), read in the same transfer as the export
+        flag: a read of its own for each costs a step some 6 us apiece."""
+        t, dt, _, _, due = self._ctrl[:5].tolist()
+        if due > 0:
             self._ctrl[4] = 0.0
             # the reference exports before t += dt, naming the files t + dt,
             # which is the already advanced t here
-            self._export(self._time_tag(self.t.item()))
+            self._export(self._time_tag(t))
             print("give a output")
+        return t, dt
 
     def time_friction_euler_update_cuda(self, device):
         """Friction + update + time control (SWE_CUDA.py:780-831)."""
+        self._step_and_clock()
+
+    def _step_and_clock(self):
         self._run_update(_lib.HP_UPDATE_STEP)
-        self._export_if_due()
+        return self._export_if_due()
 
     def friction_euler_update_cuda(self):
         """Friction + update without time control (SWE_CUDA.py:766-778)."""

@@ -38,6 +38,8 @@ import msgpack
 import numpy as np
 import torch
 
+from .SWE_CUDA import Godunov
+
 TIME_STEP = 120  # functions.c:47
 
 
@@ -68,9 +70,14 @@ class Simulation:
         num = self.numerical
         num.addFlux()
         num.addStation_PrecipitationSource(self.rainfallMatrix, self.device)
-        num.time_friction_euler_update_cuda(self.device)
-        self.dt_list.append(num.dt.item())
-        self.t_list.append(num.t.item())
+        step = num.time_friction_euler_update_cuda
+        if getattr(step, "__func__", None) is Godunov.time_friction_euler_update_cuda:
+            t, dt = num._step_and_clock()  # the same call, handing on the clock it read
+        else:
+            step(self.device)
+            dt, t = num.dt.item(), num.t.item()
+        self.dt_list.append(dt)
+        self.t_list.append(t)
         self.results = num.get_h()[self.idx_target]
 
     def time(self) -> float:
