@@ -796,12 +796,26 @@ __global__ __launch_bounds__(kWalkLanes, walk_waves<T>()) void k_walk(hp_grid_de
 }
 
 // Every unit of every domain of an ensemble; map[i] = (domain, unit), domain
-// by domain, so a domain's partial records are one contiguous range.
+// by domain, so a domain's partial records are one contiguous range
+// (ranges[domain] = first, count).
+// With fold.st set (one state per domain) the time control of every domain is
+// folded, as in k_walk, and with prev set the grid begins with the sum blocks
+// of every domain.
 template <class T, int ORDER, bool FUSED>
 __global__ __launch_bounds__(kWalkLanes, walk_waves<T>()) void k_walk_multi(const hp_grid_desc* __restrict__ doms,
                                                            const int2* __restrict__ map, void* parts, int n_total,
-                                                           int rows) {
-  const int slot = xcd_band(blockIdx.x, gridDim.x);
+                                                           int rows, WalkFold fold, const Sums* prev,
+                                                           const int2* __restrict__ ranges) {
+  const int extra = (int)gridDim.x - n_total;
+  if (FUSED && (int)blockIdx.x < extra) {
+    const int d = (int)blockIdx.x / kFoldSumBlocks;
+    const hp_grid_desc& g = doms[d];
+    if (g.mass_sums)
+      fold_sums_block(g.ctrl, fold.st + d, fold.k, (int)blockIdx.x - d * kFoldSumBlocks, prev + ranges[d].x,
+                      ranges[d].y, g.dx);
+    return;
+  }
+  const int slot = xcd_band((int)blockIdx.x - extra, n_total);
   // (the map entry is the same for the whole wave)
   const int dom = __builtin_amdgcn_readfirstlane(map[slot].x), unit = __builtin_amdgcn_readfirstlane(map[slot].y);
   // the descriptor array is read-only for the launch: read it as constant
@@ -810,7 +824,7 @@ __global__ __launch_bounds__(kWalkLanes, walk_waves<T>()) void k_walk_multi(cons
   const int nstrips = (a->nx + kWalkOwn - 1) / kWalkOwn;
   const int by = uniform(unit / nstrips);
   walk_unit<T, ORDER, FUSED>(a, unit - by * nstrips, by, rows, Partials(parts, n_total), slot, false, true, false,
-                             WalkFold{nullptr, 0, nullptr}, false,
+                             WalkFold{fold.st ? fold.st + dom : nullptr, fold.k, fold.records}, unit == 0,
                              (int)blockIdx.x >= (int)gridDim.x - walk_slots<T>());
 }
 

@@ -145,7 +145,7 @@ typedef struct hp_grid_desc {
   int32_t cell0_x, cell0_y; /* first valid cell in row-major order (-1: none) */
   int32_t n_classes;        /* entries of manning */
   int32_t rain_mode;        /* hp_rain_mode */
-  int32_t tile_rows;        /* flux unit height: float 2, 4, 6, 8, 10, 12 or 16, double 4 or 8 (other: chosen by size) */
+  int32_t tile_rows;        /* flux unit height: float 2, 4, 6, 8, 10, 12 or 16, double 4 or 8 (other: chosen by size, 1 to 32) */
   int32_t mass_sums;        /* 1: keep hp_ctrl's FP64 volume / rain / boundary-flux sums up to
                                date (diagnostics the reference does not compute); 0: skip them */
   /* state planes (dtype) */
@@ -219,7 +219,7 @@ int hp_grid_step_fused(const hp_grid_desc* g, int32_t nsteps, void* stream);
 /* Allocation-free form of hp_grid_step_fused (no reference counterpart):
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The same
- * kernels, with the per-tile partial records in a library-owned device
+ * kernels, with the per-unit partial records in a library-owned device
  * array of hp_grid_noalloc_max_bytes() bytes (8 MiB, held per GPU until the
  * process ends) instead of g->work, which is ignored.  A domain needing more
  * (over about 200 000 flux units; 8192 x 8192 float cells fit at the
@@ -261,7 +261,7 @@ typedef struct hp_ensemble {
   const void* update_map;   /* device int32[2 * n_update_blocks]       */
   const void* finalize_map; /* device int32[2 * n_domains]             */
   void* partials;           /* device reduction records                */
-  int32_t single_pass;      /* 1: one single-pass launch per step      */
+  int32_t single_pass;      /* not 0: one single-pass launch per step  */
   const void* fused_finalize_map; /* device int32[2 * n_domains]       */
 } hp_ensemble;
 
@@ -271,13 +271,15 @@ int64_t hp_ensemble_workspace_bytes(int32_t n, const hp_grid_desc* descs);
  * synchronises `stream`) and fill the handle.  The domains' planes must stay
  * allocated while the handle is used.  single_pass 1: every domain needs
  * h_out, qx_out, qy_out, and each step is one single-pass launch over every
- * tile of every domain, alternating the two sets of planes. */
+ * unit of every domain, alternating the two sets of planes. */
 int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, void* work, int64_t work_bytes,
                      hp_ensemble* out, void* stream);
 /* nsteps x (flux of every domain, update of every domain, per-domain time
- * control): three launches per step; single-pass: two (step of every domain,
- * per-domain time control), and nsteps must be even so that the state ends
- * in the domains' own planes.  Graph-capturable. */
+ * control): three launches per step; single-pass: one (the time control of a
+ * step runs inside the next one's launch, with a launch before the first and
+ * after the last), in calls of two steps two (step of every domain, per-domain
+ * time control), and nsteps must be even so that the state ends in the
+ * domains' own planes.  Graph-capturable. */
 int hp_ensemble_step(const hp_ensemble* e, int32_t nsteps, void* stream);
 
 /* ---- Adjoint of one step with a frozen time-step schedule (no reference
