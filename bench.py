@@ -43,9 +43,10 @@ def alg_bytes(esize: int, rain_field: bool) -> dict:
 
 
 def kernel_names(esize: int) -> dict:
-    """The kernel behind each pass: float domains run both the flux pass and
-    the single-pass step as column-walk kernels (k_walk, its flux-pass and
-    step instances), double domains the LDS-tile kernels."""
+    """Names of the passes' kernels in the line and in the profiles/ file
+    names.  Both the flux pass and the single-pass step are instances of the
+    column walk (k_walk) in either precision; the double ones keep the names
+    of the passes."""
     if esize == 4:
         return {"k_flux": "k_walk_flux", "k_update": "k_update", "k_step_fused": "k_walk_step"}
     return {"k_flux": "k_flux", "k_update": "k_update", "k_step_fused": "k_step_fused"}
@@ -199,7 +200,7 @@ def parse():
                         "random rain field (mean 30, std 10 mm/h)")
     p.add_argument("--dtype", choices=["fp32", "fp64"], default="fp32")
     p.add_argument("--order", type=int, choices=[1, 2], default=2)
-    p.add_argument("--tile-rows", type=int, default=0, help="flux tile height (0: the fastest of the legal heights, timed per step path)")
+    p.add_argument("--tile-rows", type=int, default=0, help="flux unit height (0: the fastest of the tuner's choices, timed per step path)")
     p.add_argument("--mass-sums", action="store_true",
                    help="also keep the FP64 volume / rain / boundary-flux sums each step (diagnostics the "
                         "reference step does not compute)")
@@ -517,7 +518,7 @@ def run_adjoint(a, fp64=True):
         s.set_station_rain(c.rain_table)
         return s
 
-    # one tile height for the plain and the calibration runs: the fastest
+    # one unit height for the plain and the calibration runs: the fastest
     # single-pass one on this domain
     from hipims_amd import autotune
     rows = autotune.tune(solver(), path="fused", apply=False)
@@ -669,8 +670,8 @@ def main():
 
     g.step(a.warmup)
     torch.cuda.synchronize()
-    # Tile height per path: the fixed --tile-rows, or the fastest legal one
-    # timed on this domain (the tuner restores the state it steps).
+    # Unit height per path: the fixed --tile-rows, or the fastest of the tuner's
+    # choices timed on this domain (the tuner restores the state it steps).
     rows, tuned = {}, {}
     for path in ("flux", "fused"):
         if a.tile_rows:

@@ -1,17 +1,17 @@
 """Flux unit-height autotuner.
 
-Float domains run the flux pass and the single-pass step as column walks:
-one wave per unit of 60 columns x R rows, R in {2, 4, 6, 8, 10, 12, 16}.  A taller
-unit re-loads fewer halo rows and solves fewer duplicate y-edges (four
-prologue rows and one edge per unit), a shorter one gives more waves, which
-matters when the last round of waves on the 256 CUs would run part-empty.
-Double domains stage 64 x TY cells plus a 2-cell halo in LDS, TY in {4, 8}: a
-taller tile solves fewer halo edges but holds more LDS per block.  Which
-wins depends on dtype, order, domain size and on the step path.  tune() times
-each legal height on the caller's own domain with HIP events - the flux pass
-alone, or whole single-pass steps - restores the domain's state afterwards
-and keeps the fastest; results are memoised per (dtype, order, size class,
-path) for the process.
+The flux pass and the single-pass step run as column walks: one wave per unit
+of 60 columns x R rows.  A taller unit re-loads fewer halo rows and solves
+fewer duplicate y-edges (four prologue rows and one edge per unit), a shorter
+one gives more waves.  Height 0 leaves the choice to the library, which takes
+any height up to 32 by the domain's size so that the units fill whole rounds
+of the GPU's wave slots (2048^2 in float: 59 us a step, against 62 at the best
+fixed height); the other choices are fixed heights, R in {2, 4, 6, 8, 10, 12,
+16} in float and {4, 8} in double.  Which wins depends on dtype, order, domain
+and on the step path.  tune() times each on the caller's own domain with HIP
+events - the flux pass alone, or whole single-pass steps - restores the
+domain's state afterwards and keeps the fastest; results are memoised per
+(dtype, order, size class, path) for the process.
 """
 from __future__ import annotations
 
@@ -19,7 +19,7 @@ import torch
 
 from .grid import GridSolver
 
-CHOICES = {torch.float32: (2, 4, 6, 8, 10, 12, 16), torch.float64: (4, 8)}
+CHOICES = {torch.float32: (0, 2, 4, 6, 8, 10, 12, 16), torch.float64: (0, 4, 8)}
 _cache: dict = {}
 
 
@@ -41,7 +41,7 @@ def _time(s: GridSolver, path: str, reps: int) -> float:
 
 
 def tune(s: GridSolver, reps: int = 20, apply: bool = True, path: str = "flux") -> int:
-    """Best tile height for `path` ("flux": the two-pass flux pass,
+    """Best unit height for `path` ("flux": the two-pass flux pass,
     "fused": the single-pass step) on this domain."""
     if path not in ("flux", "fused"):
         raise ValueError("path must be 'flux' or 'fused'")
@@ -88,7 +88,7 @@ def tune_ensemble(solvers: list[GridSolver], single_pass: bool = True, steps: in
     saved = [(s.U.clone(), s.h_max.clone(), s.ctrl.clone()) for s in solvers] if restore else []
     timings = {}
     for ty in CHOICES[dt]:
-        if max_rows is not None and ty > max_rows and ty != min(CHOICES[dt]):
+        if max_rows is not None and ty > max_rows:
             continue
         for s in solvers:
             s.set_tile_rows(ty)
