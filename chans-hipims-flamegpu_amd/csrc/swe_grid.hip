@@ -978,11 +978,10 @@ static int launch_update(const hp_grid_desc* g, int mode, hipStream_t st) {
 // Workspace of an ensemble: the descriptors twice (the second copy with the
 // two sets of state planes exchanged, for the odd steps of the single-pass
 // step), the (domain, unit) and (domain, chunk) maps, the per-domain ranges of
-// partial records for the two-pass and the single-pass step, the records; then,
-// where the workspace has room (fold_total), the folded time control's states
-// and its two arrays of sum records.
+// partial records for the two-pass and the single-pass step, the records, the
+// folded time control's states and its two arrays of sum records.
 struct EnsembleLayout {
-  int64_t off_doms, off_fmap, off_umap, off_fin, off_fin1, off_parts, total, fold_total;
+  int64_t off_doms, off_fmap, off_umap, off_fin, off_fin1, off_parts, total;
   int64_t n_ftiles, n_ublocks;
 };
 static int64_t ensemble_parts_bytes(int64_t n_ftiles, int64_t n_ublocks) {
@@ -1013,8 +1012,8 @@ static EnsembleLayout ensemble_layout(int32_t n, const hp_grid_desc* d) {
   L.off_fin = L.off_umap + align256(L.n_ublocks * 8);
   L.off_fin1 = L.off_fin + align256((int64_t)n * 8);
   L.off_parts = L.off_fin1 + align256((int64_t)n * 8);
-  L.total = L.off_parts + ensemble_parts_bytes(L.n_ftiles, L.n_ublocks);
-  L.fold_total = L.total + align256((int64_t)n * (int64_t)sizeof(FoldState)) + 2 * L.n_ftiles * (int64_t)sizeof(Sums);
+  L.total = L.off_parts + ensemble_parts_bytes(L.n_ftiles, L.n_ublocks) +
+            align256((int64_t)n * (int64_t)sizeof(FoldState)) + 2 * L.n_ftiles * (int64_t)sizeof(Sums);
   return L;
 }
 
@@ -1375,7 +1374,7 @@ int hp_grid_step(const hp_grid_desc* g, int32_t nsteps, void* stream) {
 
 int64_t hp_ensemble_workspace_bytes(int32_t n, const hp_grid_desc* descs) {
   if (n <= 0 || !descs) return 0;
-  return ensemble_layout(n, descs).fold_total;
+  return ensemble_layout(n, descs).total;
 }
 
 int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, void* work, int64_t work_bytes,
@@ -1443,7 +1442,7 @@ int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, 
   out->single_pass = single_pass;
   if (single_pass) {
     // (a negative CFL number would give negative minima, whose bits do not order)
-    bool fold = work_bytes >= L.fold_total, sums = false;
+    bool fold = true, sums = false;
     for (int k = 0; k < n; ++k) {
       fold = fold && descs[k].cfl >= 0.0;
       sums = sums || descs[k].mass_sums != 0;

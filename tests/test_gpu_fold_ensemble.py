@@ -51,21 +51,3 @@ def test_folded_call_under_graph_replay(cuda):
         for s in a + b:  # the host writes the state between replays
             s.h *= 1.001
             s.state_written()
-
-
-def test_workspace_without_room_for_the_fold(cuda):
-    """The records alone suffice: the time control then keeps its launches."""
-    import ctypes
-
-    from hipims_amd import _lib
-    a, b = domains(torch.float64), domains(torch.float64)
-    ea, eb = Ensemble(a), Ensemble(b)
-    need = ea.work.numel()
-    h = type(ea.handle)()
-    rc = _lib.lib().hp_ensemble_init(len(a), ea._descs, 1, ea.work.data_ptr(), need - 1, ctypes.byref(h),
-                                     _lib.stream_ptr(ea.device))
-    assert rc == 0 and h.single_pass & 2 == 0 and eb.handle.single_pass & 2
-    ea.handle = h
-    ea.step(6)
-    eb.step(6)
-    same(a, b, "small workspace")
