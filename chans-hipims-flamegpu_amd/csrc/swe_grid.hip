@@ -777,25 +777,28 @@ static int64_t units(const hp_grid_desc* g, int cols, int rows) {
 // a row, five in float and three in double fill the SIMD), after start[n - 1]
 // for their prologues.  More units than fit at once go in rounds; up to four
 // of them, a last round that is nearly empty takes as long as a full one, and
-// tall units spread uneven rows (dry ones, nodata) worse, by 0.25 % a row; the
-// dispatcher begins a second round some 5 % before every slot is taken.  Over
-// many rounds only the prologues and a short tail count.  Measured, float,
-// order 2, height: us (units per SIMD): 256^2 1: 10.1 (1.3), 2: 10.6 (0.6);
-// 500^2 1: 20.1 (4.4), 2: 16.4 (2.2), 3: 15.4 (1.5), 5: 17.2 (0.9); 1024^2
-// 3: 33.6 (6.0), 4: 28.4 (4.5), 5: 27.0 (3.6), 8: 28.4 (2.3); 2048^2 8: 63.2
-// (8.8), 13: 67.4 (5.4), 15: 59.0 (4.7), 18: 61.6 (3.9), 24: 68.8 (2.9);
-// 3000^2 15: 119 (9.8), 30: 141 (4.9), 31: 122 (4.7), with a flood in
-// a dry plain, order 1, 15: 102, 28: 123, 32: 119; 8192^2 8: 814, 16: 752, 24: 744,
-// 32: 737; double, order 2: 256^2 1: 12.7 (1.3), 2: 13.8 (0.6); 700^2 2: 33.0
-// (4.1), 3: 27.3 (2.7), 5: 29.1 (1.6), 8: 41.3 (1.0); 2048^2 8: 145 (8.8),
-// 14: 158 (5.0), 24: 141 (2.9).
+// tall units spread uneven rows (dry ones, nodata) worse, by 0.25 % a row.
+// The dispatcher begins a second round some 5 % before every slot is taken
+// (in double 2 %: 928^2 8 rows in two rounds 45, 5 in one of 97 % 40; kept at
+// 5 for tall units, which lose more to uneven rows than they gain).  Over many
+// rounds only the prologues and a short tail count.  Measured, order 2, height:
+// us (units per SIMD): float 256^2 1: 10.1 (1.3), 2: 10.6 (0.6); 500^2 1: 20.1
+// (4.4), 2: 16.4 (2.2), 3: 15.4 (1.5), 5: 17.2 (0.9); 1024^2 3: 33.6 (6.0),
+// 4: 28.4 (4.5), 5: 27.0 (3.6), 8: 28.4 (2.3); 2048^2 8: 63.2 (8.8), 13: 67.4
+// (5.4), 15: 59.0 (4.7), 18: 61.6 (3.9), 24: 68.8 (2.9); 3000^2 15: 119 (9.8),
+// 30: 141 (4.9), 31: 122 (4.7), with a flood in a dry plain, order 1, 15: 102,
+// 28: 123, 32: 119; 8192^2 8: 814, 16: 752, 24: 744, 32: 737; double 256^2
+// 1: 12.7 (1.3), 2: 13.8 (0.6); 700^2 2: 33.0 (4.1), 3: 27.3 (2.7), 5: 29.1
+// (1.6), 8: 41.3 (1.0); 2048^2 8: 145 (8.8), 12: 143 (5.8), 14: 158 (5.0),
+// 24: 141 (2.9), with a flood in a dry plain 12: 126, 24: 136.
 template <class T> static double walk_cost(int64_t u, int r) {
   static const double kRowF[] = {2.05, 2.4, 2.45, 2.85, 3.0}, kStartF[] = {6.3, 8.0, 10.5, 12.0, 16.0};
   static const double kRowD[] = {3.35, 4.1, 5.25}, kStartD[] = {6.7, 8.6, 11.5};
   const double *row = sizeof(T) == 4 ? kRowF : kRowD, *start = sizeof(T) == 4 ? kStartF : kStartD;
   const double x = (double)u / walk_slots<T>();
   const bool many = x > 4.0;
-  const double rounds = many ? x + 0.25 : (double)(1 + (int)(x + (x > 1.0 ? 0.02 : 0.05)));
+  const double full = x <= 1.0 && (sizeof(T) == 4 || r > 12) ? 0.05 : 0.02;
+  const double rounds = many ? x + 0.25 : (double)(1 + (int)(x + full));
   const int i = (int)(rounds > 1.0 ? walk_waves<T>() : (u + kSimds - 1) / kSimds) - 1;
   return start[i] + rounds * row[i] * r * (many ? 1.0 : 1.0 + 0.0025 * r) + 5.0 * (rounds - 1.0);
 }
