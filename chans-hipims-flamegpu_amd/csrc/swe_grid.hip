@@ -1176,15 +1176,19 @@ static int64_t fold_need(const hp_grid_desc* g) {
   return align256(sizeof(FoldState)) + (g->mass_sums ? 2 * flux_tiles(g) * (int64_t)sizeof(Sums) : 0);
 }
 
-// The checks every single-pass entry point makes.
-static int check_fused(const hp_grid_desc* g) {
+// The checks every single-pass entry point makes (need: bytes that the
+// workspace must have at least).
+static int check_fused(const hp_grid_desc* g, int64_t (*need)(const hp_grid_desc*) = workspace_need) {
   int rc = check_desc(g);
   if (rc) return rc;
   if (!g->h_out || !g->qx_out || !g->qy_out) return fail(HP_EINVAL, "the fused step needs h_out, qx_out, qy_out");
-  if (!g->work || g->work_bytes < workspace_need(g))
+  if (!g->work || g->work_bytes < need(g))
     return fail(HP_ESPACE, "workspace smaller than hp_grid_workspace_bytes()");
   return HP_OK;
 }
+
+// The records that the single-pass step itself writes.
+static int64_t fused_records(const hp_grid_desc* g) { return partials_bytes(flux_tiles(g)); }
 
 // Calls of at least this many steps fold the time control into the step
 // kernel: begin and end are launches too, so below it nothing is saved.
@@ -1242,6 +1246,15 @@ static int copy_state_back(const hp_grid_desc* g, hipStream_t st) {
   return HP_OK;
 }
 
+// nsteps single-pass steps, the state in the caller's planes at the end.
+static int step_fused(const hp_grid_desc* g, int32_t nsteps, hipStream_t st) {
+  if (nsteps < 0) return fail(HP_EINVAL, "nsteps must be >= 0");
+  int rc = single_pass_steps(g, nsteps, st, [](int) {}, [](int) {});
+  if (rc) return rc;
+  if (nsteps & 1) return copy_state_back(g, st);
+  return HP_OK;
+}
+
 }  // namespace hp
 
 using namespace hp;
@@ -1256,12 +1269,7 @@ int64_t hp_grid_workspace_bytes(const hp_grid_desc* g) {
 int hp_grid_step_fused(const hp_grid_desc* g, int32_t nsteps, void* stream) {
   int rc = check_fused(g);
   if (rc) return rc;
-  if (nsteps < 0) return fail(HP_EINVAL, "nsteps must be >= 0");
-  hipStream_t st = (hipStream_t)stream;
-  rc = single_pass_steps(g, nsteps, st, [](int) {}, [](int) {});
-  if (rc) return rc;
-  if (nsteps & 1) return copy_state_back(g, st);
-  return HP_OK;
+  return step_fused(g, nsteps, (hipStream_t)stream);
 }
 
 int64_t hp_grid_noalloc_max_bytes(void) { return kScratchBytes; }
@@ -1281,8 +1289,10 @@ int hp_grid_step_fused_noalloc(const hp_grid_desc* g, int32_t nsteps, void* stre
   d.work_bytes = kScratchBytes;
   // (an asked height whose 60-column units have more records than its
   // nominal tiles gives way to the chosen one, which has fewer)
-  if (workspace_need(&d) > kScratchBytes) d.tile_rows = 0;
-  return hp_grid_step_fused(&d, nsteps, stream);
+  if (fused_records(&d) > kScratchBytes) d.tile_rows = 0;
+  rc = check_fused(&d, fused_records);
+  if (rc) return rc;
+  return step_fused(&d, nsteps, (hipStream_t)stream);
 }
 
 int hp_grid_step_fused_timed(const hp_grid_desc* g, int32_t nsteps, int32_t sample_every, float* kernel_ms,
