@@ -29,6 +29,7 @@
 #include <math.h>
 #include <stdint.h>
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <utility>
@@ -1190,6 +1191,10 @@ static int check_fused(const hp_grid_desc* g, int64_t (*need)(const hp_grid_desc
 // The records that the single-pass step itself writes.
 static int64_t fused_records(const hp_grid_desc* g) { return partials_bytes(flux_tiles(g)); }
 
+// Whether a domain's CFL minima may be folded by the bits of the doubles: a
+// negative CFL number, zero included, gives negative ones, which do not order.
+static bool ordered_minima(const hp_grid_desc* g) { return g->cfl >= 0.0 && !std::signbit(g->cfl); }
+
 // Calls of at least this many steps fold the time control into the step
 // kernel: begin and end are launches too, so below it nothing is saved.
 constexpr int kFoldSteps = 3;
@@ -1199,8 +1204,7 @@ constexpr int kFoldSteps = 3;
 template <class Before, class After>
 static int single_pass_steps(const hp_grid_desc* g, int32_t nsteps, hipStream_t st, Before before, After after) {
   hp_grid_desc d = *g;
-  // (a negative CFL number would give negative minima, whose bits do not order)
-  const bool fold = nsteps >= kFoldSteps && g->cfl >= 0.0 && g->work_bytes >= fold_need(g);
+  const bool fold = nsteps >= kFoldSteps && ordered_minima(g) && g->work_bytes >= fold_need(g);
   FoldState* fs = fold ? (FoldState*)g->work : nullptr;
   const int64_t n = flux_tiles(g);
   Sums* rec = fold && g->mass_sums ? (Sums*)((char*)g->work + align256(sizeof(FoldState))) : nullptr;
@@ -1454,10 +1458,9 @@ int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, 
   out->partials = w + L.off_parts;
   out->single_pass = single_pass;
   if (single_pass) {
-    // (a negative CFL number would give negative minima, whose bits do not order)
     bool fold = true, sums = false;
     for (int k = 0; k < n; ++k) {
-      fold = fold && descs[k].cfl >= 0.0;
+      fold = fold && ordered_minima(&descs[k]);
       sums = sums || descs[k].mass_sums != 0;
     }
     out->single_pass |= (fold ? kEnsembleFold : 0) | (sums ? kEnsembleSums : 0);
