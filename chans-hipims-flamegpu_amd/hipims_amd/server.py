@@ -70,15 +70,22 @@ class Simulation:
         num = self.numerical
         num.addFlux()
         num.addStation_PrecipitationSource(self.rainfallMatrix, self.device)
-        step = num.time_friction_euler_update_cuda
-        if getattr(step, "__func__", None) is Godunov.time_friction_euler_update_cuda:
+        if self._library_step(num):
             t, dt = num._step_and_clock()  # the same call, handing on the clock it read
         else:
-            step(self.device)
+            num.time_friction_euler_update_cuda(self.device)
             dt, t = num.dt.item(), num.t.item()
         self.dt_list.append(dt)
         self.t_list.append(t)
         self.results = num.get_h()[self.idx_target]
+
+    @staticmethod
+    def _library_step(num) -> bool:
+        """Whether the model's step, its export hook and its clock are the
+        library's own: one that replaces any of them is asked for its clock."""
+        return (all(getattr(getattr(num, m, None), "__func__", None) is getattr(Godunov, m)
+                    for m in ("time_friction_euler_update_cuda", "_step_and_clock", "_export_if_due"))
+                and all(getattr(type(num), c, None) is getattr(Godunov, c) for c in ("t", "dt")))
 
     def time(self) -> float:
         return self.numerical.t.item()
