@@ -424,9 +424,11 @@ __global__ __launch_bounds__(kThreads) void k_infiltration(hp_grid_desc a) {
 // chain of loads, divisions and square roots, so a thread has one element
 // (with eight, in vectors of four, a 75x75 domain in double took 13.2 us and
 // takes 5.6).  Past 1024 blocks the elements per thread grow to eight, so that
-// one block can fold the records: one at a time in double (2048^2 with the
-// time control: 75 -> 68 us), in vectors of four in float, which moves half
-// the bytes per access (3000^2: 74 us one at a time, 69 in vectors).
+// one block can fold the records; from four on they come in accesses of 16
+// bytes.  Kernel time with one, two and four elements per access, us: double
+// 800^2 17.3, 16.6, -, 2048^2 71, 66, 72, 3000^2 147, 145, 147; float 800^2
+// 11.6, -, 11.4, 2048^2 35, 33, 33, 3000^2 72, 67, 64.  (One kernel for vectors
+// and single elements cost a 1024^2 float domain a sixth.)
 __host__ __device__ inline int update_loops(int64_t total) {
   int n = 1;
   while (n < 8 && total > (int64_t)n * kThreads * 1024) n *= 2;
@@ -461,15 +463,13 @@ template <class T, int MODE, int W>
 __device__ inline void update_elements(const hp_grid_desc& a, int64_t base, int rounds, int64_t total,
                                        const Partials& part, int64_t pidx, T* s_man, T* s_rate) {
   const int tid = threadIdx.x, mode = a.rain_mode;
-  // (past the end: the last elements again, with the class of no cell)
+  // (past the end: the last elements again, which the loop below leaves out.  A
+  // class of no cell put in here instead would have every load wait for the
+  // classes: 3000^2 in float 64 -> 65 us.)
   auto load = [&](int it) {
     const int64_t at = base + ((int64_t)it * kThreads + tid) * W, i = at < total ? at : total - W;
     UpdateIn<T, W> c{};
     load_w(c.cls, a.landuse + i);
-    if (at >= total) {
-#pragma unroll
-      for (int j = 0; j < W; ++j) c.cls[j] = 255;
-    }
     load_w(c.h, (const T*)a.h + i);
     load_w(c.qx, (const T*)a.qx + i);
     load_w(c.qy, (const T*)a.qy + i);
@@ -484,17 +484,25 @@ __device__ inline void update_elements(const hp_grid_desc& a, int64_t base, int 
     }
     return c;
   };
-  UpdateIn<T, W> c = load(0);  // before the tables, whose round trips it overlaps
+  // Single elements are asked for before the tables, whose round trips they
+  // overlap; vectors after them, where a launch is bound by memory and the
+  // tables, behind them in order, would wait for megabytes (float 1024^2 13.4
+  // us the other way round, 13.0 so; double 2048^2 65.3, 63.6).
+  UpdateIn<T, W> c{};
+  if (W == 1) c = load(0);
+  const double times = wave_rain_times(&a);
+  const T man = tid < a.n_classes ? ((const T*)a.manning)[tid] : T(0);
   if (stopped(a.ctrl)) {
     if (tid == 0) part.put(pidx, INFINITY, 0.0, 0.0, 0.0, a.mass_sums != 0);
     return;
   }
   const T dt = T(a.ctrl->dt);
   const T cfl_dx = T(a.cfl) * T(a.dx), rscale = T(a.rain_scale);
-  for (int k = tid; k < a.n_classes; k += kThreads) s_man[k] = ((const T*)a.manning)[k];
-  const RainRows rr = wave_rain_rows(&a, a.ctrl->t);
+  if (tid < a.n_classes) s_man[tid] = man;
+  const RainRows rr = wave_rain_rows(&a, a.ctrl->t, times);
   if (mode == HP_RAIN_STATION && tid < kRateCache) s_rate[tid] = station_rate<T>(rr, tid, a.rain_scale);
   __syncthreads();
+  if (W != 1) c = load(0);
   const bool sums = a.mass_sums != 0;
   T mn = T(INFINITY);
   double vol = 0.0, fsum = 0.0, rsum = 0.0;
@@ -503,9 +511,22 @@ __device__ inline void update_elements(const hp_grid_desc& a, int64_t base, int 
     UpdateIn<T, W> next{};
     if (W == 1 && more) next = load(it + 1);  // (vectors ahead would halve the waves in flight)
     const int64_t i = base + ((int64_t)it * kThreads + tid) * W;
+    T rate[W] = {};
+    if (MODE != HP_UPDATE_CFL) {
+      if (mode == HP_RAIN_STATION) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+          const int k = c.st[j];
+          rate[j] = (k >= 0 && k < kRateCache) ? s_rate[k] : station_rate<T>(rr, k, a.rain_scale);
+        }
+      } else if (mode == HP_RAIN_FIELD) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) rate[j] = T(c.rain[j]) * rscale;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < W; ++j) {
-      if (c.cls[j] == 255) continue;
+      if (either(c.cls[j] == 255, i >= total)) continue;
       T h = c.h[j];
       if (MODE == HP_UPDATE_CFL) {
         if (gt_hs(h)) {
@@ -513,14 +534,7 @@ __device__ inline void update_elements(const hp_grid_desc& a, int64_t base, int 
           mn = fmin(mn, cfl_candidate<T>(h, c.qx[j], c.qy[j], cfl_dx));
         }
       } else {
-        T rate = T(0);
-        if (mode == HP_RAIN_STATION) {
-          const int k = c.st[j];
-          rate = (k >= 0 && k < kRateCache) ? s_rate[k] : station_rate<T>(rr, k, a.rain_scale);
-        } else if (mode == HP_RAIN_FIELD) {
-          rate = T(c.rain[j]) * rscale;
-        }
-        const T rdt = rate * dt;
+        const T rdt = rate[j] * dt;
         const T dht = (c.dh[j] + rdt) - c.df[j];  // flux, + rain, - infiltration (the reference's order)
         const bool listed =
             (MODE == HP_UPDATE_EULER) ? (fabs(dht) > T(0) || gt_hs(h)) : (fabs(dht) > T(0) || h >= T(0));
@@ -561,9 +575,10 @@ __device__ inline void update_elements(const hp_grid_desc& a, int64_t base, int 
   block_partial<T>(mn, vol, fsum, rsum, part, pidx, sums);
 }
 
-// Elements per access of a domain's update.
+// Elements per access of a domain's update: one, or those of 16 bytes.
+template <class T> constexpr int kWide = 16 / sizeof(T);
 template <class T> __host__ __device__ inline int update_width(int64_t total) {
-  return sizeof(T) == 4 && update_loops(total) == 8 ? kVec : 1;
+  return update_loops(total) >= 4 ? kWide<T> : 1;
 }
 
 template <class T, int MODE, int W>
@@ -592,7 +607,7 @@ __global__ __launch_bounds__(kThreads) void k_update_multi(const hp_grid_desc* _
   const hp_grid_desc& a = doms[m.x];
   const Partials part(parts, gridDim.x);
   if (update_width<T>(a.pitch * (int64_t)a.ny) != 1)
-    update_chunk<T, MODE, kVec>(a, m.y, part, blockIdx.x, s_man, s_rate);
+    update_chunk<T, MODE, kWide<T>>(a, m.y, part, blockIdx.x, s_man, s_rate);
   else update_chunk<T, MODE, 1>(a, m.y, part, blockIdx.x, s_man, s_rate);
 }
 
@@ -949,12 +964,16 @@ static int launch_infiltration(const hp_grid_desc* g, hipStream_t st) {
   return check_launch("k_infiltration");
 }
 
+template <class T, int MODE>
+static void launch_update_t(const hp_grid_desc* g, int64_t nb, hipStream_t st) {
+  if (update_width<T>(g->pitch * (int64_t)g->ny) != 1)
+    hipLaunchKernelGGL((k_update<T, MODE, kWide<T>>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
+  else hipLaunchKernelGGL((k_update<T, MODE, 1>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
+}
+
 template <int MODE>
 static void launch_update_mode(const hp_grid_desc* g, int64_t nb, hipStream_t st) {
-  const bool wide = g->dtype == HP_F32 && update_width<float>(g->pitch * (int64_t)g->ny) != 1;
-  if (wide) hipLaunchKernelGGL((k_update<float, MODE, kVec>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
-  else if (g->dtype == HP_F32) hipLaunchKernelGGL((k_update<float, MODE, 1>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
-  else hipLaunchKernelGGL((k_update<double, MODE, 1>), dim3((unsigned)nb), dim3(kThreads), 0, st, *g);
+  (g->dtype == HP_F32 ? launch_update_t<float, MODE> : launch_update_t<double, MODE>)(g, nb, st);
 }
 
 static int launch_update(const hp_grid_desc* g, int mode, hipStream_t st) {
