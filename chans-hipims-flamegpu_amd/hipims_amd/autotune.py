@@ -28,10 +28,16 @@ def _key(s: GridSolver, path: str):
     return (s.dtype, s.order, max(0, cells.bit_length() - 18), path)
 
 
+# The clocks rise over the first tens of milliseconds of work, by more than the
+# heights differ: so long the tuner warms up, or for as many calls as it times.
+WARM_MS = 30.0
+
+
 def _time(s: GridSolver, path: str, reps: int) -> float:
-    # (calls of four steps: as in a run, the time control is folded in)
+    """ms per flux pass, or per call of four single-pass steps (as in a run,
+    such a call folds the time control in)."""
     run = (lambda: s.step_fused(4)) if path == "fused" else s.flux
-    run()  # warm-up (and the fused path's second buffers)
+    run()  # untimed: the fused path's second buffers
     a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     a.record()
     for _ in range(reps):
@@ -43,7 +49,9 @@ def _time(s: GridSolver, path: str, reps: int) -> float:
 
 def tune(s: GridSolver, reps: int = 20, apply: bool = True, path: str = "flux") -> int:
     """Best unit height for `path` ("flux": the two-pass flux pass,
-    "fused": the single-pass step) on this domain."""
+    "fused": the single-pass step) on this domain, 0 for the library's own
+    choice: each is timed over `reps` flux passes, or 2 * reps single-pass
+    steps in calls of four.  s.tune_timings holds the ms per pass or call."""
     if path not in ("flux", "fused"):
         raise ValueError("path must be 'flux' or 'fused'")
     key = _key(s, path)
@@ -53,19 +61,26 @@ def tune(s: GridSolver, reps: int = 20, apply: bool = True, path: str = "flux") 
         saved = [s.U.clone(), s.D.clone(), s.h_max.clone(), s.ctrl.clone(), None if s.F is None else s.F.clone()]
         saved_rows = s.tile_rows
         timings = {}
-        # three rounds, the first one untimed work for the clocks: they rise
-        # over the first tens of milliseconds, by more than the heights differ
-        for k, ty in ((k, ty) for k in range(3) for ty in CHOICES[s.dtype]):
-            s.set_tile_rows(ty)
-            ms = _time(s, path, reps)
-            if k > 0:
-                timings[ty] = min(ms, timings.get(ty, ms))
+        calls = max(1, reps // 2) if path == "fused" else reps
+
+        def timed():
+            ms = _time(s, path, calls)
             s.U.copy_(saved[0])
             s.D.copy_(saved[1])
             s.h_max.copy_(saved[2])
             s.ctrl.copy_(saved[3])
             if saved[4] is not None:
                 s.F.copy_(saved[4])
+            return ms
+
+        warm = 0.0
+        for _ in CHOICES[s.dtype]:
+            warm += timed() * calls
+            if warm >= WARM_MS:
+                break
+        for ty in CHOICES[s.dtype]:
+            s.set_tile_rows(ty)
+            timings[ty] = timed()
         s.set_tile_rows(saved_rows)
         best = min(timings, key=timings.get)
         _cache[key] = best
@@ -78,8 +93,9 @@ def tune(s: GridSolver, reps: int = 20, apply: bool = True, path: str = "flux") 
 def tune_ensemble(solvers: list[GridSolver], single_pass: bool = True, steps: int = 10,
                   max_rows: int | None = None, restore: bool = True) -> int:
     """Best unit height for one ensemble launch over `solvers` (all must share
-    dtype and order): each legal height (up to `max_rows` when given) is
-    timed over `steps` ensemble steps (after two untimed ones).  With
+    dtype and order): each legal height (up to `max_rows` when given) and the
+    library's own choice (0, of any height) is timed over `steps` ensemble
+    steps (after two untimed ones).  With
     `restore` every domain's state is put back afterwards; without it the
     steps stand as the run's own (the states do not depend on the height),
     so a run that retunes on the way loses no work to it.  Sets the winner

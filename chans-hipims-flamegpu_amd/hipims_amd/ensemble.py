@@ -101,7 +101,7 @@ class Ensemble:
         ones and the graph is captured again.  At such a rebuild, once the
         active scenarios hold less than `retune_below` of the cells the unit
         height was last chosen for, the height is timed again over them
-        (autotune.tune_ensemble, heights up to the current one): the height
+        (autotune.tune_ensemble, fixed heights up to the current one): the height
         that fills the GPU with many domains leaves it idle with a few small
         ones; its timed steps count as the run's own.  The states do not
         depend on the height, only the FP64 mass sums' rounding does; 0
