@@ -4,10 +4,15 @@ The reference runs one domain per process and steps it from Python with
 several host synchronisations per step (SWE_CUDA.py:780-831).  Here every
 scenario keeps its own planes and device control block (its own dt, t, export
 clamp and stop time), and one set of launches advances all of them by one
-step each: by default two - the single-pass step of every tile of every
-scenario (alternating each scenario's two sets of state planes), time
-control of every scenario - or, with single_pass=False, three (flux of every
-tile, update of every chunk, time control).  K such steps are captured
+step each: by default one - the single-pass step of every unit of every
+scenario (alternating each scenario's two sets of state planes), which runs
+the time control of the step before; calls of two steps launch the time
+control separately - or, with single_pass=False, three (flux of every
+unit, update of every chunk, time control).  Every scenario's state, h_max, t
+and dt are bitwise those of a run of its own; the FP64 mass sums are where the
+unit height is the same (where set_tile_rows asks for one, always; else an
+ensemble may choose another than a domain alone, and the sums add the same
+terms in another order).  K such steps are captured
 once in a HIP graph and replayed; a scenario that has reached its stop time is
 skipped by every pass, so the ensemble runs until the slowest scenario is done
 with one host check per replay.
@@ -96,7 +101,7 @@ class Ensemble:
             progress=None, retune_below: float = 0.25) -> int:
         """Replay the captured graph until every scenario has stopped; returns
         the number of replays.  Stopped scenarios cost a launched-and-exiting
-        block per tile, so once the active count falls to `compact` of the
+        block per unit, so once the active count falls to `compact` of the
         scenarios in the launch maps, the maps are rebuilt over the active
         ones and the graph is captured again.  At such a rebuild, once the
         active scenarios hold less than `retune_below` of the cells the unit

@@ -279,7 +279,11 @@ int hp_ensemble_init(int32_t n, const hp_grid_desc* descs, int32_t single_pass, 
  * step runs inside the next one's launch, with a launch before the first and
  * after the last), in calls of two steps two (step of every domain, per-domain
  * time control), and nsteps must be even so that the state ends in the
- * domains' own planes.  Graph-capturable. */
+ * domains' own planes.  Graph-capturable.  State, h_max, t and dt of a domain
+ * are bitwise those of the same steps on the domain alone; its mass sums are
+ * too where tile_rows asks for a height (where it does not, an ensemble may
+ * choose another height than the domain alone, and the single-pass step's sums
+ * then add the same terms in another order). */
 int hp_ensemble_step(const hp_ensemble* e, int32_t nsteps, void* stream);
 
 /* ---- Adjoint of one step with a frozen time-step schedule (no reference
