@@ -267,9 +267,10 @@ __global__ __launch_bounds__(kAThreads) void k_adj_update(hp_grid_desc a, AdjPla
 }
 
 // grads[b][c] (c < 15) = sum of gn over block b's cells of class c: the
-// per-class Manning gradients, folded once after the reverse sweep.
+// per-class Manning gradients, folded once after the reverse sweep.  The rows
+// beyond the blocks (rows in all) take zeros.
 __global__ __launch_bounds__(kAThreads) void k_adj_finish(hp_grid_desc a, const double* __restrict__ gn,
-                                                          double* grads) {
+                                                          double* grads, int64_t rows) {
   __shared__ double s_g[kAThreads / 64][kGradStride];
   const int tid = threadIdx.x;
   double acc[kGradStride - 1];
@@ -297,6 +298,7 @@ __global__ __launch_bounds__(kAThreads) void k_adj_finish(hp_grid_desc a, const 
     double v = 0.0;
     for (int k = 0; k < kAThreads / 64; ++k) v += s_g[k][tid];
     grads[(int64_t)blockIdx.x * kGradStride + tid] = v;
+    for (int64_t b = (int64_t)blockIdx.x + gridDim.x; b < rows; b += gridDim.x) grads[b * kGradStride + tid] = 0.0;
   }
 }
 
@@ -838,9 +840,9 @@ int hp_adjoint_step(const hp_grid_desc* g, const hp_adjoint_desc* ad, void* stre
 
 int hp_adjoint_finish(const hp_grid_desc* g, const hp_adjoint_desc* ad, void* stream) {
   if (!g || !ad || !ad->gn || !ad->grads || !g->landuse) return fail(HP_EINVAL, "null descriptor or plane");
-  const int64_t nb = hp_adjoint_grad_blocks(g);
+  const int64_t nb = (g->pitch * (int64_t)g->ny + kAChunk - 1) / kAChunk;
   hipLaunchKernelGGL(k_adj_finish, dim3((unsigned)nb), dim3(kAThreads), 0, (hipStream_t)stream, *g,
-                     (const double*)ad->gn, ad->grads);
+                     (const double*)ad->gn, ad->grads, hp_adjoint_grad_blocks(g));
   return check_launch("k_adj_finish");
 }
 
