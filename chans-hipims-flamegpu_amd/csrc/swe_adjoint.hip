@@ -58,17 +58,11 @@ __global__ void k_schedule_save(const hp_ctrl* ctrl, double* sched, int k) {
   }
 }
 
-// End of a calibration step: the gauge depths into their history row and,
-// when recording, (t, dt) of the next step (sched may be null).
+// End of a frozen run: the gauge depths into their history row.
 template <class T>
-__global__ void k_step_record(const T* __restrict__ h, const int64_t* __restrict__ off, int n, T* __restrict__ row,
-                              const hp_ctrl* ctrl, double* sched, int k_next) {
+__global__ void k_step_record(const T* __restrict__ h, const int64_t* __restrict__ off, int n, T* __restrict__ row) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) row[i] = h[off[i]];
-  if (sched && i == 0) {
-    sched[2 * (int64_t)k_next] = ctrl->t;
-    sched[2 * (int64_t)k_next + 1] = ctrl->dt;
-  }
 }
 
 template <class T> struct AdjPlanes {
@@ -953,13 +947,13 @@ int hp_calib_forward(const hp_grid_desc* g, double* sched, const hp_ctrl* frozen
                                 before)))
       return rc;
     if (frozen && gauges && j + 1 == nsteps) {
-      const unsigned nb = (unsigned)((n > 0 ? n : 1) + 255) / 256;
+      const unsigned nb = (unsigned)(n + 255) / 256;
       if (g->dtype == HP_F32)
         hipLaunchKernelGGL(k_step_record<float>, dim3(nb), dim3(256), 0, st, (const float*)out[0], gauge_off, n,
-                           (float*)row, g->ctrl, save, k + 1);
+                           (float*)row);
       else
         hipLaunchKernelGGL(k_step_record<double>, dim3(nb), dim3(256), 0, st, (const double*)out[0], gauge_off, n,
-                           (double*)row, g->ctrl, save, k + 1);
+                           (double*)row);
       if ((rc = check_launch("k_step_record"))) return rc;
     }
   }

@@ -51,13 +51,6 @@ __device__ inline bool stopped(const hp_ctrl* c) { return c->t_stop > 0.0 && c->
 
 // --- boundary series ------------------------------------------------------
 template <class T>
-__device__ inline int series_row(const T* tab, int rows, int w, T t) {
-  int r = 0;
-  while (r < rows - 1 && t > tab[r * w]) r++;
-  return r;
-}
-
-template <class T>
 __device__ inline T series_at(const T* tab, int rows, int w, int row, int col) {
   if (tab == nullptr || col < 0 || col >= w || row < 0 || row >= rows) return T(0);
   return tab[row * w + col];
@@ -67,16 +60,6 @@ template <class T> struct BcValues {
   int type;
   T gd, gwl, gqx, gqy;
 };
-
-// Global (qx, qy) of an edge-frame momentum flux (fn, ft) for direction d.
-template <class T> __device__ inline void to_global(T fn, T ft, int d, T& gx, T& gy) {
-  switch (d) {
-    case 0: gx = fn; gy = ft; break;
-    case 1: gx = -ft; gy = fn; break;
-    case 2: gx = -fn; gy = -ft; break;
-    default: gx = ft; gy = -fn; break;
-  }
-}
 
 // --- reductions ------------------------------------------------------------
 // The fields of a control block that a step advances, and those they depend on.
@@ -312,11 +295,9 @@ __device__ inline void block_partial(T mn, double vol, double fsum, double rsum,
 // Per-cell inputs of the update that do not depend on the fluxes; loaded
 // before the flux work so their latency hides behind it.
 template <class T> struct CellIn {
-  T rain;   // rain rate (m/s) of a field; of a station once resolved
-  int st;   // station index (station rain)
+  T rain;   // rain rate (m/s)
   T hmax;   // h_max before the step
   T n;      // Manning n of the cell's class
-  T F;      // cumulative infiltrated depth (when infiltration is on)
   int cls;  // landuse class
   bool on;  // landuse class != 255 (the reference's update covers the cell)
 };

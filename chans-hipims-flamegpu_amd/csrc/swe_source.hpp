@@ -1,4 +1,4 @@
-// Rain source terms and vector plane access shared by the step and its adjoint.
+// Rain source terms and the planes' alignment, shared by the step and its adjoint.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -8,28 +8,8 @@
 
 namespace hp {
 
-// Vector access to kVec consecutive plane elements (16 B in float).
+// Planes are aligned to this many elements, and rows hold a multiple of them.
 constexpr int kVec = 4;
-template <class T> struct alignas(sizeof(T) * kVec) VecT {
-  T x[kVec];
-};
-struct alignas(kVec) VecU8 {
-  uint8_t x[kVec];
-};
-struct alignas(2 * kVec) VecI16 {
-  int16_t x[kVec];
-};
-struct alignas(4 * kVec) VecI32 {
-  int32_t x[kVec];
-};
-struct alignas(4 * kVec) VecF32 {
-  float x[kVec];
-};
-struct alignas(8 * kVec) VecD {
-  double x[kVec];
-};
-template <class V, class T> __device__ inline V ldv(const T* p) { return *reinterpret_cast<const V*>(p); }
-template <class V, class T> __device__ inline void stv(T* p, const V& v) { *reinterpret_cast<V*>(p) = v; }
 
 // Station rain at time t_now (SWE_CUDA.py:472-495): linear in time between
 // the table rows that bracket t_now, 0 from the table's last row on, scaled

@@ -159,8 +159,8 @@ template <class T> struct WalkEnv {
   int n_classes;
 };
 
-// The row of a boundary series in force at t (as series_row), searched 64
-// rows at a time by the whole wave.
+// The row of a boundary series in force at t (the first whose time is not
+// before t, or the last), searched 64 rows at a time by the whole wave.
 template <class T> __device__ inline int wave_series_row(const void* tab, int rows, int w, T t) {
   if (tab == nullptr || rows <= 1) return 0;
   const T* p = (const T*)tab;
@@ -550,7 +550,7 @@ __device__ __forceinline__ void walk_row(const WalkEnv<T>& env, DP a, const Walk
       pl_st<T>(a->dqy, row, c, f.qy);
     }
     if (FUSED) {
-      CellIn<T> in{walk_rain<T>(env, a, wi, cx), 0, wi.hmax, env.s_man[min(wi.cls, env.n_classes - 1)], T(0), wi.cls,
+      CellIn<T> in{walk_rain<T>(env, a, wi, cx), wi.hmax, env.s_man[min(wi.cls, env.n_classes - 1)], wi.cls,
                    wi.cls != 255};
       T hn = cur.h, qxn = cur.qx, qyn = cur.qy, hm = in.hmax;
       T dF = T(0);
