@@ -15,7 +15,9 @@
 //           friction + update, h_max, the CFL minimum (wave64 shuffle + LDS),
 //           FP64 volume / flux / rain sums; one partial record per block.
 //   finalize one block per domain folds its partials and advances dt, t and
-//           the export clamp in the domain's control block (SWE_CUDA.py:818-831).
+//           the export clamp in the domain's control block (SWE_CUDA.py:818-831);
+//           calls of several single-pass steps do so inside the next step's
+//           launch instead (FoldState).
 // No host synchronisation anywhere in the step.
 //
 // Each pass is a device function over (domain, tile or chunk).  Single-domain
@@ -178,13 +180,14 @@ __device__ inline double wave_sum(double v) {
 // --- time control inside the step kernel --------------------------------
 // A call of several single-pass steps runs no time-control launch between
 // them (a launch costs 4 to 5 us whatever it does, and the gap before it 1 to
-// 2; a 2048^2 float step takes 62).  Each unit of step k posts its CFL minimum
+// 2; a 2048^2 float step takes 60).  Each unit of step k posts its CFL minimum
 // into one of kFoldSlots words by an atomic minimum (a non-negative double
 // orders like its bits, so the minimum does not depend on the order), and
 // every unit of step k + 1 folds the slots and advances the time control for
 // itself, from the control block of step k: one load per lane and one wave
 // reduction, in the shadow of the unit's first rows.  64 slots: at most one
-// load per lane, and 2048^2 posts 140 times to each at about 36 ns.
+// load per lane, and 2048^2 in units of 15 rows posts 75 times to each at about
+// 36 ns.
 // Step k posts to slots[k % 3], reads slots[(k - 1) % 3] and clears
 // slots[(k + 1) % 3]; its control block goes from ring[(k - 1) & 1] to
 // ring[k & 1], written by the unit 0.  Records of the FP64 sums take turns the
@@ -594,8 +597,8 @@ __global__ __launch_bounds__(kThreads) void k_update_multi(const hp_grid_desc* _
 
 // Fold a domain's partials in a fixed order and advance its time control.
 // The minima are read 24 per thread before any is used, so one block covers
-// 24 576 partials (a 2048^2 step's 17 920 four-row units) in one memory round
-// trip; the control block is read alongside them rather than ahead of them.
+// 24 576 partials (2048^2 has 4 795 units at its chosen 15 rows, 17 920 at an
+// asked height of four) in one memory round trip; the control block is read alongside them rather than ahead of them.
 // single_pass: the step just run was the single-pass one.  On a stopped
 // domain the time control records whether that step left the second set of
 // planes holding the state (the single-pass kernel copies it there on the
@@ -775,9 +778,15 @@ static int64_t units(const hp_grid_desc* g, int cols, int rows) {
 // for their prologues.  More units than fit at once go in rounds; up to four
 // of them, a last round that is nearly empty takes as long as a full one, and
 // tall units spread uneven rows (dry ones, nodata) worse, by 0.25 % a row.
-// The dispatcher begins a second round some 5 % before every slot is taken
-// (in double 2 %: 928^2 8 rows in two rounds 45, 5 in one of 97 % 40; kept at
-// 5 for tall units, which lose more to uneven rows than they gain).  Over many
+// Where every row is wet a launch is one round up to its last slot (4 to 16
+// rows: no step in its time before 1.00 of the slots, 11 to 21 % at 1.02).  On
+// rain-fed terrain, whose units take unequal times, float ran 4 850 units in
+// one round and 5 000 no more, so a first round counts as full 5 % before its
+// last slot; double did to 98 % (928^2 8 rows in two rounds 45, 5 in one of
+// 97 % 40), but tall units in double count with 5 too, on the evidence of one
+// size (2048^2 below: they lose more to uneven rows of a flood than they gain
+// under rain).  Later boundaries are no such step (float, 8 rows: 72, 75, 76 us
+// at 1.95, 2.00, 2.02 rounds); there 2 % stands in both precisions.  Over many
 // rounds only the prologues and a short tail count.  Measured, order 2, height:
 // us (units per SIMD): float 256^2 1: 10.1 (1.3), 2: 10.6 (0.6); 500^2 1: 20.1
 // (4.4), 2: 16.4 (2.2), 3: 15.4 (1.5), 5: 17.2 (0.9); 1024^2 3: 33.6 (6.0),
@@ -1133,13 +1142,15 @@ int grid_flux_launch(const hp_grid_desc* g, hipStream_t st) {
 }
 
 // ---- allocation-free single-pass step ---------------------------------------
-// The single-pass step's only scratch memory is its per-tile partial records
-// (CFL minimum, FP64 sums), normally in the caller's workspace.  For callers
-// that cannot allocate, a file-scope device array holds them instead: every
-// GPU the library runs on keeps its own copy until the process ends.  Every
-// tile writes its record in every step before the time control reads it, so
-// nothing in it must start at zero; calls that overlap on one GPU share the
-// array and race.
+// The single-pass step's only scratch memory is its units' partial records
+// (CFL minimum, FP64 sums) or, in calls that fold the time control, the fold's
+// state and sum records, normally in the caller's workspace.  For callers that
+// cannot allocate, a file-scope device array holds them instead: every GPU the
+// library runs on keeps its own copy until the process ends.  Nothing in it
+// must start at zero: a unit writes its record in every step before the time
+// control reads it, a folded call begins with a launch that fills its state,
+// and the records that the units of a stopped step leave out are not read.
+// Calls that overlap on one GPU share the array and race.
 constexpr int64_t kScratchBytes = int64_t(8) << 20;
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 constexpr int kMaxScratchDevices = 64;
@@ -1283,7 +1294,7 @@ int hp_grid_step_fused_noalloc(const hp_grid_desc* g, int32_t nsteps, void* stre
   if (rc) return rc;
   const int64_t need = partials_bytes(std::max(nominal_tiles(g), update_blocks(g)));
   if (need > kScratchBytes)
-    return fail(HP_ESPACE, "domain needs " + std::to_string(need) + " bytes of per-tile records; the allocation-free "
+    return fail(HP_ESPACE, "domain needs " + std::to_string(need) + " bytes of per-unit records; the allocation-free "
                            "step holds at most " + std::to_string(kScratchBytes) + " (use hp_grid_step_fused)");
   void* p = nullptr;
   rc = scratch_ptr(&p);

@@ -46,7 +46,7 @@
 // pass, order 2, per step at the chosen unit height, from the two-row-prologue
 // walk (double: an LDS tile of 64 x 4 cells per block) to this one: float 64^2
 // 14.4 -> 8.3 us, 2048^2 72.7 -> 60.5, 8192^2 with a rain field and mass sums
-// 921 -> 814; double 2048^2 216 -> 147, 256^2 17.1 -> 12.0.
+// 921 -> 810; double 2048^2 216 -> 139, 256^2 17.1 -> 11.8.
 //
 // Geometry: a unit is (strip bx, row block by); 60 columns x R rows.  Each
 // interior x edge is solved once, except the one between two strips (solved
