@@ -79,18 +79,16 @@ class Simulation:
         self.t_list.append(t)
         self.results = num.get_h()[self.idx_target]
 
-    _CLOCK = frozenset(("time_friction_euler_update_cuda", "_step_and_clock", "_export_if_due", "t", "dt"))
-
     @staticmethod
     def _library_step(num) -> bool:
         """Whether the model's step, its export hook and its clock are the
         library's own: one that replaces any of them, in its class or on the
-        object, is asked for its clock.  (Asked on every step: the plain model
-        first.)"""
-        cls, names = type(num), Simulation._CLOCK
-        if not getattr(num, "__dict__", {}).keys().isdisjoint(names):
+        object, is asked for its clock."""
+        cls, own = type(num), getattr(num, "__dict__", ())
+        if "_export_if_due" in own or "time_friction_euler_update_cuda" in own or "_step_and_clock" in own:
             return False
-        return cls is Godunov or all(getattr(cls, m, None) is getattr(Godunov, m) for m in names)
+        return cls is Godunov or all(getattr(cls, m, None) is getattr(Godunov, m) for m in
+                                     ("_export_if_due", "time_friction_euler_update_cuda", "_step_and_clock", "t", "dt"))
 
     def time(self) -> float:
         return self.numerical.t.item()
