@@ -263,6 +263,17 @@ template <class T> struct EdgeOut {
   bool active;
 };
 
+// A number of the sign of the contact speed num / den, which is all that is
+// used of it, without the division: num * den, where den is not 0.  It is 0 not
+// only between two dry sides: a film moving at 1e5 m/s against a side that its
+// bed keeps dry has u - sqrt(g h) rounded to u, and num is 0 too.  The quotient
+// is then not a number, and neither comparison with 0 holds (the side that
+// flows off decides); the product would choose the star region, between two
+// equal speeds, and pass an infinite flux.
+template <class T> __host__ __device__ inline T contact_sign(T num, T den) {
+  return num * (den == T(0) ? T(INFINITY) : den);
+}
+
 // HLLC with the hydrostatic reconstruction applied first.
 // eL / eR: edge states before reconstruction (h, qn, qt, z) - velocities come
 // from these.  etaC / etaR: the cells' water levels used by the clamp.
@@ -326,11 +337,8 @@ __host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T 
   const T sR_dry = uL0 + T(2) * aL, sR_wet = fmax(uR0 + aR, u_star + a_star);
   const T sL = le_hs(hL) ? sL_dry : sL_wet;
   const T sR = le_hs(hR) ? sR_dry : sR_wet;
-  // only the sign of the contact speed sM = num / den is used, and num * den
-  // has it without the division (den is 0 only between two dry sides, whose
-  // flux is 0 whatever is chosen here)
   const T num = sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), den = hR * (uR0 - sR) - hL * (uL0 - sL);
-  const T sM = num * den;
+  const T sM = contact_sign(num, den);
   const T qnfL = uL0 * qnL + T(0.5) * g * hL * hL;
   const T qnfR = uR0 * qnR + T(0.5) * g * hR * hR;
   const T rS = P::div(T(1), sR - sL);
