@@ -142,7 +142,7 @@ __host__ __device__ inline bool solve_edge_vjp(const FrameCell<T>& c, const Fram
   const T sL = sLdry ? sLd : sLw, sR = sRdry ? sRd : sRw;
   // the sign of the contact speed, as hllc_edge takes it
   const T num = sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), den = hR * (uR0 - sR) - hL * (uL0 - sL);
-  const T sM = contact_sign(num, den);
+  const T sM = P::quotient_sign(num, den);
   const bool left = T(0) <= sL, useL = both(sL < T(0), T(0) <= sM);
   const bool star = both(!left, either(useL, both(sM < T(0), T(0) <= sR)));
   const bool inL = both(flux_on, left), inS = both(flux_on, star), inR = both(flux_on, !either(left, star));

@@ -101,6 +101,19 @@ template <> struct Prec<double> {
   __host__ __device__ static inline double min2(double x, double y) { return fmin(x, y); }
   __host__ __device__ static inline double max_abs(double x, double y) { return fmax(fabs(x), fabs(y)); }
   __host__ __device__ static inline double div(double a, double b) { return a / b; }
+  // A number of the sign of a / b, or not a number where the quotient is none
+  // (0 / 0, inf / inf): the division's last instruction alone, which settles its
+  // special cases.  (The sign of a * b is not enough: beside a side that its bed
+  // keeps dry, a film at 1e5 m/s in float has u - sqrt(g h) rounded to u and both
+  // a and b 0.  A zero then reads as a contact speed inside the star region,
+  // between two equal wave speeds: an infinite flux.)
+  __host__ __device__ static inline double quotient_sign(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_div_fixup(1.0, b, a);
+#else
+    return a / b;
+#endif
+  }
   __host__ __device__ static inline double sqrt_(double x) { return __builtin_sqrt(x); }
   // h^(-1/3) for a wet depth (h > 1e-6): a single-precision seed (relative
   // error ~1e-7) refined by two Newton steps of y <- y (4 - h y^3) / 3, the
@@ -153,6 +166,7 @@ template <> struct Prec<float> {
     return r;
   }
   __device__ static inline float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+  __device__ static inline float quotient_sign(float a, float b) { return __builtin_amdgcn_div_fixupf(1.0f, b, a); }
   __device__ static inline float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
   // h^(-1/3) = exp2(-log2(h) / 3) with the hardware log2 / exp2 (h >= 1e-6)
   __device__ static inline float rcbrt_friction(float h) {
@@ -263,17 +277,6 @@ template <class T> struct EdgeOut {
   bool active;
 };
 
-// A number of the sign of the contact speed num / den, which is all that is
-// used of it, without the division: num * den, where den is not 0.  It is 0 not
-// only between two dry sides: a film moving at 1e5 m/s against a side that its
-// bed keeps dry has u - sqrt(g h) rounded to u, and num is 0 too.  The quotient
-// is then not a number, and neither comparison with 0 holds (the side that
-// flows off decides); the product would choose the star region, between two
-// equal speeds, and pass an infinite flux.
-template <class T> __host__ __device__ inline T contact_sign(T num, T den) {
-  return num * (den == T(0) ? T(INFINITY) : den);
-}
-
 // HLLC with the hydrostatic reconstruction applied first.
 // eL / eR: edge states before reconstruction (h, qn, qt, z) - velocities come
 // from these.  etaC / etaR: the cells' water levels used by the clamp.
@@ -338,7 +341,7 @@ __host__ __device__ inline void hllc_edge(FrameCell<T>& eL, FrameCell<T>& eR, T 
   const T sL = le_hs(hL) ? sL_dry : sL_wet;
   const T sR = le_hs(hR) ? sR_dry : sR_wet;
   const T num = sL * hR * (uR0 - sR) - sR * hL * (uL0 - sL), den = hR * (uR0 - sR) - hL * (uL0 - sL);
-  const T sM = contact_sign(num, den);
+  const T sM = P::quotient_sign(num, den);  // (only the contact speed's sign is used)
   const T qnfL = uL0 * qnL + T(0.5) * g * hL * hL;
   const T qnfR = uR0 * qnR + T(0.5) * g * hR * hR;
   const T rS = P::div(T(1), sR - sL);

@@ -48,3 +48,17 @@ def test_an_asked_height_keeps_the_sums(cuda, dtype):
     for s, t in zip(a, b):
         for u, v in zip(state(s), state(t)):
             assert torch.equal(u, v)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_two_pass_sums_keep_their_bits(cuda, dtype):
+    """The two-pass step's sums come from its update pass, whose blocks are a
+    domain's own: one to eight elements a thread."""
+    sizes = [(70, 61), (601, 433), (900, 700), (1101, 1000)]
+    a, b = ([solver(ny, nx, dtype, True, t=1.0) for ny, nx in sizes] for _ in range(2))
+    Ensemble(a, single_pass=False).step(3)
+    for s in b:
+        s.step(3)
+    for s, t in zip(a, b):
+        for u, v in zip(state(s), state(t)):
+            assert torch.equal(u, v)

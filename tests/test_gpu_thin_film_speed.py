@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import rel_err
+from helpers import random_state, rel_err
 from hipims_amd.adjoint import Calibration
 from hipims_amd.compact_driver import CompactGodunov
 from hipims_amd.grid import GridSolver
@@ -84,3 +84,21 @@ def test_gradient_stays_finite(cuda, order, np_dtype, lift, reverse):
         loss = cal.run(cal.theta0())
         assert torch.isfinite(torch.as_tensor(loss)), (ny, nx, turn)
         assert torch.isfinite(cal.gradient()).all(), (ny, nx, turn)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("fused", [True, False])
+def test_quotients_that_overflow_choose_no_star_region(cuda, order, fused):
+    """inf / inf is no number either: absurd single cells (1e30) leave the depths finite in float for a step, as the
+    division does; the sign of their product passed infinite fluxes."""
+    ny, nx = 40, 190
+    z, h, qx, qy = random_state(ny, nx, seed=3, rough=0.1)
+    rng = np.random.Generator(np.random.PCG64(3))
+    for v in (1e30, -1e30):
+        for a in (h, qx, qy):
+            a[rng.integers(0, ny, 2), rng.integers(0, nx, 2)] = v
+    pad = lambda a, v: np.pad(a, 1, constant_values=v)  # noqa: E731
+    s = GridSolver(pad(np.full((ny, nx), 40), -9999), pad(h, 0.0), pad(qx, 0.0), pad(qy, 0.0), pad(z, 0.0), 1.0,
+                   order=order, dtype=torch.float32, first_dt=0.005, t=1.0, manning=[0.03])
+    s.step_fused(1) if fused else s.step(1)
+    assert torch.isfinite(s.h).all()
