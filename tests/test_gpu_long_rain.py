@@ -1,0 +1,47 @@
+"""Thousands of steps of rain on rough terrain, alone and in an ensemble, in one
+and in two passes: films, bumps that fall dry and fast shallow flow meet every
+branch of the edge solver sooner or later.  The water must stay finite, the
+paths must keep each other's bits, and the depths must account for the rain."""
+import pytest
+import torch
+
+from hipims_amd import generators as gen
+from hipims_amd.ensemble import Ensemble
+from hipims_amd.grid import GridSolver
+
+pytestmark = pytest.mark.gpu
+
+# 512^2 scenarios whose runs pass films faster than a float can hold beside their wave speed
+SCENARIOS = [k for k, s in enumerate(gen.ensemble_specs(64, 2000)) if s[0] == 512][:6]
+STEPS = 6000
+
+
+def solver(k, order, dtype):
+    c = gen.ensemble_case(*gen.ensemble_specs(64, 2000)[k])
+    s = GridSolver(c.mask, c.h, c.qx, c.qy, c.z, c.dx, cfl=c.cfl, order=order, dtype=dtype, first_dt=c.first_dt,
+                   manning=c.manning, landuse=c.landuse)
+    s.set_station_rain(c.rain_table)
+    return s
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("order", [1, 2])
+def test_paths_stay_finite_and_together(cuda, order, dtype):
+    ens = [solver(k, order, dtype) for k in SCENARIOS]
+    Ensemble(ens).step(STEPS)
+    for n, (k, s) in enumerate(zip(SCENARIOS, ens)):
+        d = s.ctrl_dict()
+        for x in (s.h, s.qx, s.qy, s.h_max):
+            assert torch.isfinite(x).all(), k
+        # every step rounds each depth and its increment once (eps/2 of the water each), and a step's FP64 sums of n
+        # depths n eps/2 of it
+        tol = STEPS * torch.finfo(dtype).eps + 2 * s.layout.n_valid * torch.finfo(torch.float64).eps
+        assert abs(d["volume"] - d["rain_volume"] - d["flux_volume"]) <= tol * d["rain_volume"], k
+        if n < 2:
+            one, two = solver(k, order, dtype), solver(k, order, dtype)
+            one.step_fused(STEPS)
+            two.step(STEPS)
+            for a in (one, two):
+                for x, y in zip((a.h, a.qx, a.qy, a.h_max), (s.h, s.qx, s.qy, s.h_max)):
+                    assert torch.equal(x, y), k
+                assert a.t == s.t and a.dt == s.dt
