@@ -11,8 +11,8 @@ from hipims_amd.grid import GridSolver
 
 pytestmark = pytest.mark.gpu
 
-# 512^2 scenarios whose runs pass films faster than a float can hold beside their wave speed
-SCENARIOS = [k for k, s in enumerate(gen.ensemble_specs(64, 2000)) if s[0] == 512][:6]
+# 512^2 scenarios; the first one's film meets the edge of float's precision at step 4659 (order 2)
+SCENARIOS = [57, 19, 35, 54, 16, 29]
 STEPS = 6000
 
 
